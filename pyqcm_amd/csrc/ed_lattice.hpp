@@ -12,7 +12,7 @@
 
 namespace ed {
 
-// Green-function dimensions handled by the wave-per-matrix kernels
+// Green-function dimensions and neighbor vectors handled by the kernels
 constexpr int kLatticeMaxDim = 8;
 constexpr int kLatticeMaxNbr = 64;
 
@@ -35,11 +35,15 @@ struct KGrid {
   long count() const;
 };
 
-// device copy of a Superlattice: the elements grouped by matrix position
+// device copy of a Superlattice: the elements grouped by neighbor vector
+// (eptr[nnbr + 1]; epos: slot in plist | position << 16), plist the npos
+// column-major positions where V(k) can be nonzero (bits of mask)
 struct SuperlatticeDev {
-  int d = 0, nnbr = 0;
-  DevBuf<double> V0, val, R;
-  DevBuf<int> ptr, nbr;  // ptr: d^2 + 1 over positions (column-major)
+  int d = 0, nnbr = 0, npos = 0;
+  unsigned long long mask = 0;
+  DevBuf<double> mem;
+  const double *V0 = nullptr, *val = nullptr, *R = nullptr;
+  const int *eptr_d = nullptr, *epos_d = nullptr, *plist_d = nullptr;
   explicit SuperlatticeDev(const Superlattice &S);
 };
 
