@@ -1,7 +1,7 @@
 // ed_batch.cpp -- host side of the batched solver: builds one work item per
 // (instance, target sector) for the ground state and one per (state, spin,
-// +-, orbital pair) for the continued fractions, runs each stage as a single
-// launch, and hands the results to the instances exactly as their own solve
+// +-, orbital pair) for the continued fractions, runs the items of a stage
+// together, and hands the results to the instances exactly as their own solve
 // would (finalize_states; GFRep 'F').
 #include "ed_batch.hpp"
 
@@ -18,9 +18,10 @@ namespace {
 
 // packed device copy of many FactorizedHost tables
 struct TablePack {
+  static constexpr size_t kNone = ~size_t(0);
   std::vector<uint32_t> u32;
   std::vector<double> f64;
-  struct Off { size_t up_ptr, up_col, dn_ptr, dn_col, up_val, dn_val, diag; uint32_t du, dd, nu, nd; };
+  struct Off { size_t up_ptr, up_col, dn_ptr, dn_col, up_val, dn_val, diag, diag_t; uint32_t du, dd, nu, nd; };
   std::vector<Off> offs;
   DevBuf<uint32_t> du32;
   DevBuf<double> df64;
@@ -45,6 +46,7 @@ struct TablePack {
     o.up_val = put64(F.up_val);
     o.dn_val = put64(F.dn_val);
     o.diag = put64(F.diag);
+    o.diag_t = kNone;
     o.du = F.du;
     o.dd = F.dd;
     o.nu = (uint32_t)F.up_col.size();
@@ -75,37 +77,125 @@ struct TablePack {
     S.diag = df64.p + o.diag;
     return S;
   }
+  // the sector will be used as a wide item: its diagonal in lane order too
+  // (before upload)
+  void use_wide(int k) {
+    Off &o = offs[k];
+    if (o.dd <= o.du || o.diag_t != kNone) return;
+    o.diag_t = f64.size();
+    f64.resize(f64.size() + (size_t)o.du * o.dd);
+    for (uint32_t u = 0; u < o.du; ++u)
+      for (uint32_t d = 0; d < o.dd; ++d) f64[o.diag_t + (size_t)u * o.dd + d] = f64[o.diag + (size_t)d * o.du + u];
+  }
+  // entries of the longest row of the smaller half's table (a wide item's rows)
+  uint32_t longest_row(int k) const {
+    const Off &o = offs[k];
+    const uint32_t *p = u32.data() + (o.dd > o.du ? o.up_ptr : o.dn_ptr), n = std::min(o.du, o.dd);
+    uint32_t m = 0;
+    for (uint32_t r = 0; r < n; ++r) m = std::max(m, p[r + 1] - p[r]);
+    return m;
+  }
+  WideItem wide(int k, int swap) const {
+    const Off &o = offs[k];
+    WideItem w;
+    w.lp = du32.p + (swap ? o.dn_ptr : o.up_ptr);
+    w.lc = du32.p + (swap ? o.dn_col : o.up_col);
+    w.lv = df64.p + (swap ? o.dn_val : o.up_val);
+    w.rp = du32.p + (swap ? o.up_ptr : o.dn_ptr);
+    w.rc = du32.p + (swap ? o.up_col : o.dn_col);
+    w.rv = df64.p + (swap ? o.up_val : o.dn_val);
+    w.dg = df64.p + (swap ? o.diag_t : o.diag);
+    return w;
+  }
 };
 
-// execution class of an item: from LDS with one or four waves, global
-// vectors with one or four waves
-enum Cls { kLds = 0, kLdsWide = 1, kWave = 2, kBlock = 3 };
-constexpr int kClasses = 4;
+// where a wide item's alpha_k and beta_{k-1} go: a continued fraction's own
+// arrays, a ground state's tridiagonal arrays tri (M long each)
+void wide_coefficients(const BatchCFItem &it, double *, size_t, WideItem &w) {
+  w.a = it.a;
+  w.b = it.b;
+}
+void wide_coefficients(const BatchGSItem &, double *tri, size_t M, WideItem &w) {
+  w.a = tri;
+  w.b = tri + M - 1;
+}
+
+// execution class of an item: from LDS with one or four waves, or with the
+// other items of its shape in lockstep
+enum Cls { kLds = 0, kLdsFour = 1, kWide = 2 };
 
 // items held in LDS with at least this many states get four waves (the
 // steps are latency-bound; more waves per item hide more of it)
-constexpr uint32_t kWideDim = 128;
+constexpr uint32_t kFourWaveDim = 128;
 
-// items whose sector has at most this many states and does not fit in LDS
-// run in a one-wave workgroup with global vectors
-constexpr uint32_t kOneWaveDim = 4096;
+// Vectors of the wide items advanced together: what the 256 MB memory-side
+// cache holds beside the tables.  (4 points of 108 900-state fractions: 60 MB
+// 217 ms, 192 MB 199, 400 MB 201, all at once 201: the bound also keeps the
+// workspace small.)
+constexpr size_t kWideBytes = size_t(192) << 20;
 
+// LDS decides between one workgroup an item and lockstep: a workgroup with
+// vectors in memory, the only other way to keep an item by itself, took 1.3 to
+// 8 times the lockstep's time over sectors of 2 450 to 108 900 states (64
+// points of 3 920-state fractions 21.6 -> 17.7 ms, 4 points of 108 900-state
+// ones 1 630 -> 162 ms).
 Cls classify(size_t lds, uint32_t dim) {
-  if (lds <= kBatchLdsCap) return dim >= kWideDim ? kLdsWide : kLds;
-  return dim <= kOneWaveDim ? kWave : kBlock;
+  if (lds <= kBatchLdsCap) return dim >= kFourWaveDim ? kLdsFour : kLds;
+  return kWide;
 }
-bool in_lds(Cls c) { return c == kLds || c == kLdsWide; }
 
-// one launch per non-empty class
+// one launch per LDS class
 template <typename Item, typename Launch>
 void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls, size_t lds_max, Launch launch) {
-  std::vector<Item> part[kClasses];
-  for (size_t k = 0; k < items.size(); ++k) part[cls[k]].push_back(items[k]);
-  DevBuf<Item> d[kClasses];
-  for (int c = 0; c < kClasses; ++c) {
+  std::vector<Item> part[kWide];
+  for (size_t k = 0; k < items.size(); ++k)
+    if (cls[k] != kWide) part[cls[k]].push_back(items[k]);
+  DevBuf<Item> d[kWide];
+  for (int c = 0; c < kWide; ++c) {
     if (part[c].empty()) continue;
     d[c].upload(part[c]);
-    launch(d[c].p, (int)part[c].size(), (c == kBlock || c == kLdsWide) ? 256 : 64, in_lds((Cls)c) ? lds_max : 0);
+    launch(d[c].p, (int)part[c].size(), c == kLdsFour ? 256 : 64, lds_max);
+  }
+  sync();
+}
+
+// The wide items (tab[k]: item k's sector), by shape and then in groups whose
+// vectors (nvec each) fit kWideBytes: run(shape, device items, sources, n).
+// ntri doubles of tridiagonal arrays per item are handed out when nonzero.
+template <typename Item, typename Run>
+void launch_wide(const TablePack &tabs, const std::vector<Item> &items, const std::vector<Cls> &cls,
+                 const std::vector<int> &tab, int nvec, size_t ntri, Run run) {
+  std::map<std::pair<uint32_t, uint32_t>, std::vector<size_t>> shapes;
+  for (size_t k = 0; k < items.size(); ++k)
+    if (cls[k] == kWide) shapes[{tabs.offs[tab[k]].du, tabs.offs[tab[k]].dd}].push_back(k);
+  for (const auto &sh : shapes) {
+    const size_t dim = (size_t)sh.first.first * sh.first.second;
+    const size_t per = std::max<size_t>(1, kWideBytes / (8 * (size_t)nvec * dim));
+    const size_t ngrp = (sh.second.size() + per - 1) / per, len = (sh.second.size() + ngrp - 1) / ngrp;
+    for (size_t g0 = 0; g0 < sh.second.size(); g0 += len) {
+      const int n = (int)std::min(len, sh.second.size() - g0);
+      uint32_t emax = 0;
+      for (int k = 0; k < n; ++k) emax = std::max(emax, tabs.longest_row(tab[sh.second[g0 + k]]));
+      const WideShape W = wide_shape(sh.first.first, sh.first.second, emax, n);
+      const size_t scal = 2 * (size_t)W.nwg + kWideScalars + ntri;
+      DevBuf<double> u((size_t)nvec * dim * n), sc(scal * n);
+      std::vector<WideItem> wi(n);
+      std::vector<Item> src(n);
+      for (int k = 0; k < n; ++k) {
+        const size_t i = sh.second[g0 + k];
+        src[k] = items[i];
+        wi[k] = tabs.wide(tab[i], W.swap);
+        wi[k].u = u.p + (size_t)nvec * dim * k;
+        wi[k].part = sc.p + scal * k;
+        wi[k].sc = wi[k].part + 2 * (size_t)W.nwg;
+        wide_coefficients(items[i], ntri ? wi[k].sc + kWideScalars : nullptr, ntri / kTriArrays, wi[k]);
+      }
+      DevBuf<WideItem> dw;
+      DevBuf<Item> ds;
+      dw.upload(wi);
+      ds.upload(src);
+      run(W, dw.p, ds.p, n);
+    }
   }
   sync();
 }
@@ -244,27 +334,24 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
         gs_len += dim;
       }
     }
-    tabs.upload();
-    vlog("batch: %zu ground-state tables built and uploaded", refs.size());
     const size_t ntri = (size_t)kTriArrays * (max_iter + 2);
     std::vector<Cls> cls(refs.size());
-    size_t lds_max = 0, ws_len = 0, ntri_glob = 0;
+    std::vector<int> tab(refs.size());
+    size_t lds_max = 0;
     for (size_t k = 0; k < refs.size(); ++k) {
       const size_t b = tabs.lds(refs[k].tab, kGsVectors, ntri);
       cls[k] = classify(b, refs[k].dim);
-      if (in_lds(cls[k])) {
-        lds_max = std::max(lds_max, b);
-      } else {
-        ws_len += 2 * (size_t)refs[k].dim;
-        ++ntri_glob;
-      }
+      tab[k] = refs[k].tab;
+      if (cls[k] == kWide) tabs.use_wide(tab[k]);
+      else lds_max = std::max(lds_max, b);
     }
+    tabs.upload();
+    vlog("batch: %zu ground-state tables built and uploaded", refs.size());
     // the ground states stay here; each state's vector is a view kept alive by it
     auto gsv = std::make_shared<DevBuf<double>>(std::max<size_t>(gs_len, 1));
-    DevBuf<double> ws(std::max<size_t>(ws_len, 1)), tri(std::max<size_t>(ntri * ntri_glob, 1)),
-        out(std::max<size_t>(3 * refs.size(), 1));
+    DevBuf<double> out(std::max<size_t>(3 * refs.size(), 1));
     std::vector<BatchGSItem> items(refs.size());
-    size_t wo = 0, go = 0, to = 0;
+    size_t go = 0;
     for (size_t k = 0; k < refs.size(); ++k) {
       BatchGSItem &it = items[k];
       it.S = tabs.view(refs[k].tab);
@@ -272,14 +359,12 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
       it.gs = gsv->p + go;
       it.out = out.p + 3 * k;
       go += refs[k].dim;
-      if (!in_lds(cls[k])) {
-        it.ws = ws.p + wo;
-        it.tri = tri.p + ntri * to++;
-        wo += 2 * (size_t)refs[k].dim;
-      }
     }
     launch_classes(items, cls, lds_max, [&](const BatchGSItem *d, int n, int block, size_t lds) {
       batch_gs(d, n, block, lds, max_iter, accur, stream());
+    });
+    launch_wide(tabs, items, cls, tab, 3, ntri, [&](const WideShape &W, const WideItem *w, const BatchGSItem *q, int n) {
+      wide_gs(W, w, q, n, max_iter, accur, stream());
     });
     const std::vector<double> res = out.to_host();
     if (verbose()) {
@@ -390,32 +475,32 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
       }
     }
   }
-  tabs.upload();
-  vlog("batch: %zu continued-fraction items, tables and maps built", refs.size());
   std::vector<Cls> cls(refs.size());
-  size_t lds_max = 0, ws_len = 0;
+  std::vector<int> tab(refs.size());
+  size_t lds_max = 0;
   for (size_t k = 0; k < refs.size(); ++k) {
     const size_t b = tabs.lds(refs[k].tab, kCfVectors, 0);
     cls[k] = classify(b, refs[k].dim);
-    if (in_lds(cls[k])) lds_max = std::max(lds_max, b);
-    else ws_len += 2 * (size_t)refs[k].dim;
+    tab[k] = refs[k].tab;
+    if (cls[k] == kWide) tabs.use_wide(tab[k]);
+    else lds_max = std::max(lds_max, b);
   }
-  DevBuf<double> ws(std::max<size_t>(ws_len, 1)), av(std::max<size_t>((size_t)max_cf * refs.size(), 1)),
+  tabs.upload();
+  vlog("batch: %zu continued-fraction items, tables and maps built", refs.size());
+  DevBuf<double> av(std::max<size_t>((size_t)max_cf * refs.size(), 1)),
       bv(std::max<size_t>((size_t)(max_cf + 1) * refs.size(), 1)), out(std::max<size_t>(2 * refs.size(), 1));
-  size_t wo = 0;
   for (size_t k = 0; k < refs.size(); ++k) {
     BatchCFItem &it = items[k];
     it.S = tabs.view(refs[k].tab);
     it.a = av.p + (size_t)max_cf * k;
     it.b = bv.p + (size_t)(max_cf + 1) * k;
     it.out = out.p + 2 * k;
-    if (!in_lds(cls[k])) {
-      it.ws = ws.p + wo;
-      wo += 2 * (size_t)refs[k].dim;
-    }
   }
   launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds) {
     batch_cf(d, n, block, lds, max_cf, acc_cf, stream());
+  });
+  launch_wide(tabs, items, cls, tab, 2, 0, [&](const WideShape &W, const WideItem *w, const BatchCFItem *q, int n) {
+    wide_cf(W, w, q, n, max_cf, acc_cf, stream());
   });
   const std::vector<double> res = out.to_host();
   // the store: fraction f holds n_f coefficients (0 where psi vanished or no

@@ -1,11 +1,11 @@
-// ed_batch.hip -- one workgroup per work item: a whole Lanczos ground state or
-// a whole LanczosGreen continued fraction of one small sector, so that a
-// sweep over hundreds of parameter points x sectors is a single launch
-// instead of hundreds of thousands of tiny ones.  An item whose sector fits
-// (tables, diagonal, Lanczos vectors and tridiagonal arrays within
-// kBatchLdsCap) runs entirely from LDS; larger items keep their vectors in
-// global memory.  Every reduction is a workgroup reduction; the projected
-// tridiagonal problem is solved on the device by wave 0.
+// ed_batch.hip -- batched Lanczos ground states and LanczosGreen continued
+// fractions.  An item whose sector fits (tables, diagonal, Lanczos vectors and
+// tridiagonal arrays within kBatchLdsCap) is one workgroup that runs the whole
+// recurrence from LDS, so that a sweep over hundreds of parameter points x
+// sectors is a single launch.  Larger ("wide") items keep their vectors in
+// memory and advance in lockstep, two launches per Lanczos step for all items
+// of a shape.  The projected tridiagonal problem is solved on the device by
+// one wave per item; every reduction has a fixed order.
 #include "ed_batch.hpp"
 
 #include <cfloat>
@@ -295,7 +295,7 @@ __device__ __forceinline__ void tri_lowest_wave(int n, const double *a, const do
   }
 }
 
-template <int BS, bool LDS>
+template <int BS>
 __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int max_iter, double accur) {
   extern __shared__ double smem[];
   __shared__ double sh[BS / kW];
@@ -305,23 +305,10 @@ __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int m
   const uint32_t dim = G.du * G.dd;
   const double rdu = 1.0 / (double)G.du;
   const int M = max_iter + 2;
-  double *v, *vp, *gs, *tri;
-  BatchSector S;
-  if constexpr (LDS) {
-    v = smem;
-    vp = v + dim;
-    gs = vp + dim;
-    tri = gs + dim;
-    const uint32_t nu = G.up_ptr[G.du], nd = G.dn_ptr[G.dd];
-    double *d = tri + (size_t)kTriArrays * M;
-    S = stage_sector<BS>(G, d, reinterpret_cast<uint32_t *>(d + dim + nu + nd));
-  } else {
-    v = it.ws;
-    vp = v + dim;
-    gs = it.gs;
-    tri = it.tri;
-    S = G;
-  }
+  double *v = smem, *vp = v + dim, *gs = vp + dim, *tri = gs + dim;
+  const uint32_t nu = G.up_ptr[G.du], nd = G.dn_ptr[G.dd];
+  double *sd = tri + (size_t)kTriArrays * M;
+  const BatchSector S = stage_sector<BS>(G, sd, reinterpret_cast<uint32_t *>(sd + dim + nu + nd));
   double *al = tri, *be = al + M, *bb = be + M, *z = bb + M, *D = z + M, *l = D + M;
   // start vector (the same draws as the single-sector path)
   double nn = 0.0;
@@ -395,7 +382,7 @@ __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int m
   }
 }
 
-template <int BS, bool LDS>
+template <int BS>
 __global__ __launch_bounds__(BS) void k_batch_cf(const BatchCFItem *items, int max_cf, double acc) {
   extern __shared__ double smem[];
   __shared__ double sh[BS / kW];
@@ -411,19 +398,10 @@ __global__ __launch_bounds__(BS) void k_batch_cf(const BatchCFItem *items, int m
   double *av = itg.a, *bv = itg.b, *out = itg.out;
   const uint32_t dim = G.du * G.dd;
   const double rdu = 1.0 / (double)G.du;
-  double *v, *vp;
-  BatchSector S;
-  if constexpr (LDS) {
-    v = smem;
-    vp = v + dim;
-    const uint32_t nu = G.up_ptr[G.du], nd = G.dn_ptr[G.dd];
-    double *d = vp + dim;
-    S = stage_sector<BS>(G, d, reinterpret_cast<uint32_t *>(d + dim + nu + nd));
-  } else {
-    v = itg.ws;
-    vp = v + dim;
-    S = G;
-  }
+  double *v = smem, *vp = v + dim;
+  const uint32_t nu = G.up_ptr[G.du], nd = G.dn_ptr[G.dd];
+  double *sd = vp + dim;
+  const BatchSector S = stage_sector<BS>(G, sd, reinterpret_cast<uint32_t *>(sd + dim + nu + nd));
   // psi = c_o1 |gs> (+ c_o2 |gs>), gathered over the target sector
   double nn = 0.0;
   for (LabelWalk L(threadIdx.x, BS, G.du, rdu); L.I < dim; L.next(BS)) {
@@ -488,6 +466,363 @@ __global__ __launch_bounds__(BS) void k_batch_cf(const BatchCFItem *items, int m
   }
 }
 
+// ---------------------------------------------------------------------------
+// wide items.  The vectors stay unnormalized as in the device-driven
+// single-sector recurrence: U_k = beta_{k-1} v_k (U_0 the start vector, its
+// norm in place of beta_{-1}), buffer k & 1 holding U_k.  Step k is
+//   hv:  t = H U_k / n_k - (n_k / n_{k-1}) U_{k-1} over U_{k-1}, n_k = |U_k|
+//        folded from the previous launch's partials; partials of <t, U_k>
+//   upd: alpha_k = <t, U_k> / n_k, U_{k+1} = t - (alpha_k / n_k) U_k over t;
+//        partials of |U_{k+1}|^2
+// Every workgroup of an item folds the same partials in the same order, so
+// all take the same branch when the stop rule ends the item; workgroup 0
+// stores the scalars, which other workgroups read from the next launch on.
+// Memory bound: 6 vector accesses a step plus the neighbour rows, which hit
+// the XCD's L2 because an item's workgroups are numbered onto one XCD
+// (block b runs on XCD b % 8).  Rows of U_k are staged in LDS for the lane
+// part; a lane's table entries are loaded once for RPT rows, since they are
+// 12 bytes a hop against 8 of the vector.
+// ---------------------------------------------------------------------------
+enum { SC_N = 0, SC_NN = 1, SC_PROD = 2 /* two, by parity */, SC_HI = 4, SC_LAM = 5, SC_STATUS = 6 };
+constexpr double kRunning = -2.0;
+constexpr int kWideBlock = 256;
+constexpr int kXcd = 8;
+constexpr size_t kWideLdsMax = 144 * 1024;  // longest row staged in LDS
+
+// item and workgroup of a block (grid: kXcd * ceil(n / kXcd) * nwg blocks)
+__device__ __forceinline__ bool wide_place(int n, int nwg, int &item, int &w) {
+  const int b = blockIdx.x, j = b / kXcd;
+  item = (j / nwg) * kXcd + b % kXcd;
+  w = j % nwg;
+  return item < n;
+}
+
+// sum of nwg partials, the same in every lane of every workgroup
+__device__ __forceinline__ double wide_fold(const double *p, int nwg) {
+  double s = 0.0;
+  for (int i = threadIdx.x & (kW - 1); i < nwg; i += kW) s += p[i];
+  return wsum(s);
+}
+
+// MODE 0: step k of a continued fraction; 1: of a ground state; 2: step k
+// (>= 1) of the ground state's eigenvector replay on normalized vectors (max_k
+// is then the length of a tridiagonal array)
+template <int MODE, int RPT, bool RG1, bool STAGE>
+__global__ __launch_bounds__(kWideBlock) void k_wide_hv(const WideItem *items, int n, int nwg, uint32_t nl,
+                                                        uint32_t nr, int rg_n, uint32_t emax, int k, int max_k,
+                                                        double acc) {
+  extern __shared__ double smem[];
+  __shared__ double sh[kWideBlock / kW];
+  int item, w;
+  if (!wide_place(n, nwg, item, w)) return;
+  const WideItem it = items[item];
+  const size_t dim = (size_t)nl * nr;
+  const double *C = it.u + (MODE == 2 ? (size_t)((k - 1) & 1) : (size_t)(k & 1)) * dim;
+  double *P = it.u + (MODE == 2 ? (size_t)(k & 1) : (size_t)((k + 1) & 1)) * dim;
+  double c_h, c_p, c_x = 0.0, z = 0.0;  // t = c_h H x - c_p P - c_x x
+  if (MODE == 2) {
+    if (k >= (int)it.sc[SC_N]) return;
+    const double ib = 1.0 / it.b[k];
+    c_h = ib;
+    c_p = k >= 2 ? it.b[k - 1] * ib : 0.0;
+    c_x = it.a[k - 1] * ib;
+    z = it.a[3 * (size_t)max_k + k];  // the tridiagonal arrays start at a: alpha, beta, beta^2, z, ...
+  } else {
+    if (it.sc[SC_N] != kRunning) return;
+    const double s2 = wide_fold(it.part + nwg, nwg), nk = sqrt(s2);
+    bool stop;
+    if (k == 0) {
+      stop = MODE == 0 ? !(s2 > 1e-14) : !(s2 > 0.0);
+      if (w == 0 && threadIdx.x == 0) {
+        it.sc[SC_NN] = s2;
+        if (stop) it.sc[SC_N] = -1.0;
+      }
+    } else {
+      const double prod = it.sc[SC_PROD + ((k - 1) & 1)] * nk;
+      stop = MODE == 0 ? !(prod > acc && nk > acc && k < max_k) : !(nk > 0.0);
+      if (w == 0 && threadIdx.x == 0) {
+        it.b[k] = nk;
+        it.sc[SC_PROD + (k & 1)] = prod;
+        if (stop) it.sc[SC_N] = (double)k;
+      }
+    }
+    if (stop) return;
+    c_h = 1.0 / nk;
+    c_p = k == 0 ? 0.0 : nk / (k >= 2 ? it.b[k - 1] : sqrt(it.sc[SC_NN]));
+  }
+  const bool first = MODE == 2 ? k == 1 : k == 0;  // no previous vector: its buffer is not read
+  const uint32_t RG = RG1 ? 1u : (uint32_t)rg_n, R = RG * RPT;
+  const uint32_t d0 = (uint32_t)w * R;
+  const uint32_t nrow = d0 < nr ? min(R, nr - d0) : 0u;
+  const size_t base = (size_t)d0 * nl;
+  // staged: the neighbour lists of the R rows, padded to emax entries (own
+  // row, value 0), and the rows themselves
+  double *nval = smem, *xs = smem + (size_t)R * emax + (R * emax + 1) / 2;
+  uint32_t *ncol = reinterpret_cast<uint32_t *>(smem + (size_t)R * emax);
+  for (uint32_t f = threadIdx.x; f < R * emax; f += kWideBlock) {
+    const uint32_t r = f / emax, q = f - r * emax, d = min(d0 + r, nr - 1);
+    const uint32_t e = it.rp[d] + q;
+    const bool in = r < nrow && e < it.rp[d + 1];
+    ncol[f] = in ? it.rc[e] : d;
+    nval[f] = in ? it.rv[e] : 0.0;
+  }
+  if (STAGE)
+    for (uint32_t f = threadIdx.x; f < nrow * nl; f += kWideBlock) xs[f] = C[base + f];
+  __syncthreads();
+  const double *X = STAGE ? xs : C + base;
+  double dot = 0.0;
+  const uint32_t rg = RG1 ? 0u : threadIdx.x / nl;
+  for (uint32_t il = RG1 ? threadIdx.x : threadIdx.x - rg * nl; il < nl && rg < RG; il += RG1 ? kWideBlock : nl) {
+    // (rows past the last one repeat it, so that every load is in range; their
+    // results are not used)
+    uint32_t ro[RPT];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) ro[j] = min(rg + RG * j, nrow - 1);
+    double h[RPT], pv[RPT];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const size_t I = base + (size_t)ro[j] * nl + il;
+      h[j] = it.dg[I];
+      pv[j] = first ? 0.0 : P[I];
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) h[j] *= X[(size_t)ro[j] * nl + il];
+    const uint32_t e1 = it.lp[il + 1];
+    uint32_t e = it.lp[il];
+    for (; e + 4 <= e1; e += 4) {
+      uint32_t c[4];
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        c[q] = it.lc[e + q];
+        v[q] = it.lv[e + q];
+      }
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        const double *xr = X + (size_t)ro[j] * nl;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[j] += v[q] * xr[c[q]];
+      }
+    }
+    for (; e < e1; ++e) {
+      const uint32_t c = it.lc[e];
+      const double v = it.lv[e];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) h[j] += v * X[(size_t)ro[j] * nl + c];
+    }
+    // the row part: one neighbour of each of the RPT rows at a time, their
+    // loads in flight together
+#pragma unroll 2
+    for (uint32_t q = 0; q < emax; ++q) {
+      double x[RPT];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) x[j] = C[(size_t)ncol[ro[j] * emax + q] * nl + il];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) h[j] += nval[ro[j] * emax + q] * x[j];
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const uint32_t r = rg + RG * j;
+      if (r >= nrow) continue;
+      const size_t I = base + (size_t)r * nl + il;
+      const double x = X[(size_t)r * nl + il];
+      double t = c_h * h[j] - c_p * pv[j];
+      if (MODE == 2) t -= c_x * x;
+      P[I] = t;
+      if (MODE == 2) it.u[2 * dim + I] += z * t;
+      else dot += t * x;
+    }
+    if (!RG1) break;
+  }
+  if (MODE != 2) {
+    dot = bsum<kWideBlock>(dot, sh);
+    if (threadIdx.x == 0) it.part[w] = dot;
+  }
+}
+
+__global__ __launch_bounds__(kWideBlock) void k_wide_upd(const WideItem *items, int n, int nwg, size_t dim, int k) {
+  __shared__ double sh[kWideBlock / kW];
+  int item, w;
+  if (!wide_place(n, nwg, item, w)) return;
+  const WideItem it = items[item];
+  if (it.sc[SC_N] != kRunning) return;
+  const double inv = 1.0 / (k >= 1 ? it.b[k] : sqrt(it.sc[SC_NN]));
+  const double alpha = wide_fold(it.part, nwg) * inv;
+  if (w == 0 && threadIdx.x == 0) it.a[k] = alpha;
+  const double c = alpha * inv;
+  const double *C = it.u + (size_t)(k & 1) * dim;
+  double *T = it.u + (size_t)((k + 1) & 1) * dim;
+  const size_t chunk = (dim + nwg - 1) / nwg, i0 = (size_t)w * chunk, i1 = min(dim, i0 + chunk);
+  double s = 0.0;
+  for (size_t i = i0 + threadIdx.x; i < i1; i += kWideBlock) {
+    const double t = T[i] - c * C[i];
+    T[i] = t;
+    s += t * t;
+  }
+  s = bsum<kWideBlock>(s, sh);
+  if (threadIdx.x == 0) it.part[nwg + w] = s;
+}
+
+// U_0 of a continued fraction: psi = c_o1 |gs> (+ c_o2 |gs>)
+__global__ __launch_bounds__(kWideBlock) void k_wide_cf_init(const WideItem *items, const BatchCFItem *src, int n,
+                                                             int nwg, uint32_t nl, uint32_t nr, int swap) {
+  __shared__ double sh[kWideBlock / kW];
+  int item, w;
+  if (!wide_place(n, nwg, item, w)) return;
+  const WideItem it = items[item];
+  const BatchCFItem &q = src[item];
+  const double *gs = q.gs;
+  const uint32_t du_s = q.du_s;
+  const int spin = q.spin, norb = q.norb;
+  const int32_t *map0 = q.map[0], *map1 = q.map[1];
+  const int8_t *sgn0 = q.sgn[0], *sgn1 = q.sgn[1], *upar = q.upar;
+  const size_t dim = (size_t)nl * nr, chunk = (dim + nwg - 1) / nwg, i0 = (size_t)w * chunk;
+  const size_t i1 = min(dim, i0 + chunk);
+  double s = 0.0;
+  for (size_t J = i0 + threadIdx.x; J < i1; J += kWideBlock) {
+    const uint32_t r = (uint32_t)(J / nl), l = (uint32_t)(J - (size_t)r * nl);
+    const uint32_t iu = swap ? r : l, id = swap ? l : r;
+    const uint32_t im = spin == 0 ? iu : id;
+    double val = 0.0;
+    const int32_t s0 = map0[im];
+    if (s0 >= 0) val += (double)sgn0[im] * gs[spin == 0 ? (size_t)s0 + (size_t)du_s * id : iu + (size_t)du_s * s0];
+    if (norb == 2) {
+      const int32_t s1 = map1[im];
+      if (s1 >= 0) val += (double)sgn1[im] * gs[spin == 0 ? (size_t)s1 + (size_t)du_s * id : iu + (size_t)du_s * s1];
+    }
+    if (spin == 1) val *= (double)upar[iu];
+    it.u[J] = val;
+    s += val * val;
+  }
+  s = bsum<kWideBlock>(s, sh);
+  if (threadIdx.x == 0) {
+    it.part[nwg + w] = s;
+    if (w == 0) {
+      it.sc[SC_N] = kRunning;
+      it.sc[SC_PROD] = 1.0;
+    }
+  }
+}
+
+// U_0 of a ground state: normal draws in label order.  replay: the draws
+// normalized, and the eigenvector's first term z_0 v_0
+__global__ __launch_bounds__(kWideBlock) void k_wide_gs_init(const WideItem *items, const BatchGSItem *src, int n,
+                                                             int nwg, uint32_t nl, uint32_t nr, int swap, int M,
+                                                             int replay) {
+  __shared__ double sh[kWideBlock / kW];
+  int item, w;
+  if (!wide_place(n, nwg, item, w)) return;
+  const WideItem it = items[item];
+  const uint64_t seed = src[item].seed;
+  const size_t dim = (size_t)nl * nr, chunk = (dim + nwg - 1) / nwg, i0 = (size_t)w * chunk;
+  const size_t i1 = min(dim, i0 + chunk);
+  const double inv = replay ? 1.0 / sqrt(it.sc[SC_NN]) : 1.0, z0 = replay ? it.a[3 * (size_t)M] : 0.0;
+  double s = 0.0;
+  for (size_t J = i0 + threadIdx.x; J < i1; J += kWideBlock) {
+    const uint32_t r = (uint32_t)(J / nl), l = (uint32_t)(J - (size_t)r * nl);
+    const size_t I = swap ? (size_t)r + (size_t)nr * l : J;
+    const double x = normal_draw(seed, I) * inv;
+    it.u[J] = x;
+    if (replay) it.u[2 * dim + J] = z0 * x;
+    s += x * x;
+  }
+  if (replay) return;
+  s = bsum<kWideBlock>(s, sh);
+  if (threadIdx.x == 0) {
+    it.part[nwg + w] = s;
+    if (w == 0) {
+      it.sc[SC_N] = kRunning;
+      it.sc[SC_PROD] = 1.0;
+      it.sc[SC_HI] = __builtin_nan("");
+      it.sc[SC_STATUS] = 0.0;
+    }
+  }
+}
+
+// after step k: the Ritz pair of the (k + 1) x (k + 1) tridiagonal and the
+// stop rule of the ground state, one wave per item
+__global__ __launch_bounds__(kW) void k_wide_ritz(const WideItem *items, int nwg, int M, int k, int max_iter,
+                                                  double accur) {
+  extern __shared__ double smem[];
+  __shared__ double s_lam, s_zl, s_hi;
+  const WideItem it = items[blockIdx.x];
+  if (it.sc[SC_N] != kRunning) return;
+  // the tridiagonal in LDS: the Sturm counts and the inverse iteration walk it serially
+  double *al = smem, *be = al + k + 1, *bb = be + k + 1, *z = bb + k + 1, *D = z + k + 1, *l = D + k + 1;
+  double *be_g = it.a + M, *z_g = it.a + 3 * (size_t)M;
+  const double beta = sqrt(wide_fold(it.part + nwg, nwg));
+  for (int i = threadIdx.x; i <= k; i += kW) {
+    const double bi = i < k ? be_g[i] : beta;
+    al[i] = it.a[i];
+    be[i] = bi;
+    bb[i] = bi * bi;
+  }
+  if (threadIdx.x == 0) {
+    be_g[k] = beta;
+    s_hi = it.sc[SC_HI];
+  }
+  __syncthreads();
+  tri_lowest_wave(k + 1, al, be, bb, &s_hi, z, D, l, &s_lam, &s_zl);
+  __syncthreads();
+  for (int i = threadIdx.x; i <= k; i += kW) z_g[i] = z[i];
+  if (threadIdx.x == 0) {
+    it.sc[SC_HI] = s_hi;
+    it.sc[SC_LAM] = s_lam;
+    if (!(beta > 0.0) || fabs(s_zl * beta) <= accur) it.sc[SC_N] = (double)(k + 1);
+    else if (k + 1 > max_iter) {
+      it.sc[SC_STATUS] = 1.0;
+      it.sc[SC_N] = (double)(k + 1);
+    }
+  }
+}
+
+// norm partials of the eigenvector, then (scale) the normalized eigenvector in
+// label order and the item's results
+__global__ __launch_bounds__(kWideBlock) void k_wide_gs_out(const WideItem *items, const BatchGSItem *src, int n,
+                                                            int nwg, uint32_t nl, uint32_t nr, int swap, int scale) {
+  __shared__ double sh[kWideBlock / kW];
+  int item, w;
+  if (!wide_place(n, nwg, item, w)) return;
+  const WideItem it = items[item];
+  const size_t dim = (size_t)nl * nr, chunk = (dim + nwg - 1) / nwg, i0 = (size_t)w * chunk;
+  const size_t i1 = min(dim, i0 + chunk);
+  const double *g = it.u + 2 * dim;
+  if (!scale) {
+    double s = 0.0;
+    for (size_t J = i0 + threadIdx.x; J < i1; J += kWideBlock) s += g[J] * g[J];
+    s = bsum<kWideBlock>(s, sh);
+    if (threadIdx.x == 0) it.part[w] = s;
+    return;
+  }
+  const double ig = 1.0 / sqrt(wide_fold(it.part, nwg));
+  double *gs = src[item].gs;
+  for (size_t J = i0 + threadIdx.x; J < i1; J += kWideBlock) {
+    const uint32_t r = (uint32_t)(J / nl), l = (uint32_t)(J - (size_t)r * nl);
+    gs[swap ? (size_t)r + (size_t)nr * l : J] = g[J] * ig;
+  }
+  if (w == 0 && threadIdx.x == 0) {
+    src[item].out[0] = it.sc[SC_LAM];
+    src[item].out[1] = it.sc[SC_N];
+    src[item].out[2] = it.sc[SC_STATUS];
+  }
+}
+
+__global__ void k_wide_cf_out(const WideItem *items, const BatchCFItem *src, int n) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  src[k].out[0] = items[k].sc[SC_N];
+  src[k].out[1] = items[k].sc[SC_NN];
+}
+
+// number of items still running
+__global__ __launch_bounds__(kW) void k_wide_running(const WideItem *items, int n, int *count) {
+  int c = 0;
+  for (int k = threadIdx.x; k < n; k += kW) c += items[k].sc[SC_N] == kRunning;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, kW);
+  if (threadIdx.x == 0) *count = c;
+}
+
 // writes item k's fraction, transformed as the continued_fraction ctor
 // (src_ed/continued_fraction.cpp:33-42) does, at off[fid[k]] of the store:
 // a_i - E0 (electrons, pm > 0) or E0 - a_i (holes) in A; b_0 = ||psi||^2 w
@@ -514,28 +849,132 @@ __global__ void k_cf_store(int nitems, int max_cf, const double *out, const doub
 void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, int max_iter, double accur, hipStream_t s) {
   if (n <= 0) return;
   if (lds > kBatchLdsCap) fail(ED_ERR_INVALID, "batch_gs: LDS request above the cap");
-  if (lds > 0 && block == 256)
-    hipLaunchKernelGGL((k_batch_gs<256, true>), dim3(n), dim3(256), lds, s, d_items, max_iter, accur);
-  else if (lds > 0)
-    hipLaunchKernelGGL((k_batch_gs<64, true>), dim3(n), dim3(64), lds, s, d_items, max_iter, accur);
-  else if (block == 64)
-    hipLaunchKernelGGL((k_batch_gs<64, false>), dim3(n), dim3(64), 0, s, d_items, max_iter, accur);
+  if (block == 256)
+    hipLaunchKernelGGL((k_batch_gs<256>), dim3(n), dim3(256), lds, s, d_items, max_iter, accur);
   else
-    hipLaunchKernelGGL((k_batch_gs<256, false>), dim3(n), dim3(256), 0, s, d_items, max_iter, accur);
+    hipLaunchKernelGGL((k_batch_gs<64>), dim3(n), dim3(64), lds, s, d_items, max_iter, accur);
   ED_HIP(hipGetLastError());
 }
 
 void batch_cf(const BatchCFItem *d_items, int n, int block, size_t lds, int max_cf, double acc, hipStream_t s) {
   if (n <= 0) return;
   if (lds > kBatchLdsCap) fail(ED_ERR_INVALID, "batch_cf: LDS request above the cap");
-  if (lds > 0 && block == 256)
-    hipLaunchKernelGGL((k_batch_cf<256, true>), dim3(n), dim3(256), lds, s, d_items, max_cf, acc);
-  else if (lds > 0)
-    hipLaunchKernelGGL((k_batch_cf<64, true>), dim3(n), dim3(64), lds, s, d_items, max_cf, acc);
-  else if (block == 64)
-    hipLaunchKernelGGL((k_batch_cf<64, false>), dim3(n), dim3(64), 0, s, d_items, max_cf, acc);
+  if (block == 256)
+    hipLaunchKernelGGL((k_batch_cf<256>), dim3(n), dim3(256), lds, s, d_items, max_cf, acc);
   else
-    hipLaunchKernelGGL((k_batch_cf<256, false>), dim3(n), dim3(256), 0, s, d_items, max_cf, acc);
+    hipLaunchKernelGGL((k_batch_cf<64>), dim3(n), dim3(64), lds, s, d_items, max_cf, acc);
+  ED_HIP(hipGetLastError());
+}
+
+WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax, int nitems) {
+  WideShape W;
+  W.emax = emax;
+  W.swap = dd > du;
+  W.nl = W.swap ? dd : du;
+  W.nr = W.swap ? du : dd;
+  int rg = 1;
+  const size_t row = W.nl * sizeof(double);
+  if (row > kWideLdsMax) {
+    W.rpt = 1;
+  } else if (W.nl > (uint32_t)kWideBlock / 2) {
+    // one row at a time per thread column; eight rows share a table load
+    W.rpt = 8;
+    while (W.rpt > 1 && W.rpt * row > 64 * 1024) W.rpt /= 2;
+  } else {
+    rg = kWideBlock / (int)W.nl;
+    W.rpt = 4;
+  }
+  // fewer rows per thread where that leaves compute units without a workgroup
+  auto groups = [&](int rpt) { return (int)((W.nr + rg * rpt - 1) / (rg * rpt)); };
+  while (W.rpt > 1 && (long)nitems * groups(W.rpt) < 1024) W.rpt /= 2;
+  W.rows = rg * W.rpt;
+  W.nwg = groups(W.rpt);
+  W.stage = row <= kWideLdsMax;
+  W.lds = ((size_t)W.rows * emax + ((size_t)W.rows * emax + 1) / 2) * sizeof(double) + (W.stage ? W.rows * row : 0);
+  return W;
+}
+
+namespace {
+unsigned wide_grid(const WideShape &W, int n) { return (unsigned)(kXcd * ((n + kXcd - 1) / kXcd) * W.nwg); }
+
+template <int MODE>
+void wide_hv(const WideShape &W, const WideItem *items, int n, int k, int max_k, double acc, hipStream_t s) {
+  const int rg = W.rows / W.rpt;
+#define ED_WIDE(RPT, RG1, STG)                                                                                    \
+  do {                                                                                                            \
+    if (W.lds > 64 * 1024)                                                                                        \
+      ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_wide_hv<MODE, RPT, RG1, STG>),                  \
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)W.lds));                        \
+    hipLaunchKernelGGL((k_wide_hv<MODE, RPT, RG1, STG>), dim3(wide_grid(W, n)), dim3(kWideBlock), W.lds, s,       \
+                       items, n, W.nwg, W.nl, W.nr, rg, W.emax, k, max_k, acc);                                          \
+  } while (0)
+  if (!W.stage) ED_WIDE(1, true, false);
+  else if (rg > 1) {
+    if (W.rpt == 4) ED_WIDE(4, false, true);
+    else if (W.rpt == 2) ED_WIDE(2, false, true);
+    else ED_WIDE(1, false, true);
+  } else if (W.rpt == 8) ED_WIDE(8, true, true);
+  else if (W.rpt == 4) ED_WIDE(4, true, true);
+  else if (W.rpt == 2) ED_WIDE(2, true, true);
+  else ED_WIDE(1, true, true);
+#undef ED_WIDE
+}
+
+void wide_upd(const WideShape &W, const WideItem *items, int n, int k, hipStream_t s) {
+  hipLaunchKernelGGL(k_wide_upd, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, n, W.nwg,
+                     (size_t)W.nl * W.nr, k);
+}
+
+// items still running, asked of the device every kWideCheck steps
+constexpr int kWideCheck = 16;
+bool wide_running(const WideItem *items, int n, DevBuf<int> &count, hipStream_t s) {
+  check_cancel();
+  hipLaunchKernelGGL(k_wide_running, dim3(1), dim3(kW), 0, s, items, n, count.p);
+  ED_HIP(hipGetLastError());
+  return count.to_host()[0] > 0;
+}
+}  // namespace
+
+void wide_cf(const WideShape &W, const WideItem *items, const BatchCFItem *src, int n, int max_cf, double acc,
+             hipStream_t s) {
+  if (n <= 0) return;
+  DevBuf<int> count(1);
+  hipLaunchKernelGGL(k_wide_cf_init, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr,
+                     W.swap);
+  for (int k = 0; k <= max_cf; ++k) {
+    wide_hv<0>(W, items, n, k, max_cf, acc, s);  // k == max_cf only ends the items
+    if (k == max_cf) break;
+    wide_upd(W, items, n, k, s);
+    if ((k + 1) % kWideCheck == 0 && !wide_running(items, n, count, s)) break;
+  }
+  hipLaunchKernelGGL(k_wide_cf_out, dim3((n + 255) / 256), dim3(256), 0, s, items, src, n);
+  ED_HIP(hipGetLastError());
+}
+
+void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, int n, int max_iter, double accur,
+             hipStream_t s) {
+  if (n <= 0) return;
+  DevBuf<int> count(1);
+  const int M = max_iter + 2;
+  const unsigned g = wide_grid(W, n);
+  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap, M, 0);
+  int k = 0;
+  for (;; ++k) {
+    wide_hv<1>(W, items, n, k, 0, 0.0, s);
+    wide_upd(W, items, n, k, s);
+    const size_t tri = (size_t)kTriArrays * (k + 1) * sizeof(double);
+    if (tri > 64 * 1024)
+      ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_wide_ritz),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri));
+    hipLaunchKernelGGL(k_wide_ritz, dim3(n), dim3(kW), tri, s, items, W.nwg, M, k, max_iter, accur);
+    // (k_wide_ritz ends every item by step max_iter)
+    if ((k >= max_iter || (k + 1) % kWideCheck == 0) && !wide_running(items, n, count, s)) break;
+  }
+  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap, M, 1);
+  for (int j = 1; j <= k; ++j) wide_hv<2>(W, items, n, j, M, 0.0, s);
+  for (int scale = 0; scale < 2; ++scale)
+    hipLaunchKernelGGL(k_wide_gs_out, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap,
+                       scale);
   ED_HIP(hipGetLastError());
 }
 

@@ -1,6 +1,7 @@
-// ed_batch.hpp -- batched solves of many small sectors (parameter points of a
-// VCA / CDMFT sweep): one workgroup runs a whole Lanczos ground state, or a
-// whole LanczosGreen continued fraction, for one work item.
+// ed_batch.hpp -- batched solves of many sectors (parameter points of a VCA /
+// CDMFT sweep).  An item that fits in LDS runs as one workgroup, a whole
+// Lanczos ground state or LanczosGreen continued fraction; larger items
+// ("wide") advance together, one Lanczos step of every item per launch.
 #pragma once
 
 #include <vector>
@@ -23,13 +24,11 @@ struct BatchSector {
 // Lanczos ground state of one sector (LanczosEigenvalue + LanczosEigenvector,
 // src_ed/Hamiltonian/Lanczos.hpp:41-143): start vector normal_draw(seed, .)
 // normalized, Ritz stop |z_last beta| <= accur, eigenvector by replaying the
-// recurrence.  ws and tri are used only by items that do not fit in LDS.
+// recurrence
 struct BatchGSItem {
   BatchSector S;
   uint64_t seed = 0;
-  double *ws = nullptr;   // 2 dim
   double *gs = nullptr;   // dim: normalized ground state (output)
-  double *tri = nullptr;  // kTriArrays (max_iter + 2): alpha, beta, beta^2, z, pivots
   double *out = nullptr;  // E0, iterations, status (0 ok, 1 not converged)
 };
 
@@ -43,7 +42,6 @@ struct BatchCFItem {
   const int32_t *map[2] = {nullptr, nullptr};
   const int8_t *sgn[2] = {nullptr, nullptr};
   const int8_t *upar = nullptr;  // spin-down orbitals: (-1)^(up occupation)
-  double *ws = nullptr;       // 2 dim (items that do not fit in LDS)
   double *a = nullptr;        // max_cf
   double *b = nullptr;        // max_cf + 1 (b[0] = 1)
   double *out = nullptr;      // n (-1: psi vanishes), ||psi||^2
@@ -65,8 +63,44 @@ __host__ __device__ inline size_t batch_lds_bytes(int nvec, size_t ntri, uint32_
 constexpr int kGsVectors = 3;  // two Lanczos vectors, ground state
 constexpr int kCfVectors = 2;  // two Lanczos vectors
 
-// lds > 0: every item runs from LDS with that many dynamic LDS bytes;
-// lds == 0: vectors in global memory.  block: 64 or 256 threads per item
+// One wide item.  Its vectors are stored with the larger half basis as the
+// fast index ("lanes", nl states; the other half is "rows", nr states):
+// J = lane + nl * row, which is the label order unless swap.  dg is the
+// diagonal in that order.
+struct WideItem {
+  const uint32_t *lp = nullptr, *lc = nullptr, *rp = nullptr, *rc = nullptr;  // lane / row one-body tables (CSR)
+  const double *lv = nullptr, *rv = nullptr, *dg = nullptr;
+  double *u = nullptr;     // 2 dim: the two Lanczos vectors (a ground state: 3 dim, the eigenvector last)
+  double *part = nullptr;  // 2 nwg: dot and norm partials
+  double *a = nullptr;     // alpha_k at a[k]
+  double *b = nullptr;     // beta_{k-1} at b[k], k >= 1
+  double *sc = nullptr;    // kWideScalars, see ed_batch.hip
+};
+constexpr int kWideScalars = 8;
+
+// items of one shape (nl x nr), advanced together
+struct WideShape {
+  uint32_t nl = 0, nr = 0;
+  int swap = 0;
+  int rows = 1;     // rows per workgroup
+  int rpt = 1;      // rows per thread
+  int nwg = 1;      // workgroups per item
+  uint32_t emax = 0;  // longest row of the row tables
+  bool stage = true;  // rows fit in LDS (else read from memory)
+  size_t lds = 0;
+};
+WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax, int nitems);
+
+// continued fractions of n items of one shape; src[k] is item k's start state
+void wide_cf(const WideShape &W, const WideItem *items, const BatchCFItem *src, int n, int max_cf, double acc,
+             hipStream_t s);
+// ground states of n items of one shape: src[k].gs and src[k].out as for
+// batch_gs; item k's a is its kTriArrays tridiagonal arrays (max_iter + 2 long
+// each: alpha, beta, ...) and b points one before the second of them
+void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, int n, int max_iter, double accur,
+             hipStream_t s);
+
+// items run from LDS, lds dynamic bytes each; block: 64 or 256 threads per item
 void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, int max_iter, double accur, hipStream_t s);
 void batch_cf(const BatchCFItem *d_items, int n, int block, size_t lds, int max_cf, double acc, hipStream_t s);
 

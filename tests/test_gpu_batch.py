@@ -157,3 +157,44 @@ def test_batch_mixed_formats_and_empty():
             assert np.abs(Ga - Gb).max() < 1e-8
         qcm.erase_model_instance(la)
         qcm.erase_model_instance(lb)
+
+
+@pytest.mark.parametrize("nx,ny,nb,N,S,npts", [(2, 2, 4, 8, 0, 1), (2, 2, 4, 7, -1, 5), (2, 2, 5, 8, 0, 2),
+                                               (2, 3, 4, 6, 0, 2), (2, 2, 8, 4, 0, 3), (2, 2, 8, 6, 0, 1),
+                                               (2, 1, 16, 8, 8, 1)])
+def test_items_beyond_lds_match_single_solves(nx, ny, nb, N, S, npts):
+    """Sectors too large for LDS advance in lockstep: shapes with several rows
+    per workgroup pass (larger half basis up to 128 states), with one, and with
+    the spin-down half the larger (N odd or the fractions' targets), one item
+    and several per shape, ragged row counts.  Against the instance's own
+    solve: E0 to 1e-11 relative, G on the Matsubara axis to 1e-8 (the fractions
+    are 400 steps without reorthogonalization, which drift apart on the real
+    axis only)."""
+    wl = W.vca_cluster_bath(nx, ny, nb, N=N)
+    sector = "R0:N%d:S%d" % (N, S)
+    name = "wide_%d%d%d_%d" % (nx, ny, nb, N)
+    qcm.new_model(name, wl.n_sites, wl.n_bath)
+    for op, (typ, el) in wl.operators.items():
+        qcm.new_operator(name, op, typ, [(r + 1, c + 1, v) for (r, c, v) in el])
+    z = W.matsubara(24, 12.0)
+    qcm.set_global_parameterC("GF_method", "F")
+    qcm.set_global_parameterC("hv_variant", 1)  # the single solves' product: the row kernel, for every shape
+    try:
+        pts = [{**wl.values, **v} for v in W.vca_points(npts, seed=11)]
+        labs = list(range(30100, 30100 + npts))
+        for lab, v in zip(labs, pts):
+            qcm.new_model_instanceC(name, v, sector, lab)
+        qcm.solve_batch(labs)
+        for lab, v in zip(labs, pts):
+            E = qcm.ground_state_solve(lab)[0]
+            G = [qcm.Green_function_grid(z, s, lab) for s in (0, 1)]
+            qcm.new_model_instanceC(name, v, sector, lab + 500)
+            E1 = qcm.ground_state_solve(lab + 500)[0]
+            assert abs(E - E1) < 1e-11 * abs(E1)
+            for s in (0, 1):
+                assert np.abs(G[s] - qcm.Green_function_grid(z, s, lab + 500)).max() < 1e-8
+            qcm.erase_model_instance(lab)
+            qcm.erase_model_instance(lab + 500)
+    finally:
+        qcm.set_global_parameterC("GF_method", "L")
+        qcm.set_global_parameterC("hv_variant", 0)
