@@ -134,6 +134,15 @@ constexpr uint32_t kFourWaveDim = 128;
 // workspace small.)
 constexpr size_t kWideBytes = size_t(192) << 20;
 
+// Target sectors of at most this many states: an instance's own continued
+// fractions run together too.  One after the other through the single-sector
+// recurrence, each step of each fraction pays two dependent launches (8-site
+// chain, 72 fractions of 3 920 states: 626 ms against 9.3 together; plaquette +
+// 7 bath, 213 444 states: 542 against 101; + 8 bath, 731 808: 260 against 173);
+// from there on one product fills the chip and its tuned kernels win (+ 9
+// bath, 2.9 M states: 1.24 s against 1.81 together).
+constexpr size_t kTogetherDim = size_t(1) << 20;
+
 // LDS decides between one workgroup an item and lockstep: a workgroup with
 // vectors in memory, the only other way to keep an item by itself, took 1.3 to
 // 8 times the lockstep's time over sectors of 2 450 to 108 900 states (64
@@ -176,7 +185,7 @@ void launch_wide(const TablePack &tabs, const std::vector<Item> &items, const st
       const int n = (int)std::min(len, sh.second.size() - g0);
       uint32_t emax = 0;
       for (int k = 0; k < n; ++k) emax = std::max(emax, tabs.longest_row(tab[sh.second[g0 + k]]));
-      const WideShape W = wide_shape(sh.first.first, sh.first.second, emax, n);
+      const WideShape W = wide_shape(sh.first.first, sh.first.second, emax);
       const size_t scal = 2 * (size_t)W.nwg + kWideScalars + ntri;
       DevBuf<double> u((size_t)nvec * dim * n), sc(scal * n);
       std::vector<WideItem> wi(n);
@@ -286,6 +295,86 @@ struct TableCache {
     return combine_tables(it->second, T);
   }
 };
+
+// device maps of c / c^dagger_a on a sector, built once per batched solve
+struct MapCache {
+  struct Set { DevBuf<int32_t> map; DevBuf<int8_t> sgn, upar; };
+  std::map<std::tuple<int, int, int, int, int>, std::unique_ptr<Set>> m;  // (L, Nup, Ndw, pm, a)
+  Set &get(int L, const Sector &src, int pm, int a) {
+    auto key = std::make_tuple(L, src.Nup(), src.Ndw(), pm, a);
+    auto it = m.find(key);
+    if (it != m.end()) return *it->second;
+    const CdagMaps C = cdag_maps(L, pm, a, src);
+    auto M = std::make_unique<Set>();
+    M->map.upload(C.map.empty() ? std::vector<int32_t>{-1} : C.map);
+    M->sgn.upload(C.sgn.empty() ? std::vector<int8_t>{1} : C.sgn);
+    M->upar.upload(C.upar.empty() ? std::vector<int8_t>{1} : C.upar);
+    return *(m[key] = std::move(M));
+  }
+};
+
+// all orbital pairs o1 >= o2, row by row
+std::vector<std::pair<int, int>> all_pairs(int ns) {
+  std::vector<std::pair<int, int>> p;
+  for (int o1 = 0; o1 < ns; ++o1)
+    for (int o2 = 0; o2 <= o1; ++o2) p.push_back({o1, o2});
+  return p;
+}
+
+// one item per orbital pair of c^{pm} on state st, the target sector and the
+// result arrays left to the caller
+void append_pairs(std::vector<BatchCFItem> &items, MapCache &maps, int L, const std::vector<std::pair<int, int>> &pairs,
+                  const State &st, int spin, int pm) {
+  for (const auto &p : pairs) {
+    const MapCache::Set &m0 = maps.get(L, st.sec, pm, p.first + spin * L);
+    BatchCFItem it;
+    it.gs = st.psi.p;
+    it.du_s = half_basis(L, st.sec.Nup())->dim;
+    it.spin = spin;
+    it.norb = p.second == p.first ? 1 : 2;
+    it.map[0] = m0.map.p;
+    it.sgn[0] = m0.sgn.p;
+    it.upar = m0.upar.p;
+    if (p.second != p.first) {
+      const MapCache::Set &m1 = maps.get(L, st.sec, pm, p.second + spin * L);
+      it.map[1] = m1.map.p;
+      it.sgn[1] = m1.sgn.p;
+    }
+    items.push_back(it);
+  }
+}
+
+// Runs the fractions of items (tab[k]: item k's sector in tabs, not uploaded
+// yet) into av (max_cf per item), bv (max_cf + 1) and out (2).
+void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::vector<int> &tab, int max_cf,
+                   double acc, DevBuf<double> &av, DevBuf<double> &bv, DevBuf<double> &out) {
+  std::vector<Cls> cls(items.size());
+  size_t lds_max = 0;
+  for (size_t k = 0; k < items.size(); ++k) {
+    const size_t b = tabs.lds(tab[k], kCfVectors, 0);
+    cls[k] = classify(b, tabs.offs[tab[k]].du * tabs.offs[tab[k]].dd);
+    if (cls[k] == kWide) tabs.use_wide(tab[k]);
+    else lds_max = std::max(lds_max, b);
+  }
+  tabs.upload();
+  vlog("batch: %zu continued-fraction items, tables and maps built", items.size());
+  av.alloc(std::max<size_t>((size_t)max_cf * items.size(), 1));
+  bv.alloc(std::max<size_t>((size_t)(max_cf + 1) * items.size(), 1));
+  out.alloc(std::max<size_t>(2 * items.size(), 1));
+  for (size_t k = 0; k < items.size(); ++k) {
+    BatchCFItem &it = items[k];
+    it.S = tabs.view(tab[k]);
+    it.a = av.p + (size_t)max_cf * k;
+    it.b = bv.p + (size_t)(max_cf + 1) * k;
+    it.out = out.p + 2 * k;
+  }
+  launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds) {
+    batch_cf(d, n, block, lds, max_cf, acc, stream());
+  });
+  launch_wide(tabs, items, cls, tab, 2, 0, [&](const WideShape &W, const WideItem *w, const BatchCFItem *q, int n) {
+    wide_cf(W, w, q, n, max_cf, acc, stream());
+  });
+}
 
 bool batchable(const Instance &I) {
   const Params &P = params();
@@ -409,26 +498,16 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
   if (cf.empty()) return;
   TablePack tabs;
   std::map<std::pair<Instance *, Sector>, int> tab_of;
-  struct MapSet { DevBuf<int32_t> map; DevBuf<int8_t> sgn, upar; };
-  std::map<std::tuple<int, int, int, int, int>, std::unique_ptr<MapSet>> maps;  // (L, Nup, Ndw, pm, a)
-  auto get_maps = [&](int L, const Sector &src, int pm, int a) -> MapSet & {
-    auto key = std::make_tuple(L, src.Nup(), src.Ndw(), pm, a);
-    auto it = maps.find(key);
-    if (it != maps.end()) return *it->second;
-    const CdagMaps C = cdag_maps(L, pm, a, src);
-    auto M = std::make_unique<MapSet>();
-    M->map.upload(C.map.empty() ? std::vector<int32_t>{-1} : C.map);
-    M->sgn.upload(C.sgn.empty() ? std::vector<int8_t>{1} : C.sgn);
-    M->upar.upload(C.upar.empty() ? std::vector<int8_t>{1} : C.upar);
-    return *(maps[key] = std::move(M));
-  };
-  struct CFRef { Instance *I; State *st; int spin, pm, idx; uint32_t dim; int tab; int fid; };
+  MapCache maps;
+  struct CFRef { State *st; int pm; int fid; };
   std::vector<CFRef> refs;
   std::vector<BatchCFItem> items;
+  std::vector<int> tab;
   auto store = std::make_shared<CfStore>();
   int nfrac = 0;
   for (Instance *I : cf) {
     const int L = I->model->L, ns = I->model->n_sites;
+    const auto pairs = all_pairs(ns);
     const TermList T = I->terms();
     for (auto &stp : I->states) {
       State &st = *stp;
@@ -445,63 +524,20 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
           if (!sector_valid(L, tgt)) continue;
           const size_t dt = sector_dim(L, tgt);
           if (dt == 0) continue;
+          if (dt > 0xffffffffull) fail(ED_ERR_UNSUPPORTED, "batched sector too large");
           auto key = std::make_pair(I, tgt);
           auto ti = tab_of.find(key);
-          const int tab = ti != tab_of.end() ? ti->second : (tab_of[key] = tabs.add(cache.get(T, tgt)));
-          const uint32_t du_s = half_basis(L, st.sec.Nup())->dim;
-          std::vector<MapSet *> mo(ns);
-          for (int o = 0; o < ns; ++o) mo[o] = &get_maps(L, st.sec, pm, o + spin * L);
-          int idx = 0;
-          for (int o1 = 0; o1 < ns; ++o1)
-            for (int o2 = 0; o2 <= o1; ++o2, ++idx) {
-              BatchCFItem it;
-              it.gs = st.psi.p;
-              it.du_s = du_s;
-              it.spin = spin;
-              it.norb = o2 == o1 ? 1 : 2;
-              MapSet &m1 = *mo[o1];
-              it.map[0] = m1.map.p;
-              it.sgn[0] = m1.sgn.p;
-              it.upar = m1.upar.p;
-              if (o2 != o1) {
-                MapSet &m2 = *mo[o2];
-                it.map[1] = m2.map.p;
-                it.sgn[1] = m2.sgn.p;
-              }
-              items.push_back(it);
-              refs.push_back({I, &st, spin, pm, idx, (uint32_t)dt, tab, G.frac0 + 2 * idx + (pm == 1 ? 0 : 1)});
-            }
+          const int t = ti != tab_of.end() ? ti->second : (tab_of[key] = tabs.add(cache.get(T, tgt)));
+          append_pairs(items, maps, L, pairs, st, spin, pm);
+          tab.resize(items.size(), t);
+          for (int idx = 0; (int)refs.size() < (int)items.size(); ++idx)
+            refs.push_back({&st, pm, G.frac0 + 2 * idx + (pm == 1 ? 0 : 1)});
         }
       }
     }
   }
-  std::vector<Cls> cls(refs.size());
-  std::vector<int> tab(refs.size());
-  size_t lds_max = 0;
-  for (size_t k = 0; k < refs.size(); ++k) {
-    const size_t b = tabs.lds(refs[k].tab, kCfVectors, 0);
-    cls[k] = classify(b, refs[k].dim);
-    tab[k] = refs[k].tab;
-    if (cls[k] == kWide) tabs.use_wide(tab[k]);
-    else lds_max = std::max(lds_max, b);
-  }
-  tabs.upload();
-  vlog("batch: %zu continued-fraction items, tables and maps built", refs.size());
-  DevBuf<double> av(std::max<size_t>((size_t)max_cf * refs.size(), 1)),
-      bv(std::max<size_t>((size_t)(max_cf + 1) * refs.size(), 1)), out(std::max<size_t>(2 * refs.size(), 1));
-  for (size_t k = 0; k < refs.size(); ++k) {
-    BatchCFItem &it = items[k];
-    it.S = tabs.view(refs[k].tab);
-    it.a = av.p + (size_t)max_cf * k;
-    it.b = bv.p + (size_t)(max_cf + 1) * k;
-    it.out = out.p + 2 * k;
-  }
-  launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds) {
-    batch_cf(d, n, block, lds, max_cf, acc_cf, stream());
-  });
-  launch_wide(tabs, items, cls, tab, 2, 0, [&](const WideShape &W, const WideItem *w, const BatchCFItem *q, int n) {
-    wide_cf(W, w, q, n, max_cf, acc_cf, stream());
-  });
+  DevBuf<double> av, bv, out;
+  run_fractions(tabs, items, tab, max_cf, acc_cf, av, bv, out);
   const std::vector<double> res = out.to_host();
   // the store: fraction f holds n_f coefficients (0 where psi vanished or no
   // target sector exists)
@@ -541,6 +577,50 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
   vlog("batch: %zu continued fractions built and stored on the device (%zu coefficients)", refs.size(), total);
   for (Instance *I : cf) I->gf_solved = true;
   vlog("batch: continued fractions stored");
+}
+
+bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin) {
+  Params &P = params();
+  if ((I.format != 'G' && I.format != 'F') || P.geti("lanczos_block") == 0 || P.getb("lanczos_reorth") ||
+      P.geti("max_iter_CF") <= 0 || !terms_factorizable(T))
+    return false;
+  for (int pm = -1; pm <= 1; pm += 2) {
+    const Sector tgt = shift_sector(st.sec, pm, spin);
+    if (sector_valid(I.model->L, tgt) && sector_dim(I.model->L, tgt) > kTogetherDim) return false;
+  }
+  return true;
+}
+
+std::vector<Fraction> state_fractions(const Instance &I, const TermList &T, const State &st, int spin,
+                                      const std::vector<std::pair<int, int>> &pairs, int max_cf) {
+  const int L = I.model->L;
+  TablePack tabs;
+  MapCache maps;
+  std::vector<BatchCFItem> items;
+  std::vector<int> tab, at;
+  std::vector<Fraction> F(2 * pairs.size());
+  for (int pm = -1; pm <= 1; pm += 2) {
+    const Sector tgt = shift_sector(st.sec, pm, spin);
+    if (!sector_valid(L, tgt) || sector_dim(L, tgt) == 0) continue;
+    append_pairs(items, maps, L, pairs, st, spin, pm);
+    tab.resize(items.size(), tabs.add(factorized_tables(T, tgt)));
+    for (size_t k = 0; k < pairs.size(); ++k) at.push_back(2 * (int)k + (pm < 0));
+  }
+  if (items.empty()) return F;
+  DevBuf<double> av, bv, out;
+  run_fractions(tabs, items, tab, max_cf, params().getd("accur_continued_fraction"), av, bv, out);
+  const std::vector<double> a = av.to_host(), b = bv.to_host(), res = out.to_host();
+  for (size_t k = 0; k < items.size(); ++k) {
+    const int n = (int)res[2 * k];
+    if (n <= 0) continue;  // psi vanishes
+    const double *ak = a.data() + (size_t)max_cf * k, *bk = b.data() + (size_t)(max_cf + 1) * k;
+    Fraction &f = F[at[k]];
+    f.norm2 = res[2 * k + 1];
+    f.a.assign(ak, ak + n);
+    f.b.assign(bk, bk + n + 1);
+    f.b[0] = 1.0;
+  }
+  return F;
 }
 
 }  // namespace ed

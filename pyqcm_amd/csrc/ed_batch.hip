@@ -866,30 +866,23 @@ void batch_cf(const BatchCFItem *d_items, int n, int block, size_t lds, int max_
   ED_HIP(hipGetLastError());
 }
 
-WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax, int nitems) {
+WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax) {
   WideShape W;
   W.emax = emax;
   W.swap = dd > du;
   W.nl = W.swap ? dd : du;
   W.nr = W.swap ? du : dd;
-  int rg = 1;
   const size_t row = W.nl * sizeof(double);
-  if (row > kWideLdsMax) {
-    W.rpt = 1;
-  } else if (W.nl > (uint32_t)kWideBlock / 2) {
-    // one row at a time per thread column; eight rows share a table load
-    W.rpt = 8;
-    while (W.rpt > 1 && W.rpt * row > 64 * 1024) W.rpt /= 2;
-  } else {
-    rg = kWideBlock / (int)W.nl;
-    W.rpt = 4;
-  }
-  // fewer rows per thread where that leaves compute units without a workgroup
-  auto groups = [&](int rpt) { return (int)((W.nr + rg * rpt - 1) / (rg * rpt)); };
-  while (W.rpt > 1 && (long)nitems * groups(W.rpt) < 1024) W.rpt /= 2;
-  W.rows = rg * W.rpt;
-  W.nwg = groups(W.rpt);
   W.stage = row <= kWideLdsMax;
+  // rows longer than half a workgroup: one row at a time per thread column,
+  // four rows sharing a table load; shorter ones several side by side.  The
+  // split depends on the sector alone, so an item's sums, and its fraction to
+  // the last bit, do not depend on what runs beside it.
+  const int rg = W.nl > (uint32_t)kWideBlock / 2 ? 1 : kWideBlock / (int)W.nl;
+  W.rpt = rg > 1 ? 2 : 4;
+  while (W.rpt > 1 && (!W.stage || W.rpt * row > 64 * 1024)) W.rpt /= 2;
+  W.rows = rg * W.rpt;
+  W.nwg = (int)((W.nr + W.rows - 1) / W.rows);
   W.lds = ((size_t)W.rows * emax + ((size_t)W.rows * emax + 1) / 2) * sizeof(double) + (W.stage ? W.rows * row : 0);
   return W;
 }
@@ -909,11 +902,7 @@ void wide_hv(const WideShape &W, const WideItem *items, int n, int k, int max_k,
                        items, n, W.nwg, W.nl, W.nr, rg, W.emax, k, max_k, acc);                                          \
   } while (0)
   if (!W.stage) ED_WIDE(1, true, false);
-  else if (rg > 1) {
-    if (W.rpt == 4) ED_WIDE(4, false, true);
-    else if (W.rpt == 2) ED_WIDE(2, false, true);
-    else ED_WIDE(1, false, true);
-  } else if (W.rpt == 8) ED_WIDE(8, true, true);
+  else if (rg > 1) ED_WIDE(2, false, true);
   else if (W.rpt == 4) ED_WIDE(4, true, true);
   else if (W.rpt == 2) ED_WIDE(2, true, true);
   else ED_WIDE(1, true, true);

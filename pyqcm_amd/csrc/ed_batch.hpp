@@ -89,7 +89,7 @@ struct WideShape {
   bool stage = true;  // rows fit in LDS (else read from memory)
   size_t lds = 0;
 };
-WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax, int nitems);
+WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax);
 
 // continued fractions of n items of one shape; src[k] is item k's start state
 void wide_cf(const WideShape &W, const WideItem *items, const BatchCFItem *src, int n, int max_cf, double acc,
@@ -115,5 +115,22 @@ void batch_cf_store(int nitems, int max_cf, const double *out, const double *a, 
 // instance; factorizable instances using Lanczos + continued fractions run
 // batched, the others through their own solve
 void solve_batch(const std::vector<Instance *> &insts, bool want_gf);
+
+// One LanczosGreen run: alpha_n and beta_{n-1} (b[0] = 1, one entry more than
+// a) and the start vector's squared norm; empty where that vanishes.
+struct Fraction {
+  std::vector<double> a, b;
+  double norm2 = 0.0;
+};
+struct State;
+struct TermList;
+// whether an instance's fractions from state st run as a batch (the same
+// recurrence and stop rule as lanczos_green, all orbital pairs together)
+bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin);
+// the fractions of c^{pm}_o1 (+ c^{pm}_o2) |st> for the given pairs, at most
+// max_cf levels: entry 2 k + (pm < 0) for pair k; the hole and the electron
+// part run together.  Empty where the target sector is invalid or empty.
+std::vector<Fraction> state_fractions(const Instance &I, const TermList &T, const State &st, int spin,
+                                      const std::vector<std::pair<int, int>> &pairs, int max_cf);
 
 }  // namespace ed

@@ -11,6 +11,7 @@
 #include <random>
 #include <sstream>
 
+#include "ed_batch.hpp"
 #include "ed_dense.hpp"
 #include "ed_solvers.hpp"
 
@@ -985,6 +986,15 @@ static void build_gf_complex(Instance &I, State &st, int spin) {
   }
 }
 
+// coefficients as continued_fraction's constructor leaves them
+// (src_ed/continued_fraction.cpp:33-42): a shifted by the state energy (negated
+// for holes), b squared, b_0 the weighted norm
+static void as_evaluated(Fraction &f, int pm, const State &st) {
+  for (auto &x : f.b) x *= x;
+  f.b[0] = f.norm2 * st.weight;
+  for (auto &x : f.a) x = pm == 1 ? x - st.energy : st.energy - x;
+}
+
 static void build_gf(Instance &I, State &st, int spin) {
   if (I.complex_hs()) {
     build_gf_complex(I, st, spin);
@@ -1073,6 +1083,21 @@ static void build_gf(Instance &I, State &st, int spin) {
     Vh.swap(h.second);
     ee.swap(e.first);
     Ve.swap(e.second);
+  }
+  if (G.kind == 'F' && fractions_together(I, T, st, spin)) {
+    // build_cf (src_ed/model_instance.cpp:35-100) for all pairs at once
+    check_cancel();
+    std::vector<std::pair<int, int>> pairs;
+    for (int o1 = 0; o1 < ns; ++o1)
+      for (int o2 = 0; o2 <= o1; ++o2) pairs.push_back({o1, o2});
+    std::vector<Fraction> fr = state_fractions(I, T, st, spin, pairs, (int)params().geti("max_iter_CF"));
+    for (int k = 0; k < 2 * np; ++k) {
+      if (fr[k].a.empty()) continue;
+      as_evaluated(fr[k], k & 1 ? -1 : 1, st);
+      (k & 1 ? G.ha : G.ea)[k / 2] = std::move(fr[k].a);
+      (k & 1 ? G.hb : G.eb)[k / 2] = std::move(fr[k].b);
+    }
+    return;
   }
   for (int pm = -1; pm <= 1 && G.kind != 'L'; pm += 2) {
     check_cancel();
@@ -1241,6 +1266,18 @@ void cf_pairs(Instance &I, int spin, const std::vector<std::pair<int, int>> &pai
   const TermList T = I.terms();
   a.assign(2 * pairs.size(), {});
   b.assign(2 * pairs.size(), {});
+  if (cap > 0 && fractions_together(I, T, st, sp)) {
+    check_cancel();
+    std::vector<Fraction> fr = state_fractions(I, T, st, sp, pairs, cap);
+    for (size_t k = 0; k < fr.size(); ++k) {
+      if (fr[k].a.empty()) continue;
+      as_evaluated(fr[k], k & 1 ? -1 : 1, st);
+      fr[k].b.resize(fr[k].a.size());
+      a[k] = std::move(fr[k].a);
+      b[k] = std::move(fr[k].b);
+    }
+    return;
+  }
   for (int pm = -1; pm <= 1; pm += 2) {
     check_cancel();
     const Sector tgt = shift_sector(st.sec, pm, sp);
