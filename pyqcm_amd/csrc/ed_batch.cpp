@@ -120,9 +120,15 @@ void wide_coefficients(const BatchGSItem &, double *tri, size_t M, WideItem &w) 
   w.b = tri + M - 1;
 }
 
-// execution class of an item: from LDS with one or four waves, or with the
-// other items of its shape in lockstep
-enum Cls { kLds = 0, kLdsFour = 1, kWide = 2 };
+// execution class of an item: from LDS with one or four waves, with the other
+// items of its shape in lockstep, or (fractions) from registers
+enum Cls { kLds = 0, kLdsFour = 1, kWide = 2, kTile = 3 };
+constexpr int kLdsClasses = 2;
+// Both halves up to two tiles of 16: the register kernel at any size (512
+// points of the 2x3 sweep, 225-400 states: 67 ms of LDS kernels -> 31 ms; 2x2
+// with 2 bath orbitals 34.3 -> 26.5 ms a whole sweep, with 1 23.6 -> 20.7; 24 -
+// 36 states, where neither kernel counts: level).
+constexpr uint32_t kTileDim = 32;
 
 // items held in LDS with at least this many states get four waves (the
 // steps are latency-bound; more waves per item hide more of it)
@@ -156,16 +162,31 @@ Cls classify(size_t lds, uint32_t dim) {
 // one launch per LDS class
 template <typename Item, typename Launch>
 void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls, size_t lds_max, Launch launch) {
-  std::vector<Item> part[kWide];
+  std::vector<Item> part[kLdsClasses];
   for (size_t k = 0; k < items.size(); ++k)
-    if (cls[k] != kWide) part[cls[k]].push_back(items[k]);
-  DevBuf<Item> d[kWide];
-  for (int c = 0; c < kWide; ++c) {
+    if (cls[k] < kLdsClasses) part[cls[k]].push_back(items[k]);
+  DevBuf<Item> d[kLdsClasses];
+  for (int c = 0; c < kLdsClasses; ++c) {
     if (part[c].empty()) continue;
     d[c].upload(part[c]);
     launch(d[c].p, (int)part[c].size(), c == kLdsFour ? 256 : 64, lds_max);
   }
   sync();
+}
+
+// the register-tile fractions, by tile shape
+void launch_tiles(const TablePack &tabs, const std::vector<BatchCFItem> &items, const std::vector<Cls> &cls,
+                  const std::vector<int> &tab, int max_cf, double acc) {
+  std::vector<BatchCFItem> part[2][2];
+  for (size_t k = 0; k < items.size(); ++k)
+    if (cls[k] == kTile) part[tabs.offs[tab[k]].dd > 16][tabs.offs[tab[k]].du > 16].push_back(items[k]);
+  DevBuf<BatchCFItem> d[2][2];
+  for (int r = 0; r < 2; ++r)
+    for (int c = 0; c < 2; ++c) {
+      if (part[r][c].empty()) continue;
+      d[r][c].upload(part[r][c]);
+      tile_cf(d[r][c].p, (int)part[r][c].size(), r + 1, c + 1, max_cf, acc, stream());
+    }
 }
 
 // The wide items (tab[k]: item k's sector), by shape and then in groups whose
@@ -351,6 +372,11 @@ void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::
   std::vector<Cls> cls(items.size());
   size_t lds_max = 0;
   for (size_t k = 0; k < items.size(); ++k) {
+    const TablePack::Off &o = tabs.offs[tab[k]];
+    if (o.du <= kTileDim && o.dd <= kTileDim) {
+      cls[k] = kTile;
+      continue;
+    }
     const size_t b = tabs.lds(tab[k], kCfVectors, 0);
     cls[k] = classify(b, tabs.offs[tab[k]].du * tabs.offs[tab[k]].dd);
     if (cls[k] == kWide) tabs.use_wide(tab[k]);
@@ -371,6 +397,7 @@ void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::
   launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds) {
     batch_cf(d, n, block, lds, max_cf, acc, stream());
   });
+  launch_tiles(tabs, items, cls, tab, max_cf, acc);
   launch_wide(tabs, items, cls, tab, 2, 0, [&](const WideShape &W, const WideItem *w, const BatchCFItem *q, int n) {
     wide_cf(W, w, q, n, max_cf, acc, stream());
   });

@@ -467,6 +467,195 @@ __global__ __launch_bounds__(BS) void k_batch_cf(const BatchCFItem *items, int m
 }
 
 // ---------------------------------------------------------------------------
+// Tile kernel: continued fractions of sectors of at most 32 x 32 half states.
+// One wave holds the vector X[i_dn][i_up] in registers as RT x CT tiles of
+// 16 x 16 and applies the one-body operators as small dense products on the
+// FP64 matrix cores: Y = K_dn X + X K_up^T on top of diag o X - beta X_prev as
+// the accumulator's start.  v_mfma_f64_16x16x4: lane l supplies A(l % 16,
+// l / 16) and B(l / 16, l % 16), and register r of D holds (4 r + l / 16,
+// l % 16), so register s % 4 of X's tile row s / 4 already is the B operand
+// of K_dn X's k-step s; only X K_up^T needs X in A order, one pass through
+// LDS.  No barriers, no table reads in a step: the sparse form read 12 bytes
+// of tables from LDS per hop beside 8 of the vector.
+// ---------------------------------------------------------------------------
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// x moved across lanes by a DPP control; lanes without a source give 0
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp0(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double((long long)hi << 32 | (unsigned)lo);
+}
+// wave sum, the same in every lane: shifts within rows of 16, then the row
+// sums handed on (no LDS permutes: their latency is most of a tile step)
+__device__ __forceinline__ double wsum_dpp(double v) {
+  v += dpp0<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v += dpp0<0x112, 0xf>(v);
+  v += dpp0<0x114, 0xf>(v);
+  v += dpp0<0x118, 0xf>(v);
+  v += dpp0<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v += dpp0<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double((long long)hi << 32 | (unsigned)lo);
+}
+
+// operand k[t][s] = K(16 t + lane % 16, 4 s + lane / 16) of the CSR matrix K
+// (n rows), spread densely over xt (16 T x 16 T, stride 16 T + 1) on the way
+template <int T>
+__device__ __forceinline__ void tile_operand(uint32_t n, const uint32_t *ptr, const uint32_t *col, const double *val,
+                                             double *xt, double (*k)[4 * T]) {
+  constexpr int S = 16 * T + 1;
+  const int lane = threadIdx.x;
+  __syncthreads();
+  for (int i = lane; i < 16 * T * S; i += kW) xt[i] = 0.0;
+  __syncthreads();
+  if ((uint32_t)lane < n)
+    for (uint32_t e = ptr[lane]; e < ptr[lane + 1]; ++e) xt[lane * S + col[e]] = val[e];
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int s = 0; s < 4 * T; ++s) k[t][s] = xt[(16 * t + lane % 16) * S + 4 * s + lane / 16];
+}
+
+template <int RT, int CT>
+__global__ __launch_bounds__(kW) void k_tile_cf(const BatchCFItem *items, int max_cf, double acc) {
+  constexpr int MT = RT > CT ? RT : CT, S = 16 * CT + 1;
+  __shared__ double xt[16 * MT * (16 * MT + 1)];
+  const BatchCFItem &itg = items[blockIdx.x];
+  const BatchSector G = itg.S;
+  const int lane = threadIdx.x, lr = lane / 16, lc = lane % 16;
+  double kd[RT][4 * RT], ku[CT][4 * CT];
+  tile_operand<RT>(G.dd, G.dn_ptr, G.dn_col, G.dn_val, xt, kd);
+  tile_operand<CT>(G.du, G.up_ptr, G.up_col, G.up_val, xt, ku);
+  const int nkr = (int)(G.dd + 3) / 4, nkc = (int)(G.du + 3) / 4;
+  // psi = c_o1 |gs> (+ c_o2 |gs>); padding stays zero throughout
+  f64x4 v[RT][CT], vp[RT][CT], dg[RT][CT];
+  double nn = 0.0;
+  {
+    const double *gs = itg.gs;
+    const uint32_t du_s = itg.du_s;
+    const int spin = itg.spin, norb = itg.norb;
+    const int32_t *map0 = itg.map[0], *map1 = itg.map[1];
+    const int8_t *sgn0 = itg.sgn[0], *sgn1 = itg.sgn[1], *upar = itg.upar;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t id = 16 * t + 4 * r + lr, iu = 16 * c + lc;
+          double x = 0.0, d = 0.0;
+          if (id < G.dd && iu < G.du) {
+            d = G.diag[id * G.du + iu];
+            const uint32_t im = spin == 0 ? iu : id;
+            const int32_t s0 = map0[im];
+            if (s0 >= 0)
+              x += (double)sgn0[im] * gs[spin == 0 ? (size_t)s0 + (size_t)du_s * id : iu + (size_t)du_s * s0];
+            if (norb == 2) {
+              const int32_t s1 = map1[im];
+              if (s1 >= 0)
+                x += (double)sgn1[im] * gs[spin == 0 ? (size_t)s1 + (size_t)du_s * id : iu + (size_t)du_s * s1];
+            }
+            if (spin == 1) x *= (double)upar[iu];
+          }
+          v[t][c][r] = x;
+          vp[t][c][r] = 0.0;
+          dg[t][c][r] = d;
+          nn += x * x;
+        }
+  }
+  nn = wsum_dpp(nn);
+  if (!(nn > 1e-14)) {
+    if (lane == 0) {
+      itg.out[0] = -1.0;
+      itg.out[1] = nn;
+    }
+    return;
+  }
+  const double inv = 1.0 / sqrt(nn);
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) v[t][c] *= inv;
+  double *av = itg.a, *bv = itg.b;
+  if (lane == 0) bv[0] = 1.0;
+  int n = 0;
+  double bprev = 0.0, prod = 1.0, blast = 1.0;
+  while (prod > acc && fabs(blast) > acc && n < max_cf) {
+    f64x4 y[RT][CT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        y[t][c] = dg[t][c] * v[t][c] - bprev * vp[t][c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xt[(16 * t + 4 * r + lr) * S + 16 * c + lc] = v[t][c][r];
+      }
+#pragma unroll
+    for (int s = 0; s < 4 * RT; ++s)
+      if (s < nkr)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int c = 0; c < CT; ++c)
+            y[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(kd[t][s], v[s / 4][c][s % 4], y[t][c], 0, 0, 0);
+    __syncthreads();  // one wave: orders the LDS writes before the reads
+#pragma unroll
+    for (int s = 0; s < 4 * CT; ++s)
+      if (s < nkc)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          const double a = xt[(16 * t + lc) * S + 4 * s + lr];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) y[t][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, ku[c][s], y[t][c], 0, 0, 0);
+        }
+    __syncthreads();
+    double dot = 0.0;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dot += y[t][c][r] * v[t][c][r];
+    const double alpha = wsum_dpp(dot);
+    double n2 = 0.0;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        y[t][c] -= alpha * v[t][c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) n2 += y[t][c][r] * y[t][c][r];
+      }
+    const double beta = sqrt(wsum_dpp(n2));
+    if (lane == 0) {
+      av[n] = alpha;
+      bv[n + 1] = beta;
+    }
+    prod *= fabs(beta);
+    blast = beta;
+    bprev = beta;
+    ++n;
+    const double ib = 1.0 / beta;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        vp[t][c] = v[t][c];
+        v[t][c] = y[t][c] * ib;
+      }
+  }
+  if (lane == 0) {
+    itg.out[0] = (double)n;
+    itg.out[1] = nn;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // wide items.  The vectors stay unnormalized as in the device-driven
 // single-sector recurrence: U_k = beta_{k-1} v_k (U_0 the start vector, its
 // norm in place of beta_{-1}), buffer k & 1 holding U_k.  Step k is
@@ -964,6 +1153,18 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
   for (int scale = 0; scale < 2; ++scale)
     hipLaunchKernelGGL(k_wide_gs_out, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap,
                        scale);
+  ED_HIP(hipGetLastError());
+}
+
+void tile_cf(const BatchCFItem *d_items, int n, int rt, int ct, int max_cf, double acc, hipStream_t s) {
+  if (n <= 0) return;
+  if (rt < 1 || rt > 2 || ct < 1 || ct > 2) fail(ED_ERR_INTERNAL, "tile_cf: sector beyond 32 x 32 half states");
+#define ED_TILE(R, C) hipLaunchKernelGGL((k_tile_cf<R, C>), dim3(n), dim3(kW), 0, s, d_items, max_cf, acc)
+  if (rt == 1 && ct == 1) ED_TILE(1, 1);
+  else if (rt == 1) ED_TILE(1, 2);
+  else if (ct == 1) ED_TILE(2, 1);
+  else ED_TILE(2, 2);
+#undef ED_TILE
   ED_HIP(hipGetLastError());
 }
 

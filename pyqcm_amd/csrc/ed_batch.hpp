@@ -104,6 +104,10 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
 void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, int max_iter, double accur, hipStream_t s);
 void batch_cf(const BatchCFItem *d_items, int n, int block, size_t lds, int max_cf, double acc, hipStream_t s);
 
+// fractions of sectors of at most 16 rt down and 16 ct up half states (rt, ct
+// in 1, 2): vectors in registers, one wave an item
+void tile_cf(const BatchCFItem *d_items, int n, int rt, int ct, int max_cf, double acc, hipStream_t s);
+
 // writes item k's continued fraction (out[2k] = n steps, out[2k + 1] =
 // ||psi||^2), transformed with the state's energy e0[k], weight w[k] and
 // electron / hole pm[k], into a continued-fraction store at off[fid[k]]

@@ -198,3 +198,37 @@ def test_items_beyond_lds_match_single_solves(nx, ny, nb, N, S, npts):
     finally:
         qcm.set_global_parameterC("GF_method", "L")
         qcm.set_global_parameterC("hv_variant", 0)
+
+
+@pytest.mark.parametrize("nb", [1, 13, 14, 15, 28])
+def test_register_tiles_at_their_edges(nb):
+    """Fractions whose halves have 3, 15, 16, 17 and 30 states (one up electron,
+    so that adding a down one leads to an L x L sector): partial, full and
+    two-tile register kernels against the host-driven recurrence
+    (lanczos_block 0), which runs the row product; also the sectors around
+    them (1 state, L, and L (L - 1) / 2 x 1).  Matsubara axis, 1e-9: the
+    recurrences differ by rounding only."""
+    wl = W.vca_cluster_bath(2, 1, nb, N=1)
+    name = "tile_%d" % nb
+    qcm.new_model(name, wl.n_sites, wl.n_bath)
+    for op, (typ, el) in wl.operators.items():
+        qcm.new_operator(name, op, typ, [(r + 1, c + 1, v) for (r, c, v) in el])
+    z = W.matsubara(16, 8.0)
+    vals = {**wl.values, "U": 5.0, "M": 0.3, "mu": 1.0}
+    qcm.set_global_parameterC("GF_method", "F")
+    qcm.set_global_parameterC("hv_variant", 1)
+    try:
+        for lab, block in ((30900, 12), (30901, 0)):
+            qcm.set_global_parameterC("lanczos_block", block)
+            qcm.new_model_instanceC(name, vals, "R0:N1:S1", lab)
+            qcm.ground_state_solve(lab)
+            qcm.Green_function_solveC(lab)
+        for s in (0, 1):
+            a, b = (qcm.Green_function_grid(z, s, lab) for lab in (30900, 30901))
+            assert np.abs(a - b).max() < 1e-9
+    finally:
+        qcm.set_global_parameterC("lanczos_block", 12)
+        qcm.set_global_parameterC("GF_method", "L")
+        qcm.set_global_parameterC("hv_variant", 0)
+        for lab in (30900, 30901):
+            qcm.erase_model_instance(lab)
