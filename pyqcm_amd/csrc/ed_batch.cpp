@@ -532,13 +532,15 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
   std::vector<int> tab;
   auto store = std::make_shared<CfStore>();
   int nfrac = 0;
-  for (Instance *I : cf) {
-    const int L = I->model->L, ns = I->model->n_sites;
-    const auto pairs = all_pairs(ns);
-    const TermList T = I->terms();
-    for (auto &stp : I->states) {
-      State &st = *stp;
-      for (int spin = 0; spin < ((I->mixing & 4) ? 2 : 1); ++spin) {
+  // numbered spin by spin: a Green-function call evaluates one spin's run of fractions
+  for (int spin = 0; spin < 2; ++spin) {
+    for (Instance *I : cf) {
+      if (spin && !(I->mixing & 4)) continue;
+      const int L = I->model->L, ns = I->model->n_sites;
+      const auto pairs = all_pairs(ns);
+      const TermList T = I->terms();
+      for (auto &stp : I->states) {
+        State &st = *stp;
         GFRep &G = st.gf[spin];
         G = GFRep();
         G.kind = 'F';
