@@ -14,6 +14,8 @@
 namespace ed {
 
 namespace {
+// row pitch of the feature-major matrices: whole k-steps of 32
+long rows_pitch(int B) { return (B + 31) / 32 * 32; }
 int round8(int n) { return (n + 7) / 8 * 8; }
 
 // deterministic standard normals (Box-Muller on a 64-bit Mersenne twister), so
@@ -54,6 +56,7 @@ Surrogate::Surrogate(int ni, int no, int w, int d, uint64_t seed) : n_in(ni), n_
     L.out = l == d ? no : w;
     L.in_pad = round8(L.in);
     L.out_pad = round8(L.out);
+    L.out32 = (L.out + 31) / 32 * 32;
     const size_t nw = (size_t)L.out_pad * L.in_pad;
     std::vector<float> W(nw, 0.f), b(L.out_pad, 0.f);
     const double sc = 1.0 / std::sqrt((double)L.in);
@@ -69,9 +72,17 @@ Surrogate::Surrogate(int ni, int no, int w, int d, uint64_t seed) : n_in(ni), n_
       B->alloc(L.out_pad);
       zero(B->p, L.out_pad);
     }
-    L.Wb.alloc(nw);
-    mlp_to_bf16(nw, L.W.p, L.Wb.p, stream());
+    // (the row-block kernels read up to a layer width past the last row)
+    L.Wb.alloc(nw + kMlpSpare);
+    zero(L.Wb.p, L.Wb.n);
+    L.Wt.alloc((size_t)L.in_pad * L.out32 + kMlpSpare);
+    zero(L.Wt.p, L.Wt.n);
   }
+  copy_weights();
+  // the range of the row-block kernels; other widths, deeper or wider networks
+  // run layer by layer
+  rows_ok = (w == 64 || w == 128 || w == 256) && d < kMlpLayers && layers[0].in_pad <= w &&
+            mlp_rows_lds(w, d, no, true) <= kMlpRowsLds;
   x_mean.assign(ni, 0.0);
   x_std.assign(ni, 1.0);
   y_mean.assign(no, 0.0);
@@ -127,15 +138,121 @@ void Surrogate::set_weights(const double *w) {
     for (int o = 0; o < L.out; ++o) b[o] = (float)w[k++];
     L.W.upload(W);
     L.b.upload(b);
-    mlp_to_bf16(W.size(), L.W.p, L.Wb.p, stream());
     // a new starting point: the optimizer restarts
     zero(L.mW.p, L.mW.n);
     zero(L.vW.p, L.vW.n);
     zero(L.mb.p, L.mb.n);
     zero(L.vb.p, L.vb.n);
   }
+  copy_weights();
   adam_t = 0;
   sync();
+}
+
+void Surrogate::copy_weights() {
+  for (Layer &L : layers) mlp_copies(L.out, L.in, L.in_pad, L.out32, L.W.p, L.Wb.p, L.Wt.p, stream());
+}
+
+MlpRows Surrogate::rows_args(int B, const bf16_t *X, const float *T, const int *idx) {
+  MlpRows P;
+  P.depth = depth;
+  P.n_in = n_in;
+  P.n_out = n_out;
+  P.in_pad = layers[0].in_pad;
+  P.out_pad = layers[depth].out_pad;
+  P.out32 = layers[depth].out32;
+  P.B = B;
+  P.Bp = rows_pitch(B);
+  for (int l = 0; l <= depth; ++l) {
+    P.W[l] = layers[l].Wb.p;
+    P.Wt[l] = layers[l].Wt.p;
+    P.bias[l] = layers[l].b.p;
+  }
+  P.X = X;
+  P.T = T;
+  P.lw = dloss_w.p;
+  P.idx = idx;
+  P.scale = 2.f / (float)B;
+  P.actT = actT.p;
+  P.dzT = dzT.p;
+  P.db = db.p;
+  return P;
+}
+
+MlpShape Surrogate::shape() const {
+  MlpShape S;
+  S.nl = depth + 1;
+  for (int l = 0; l <= depth; ++l) {
+    const Layer &L = layers[l];
+    S.in[l] = L.in;
+    S.out[l] = L.out;
+    S.aoff[l] = l == 0 ? 0 : n_in + (long)(l - 1) * width;
+    S.zoff[l] = (long)l * width;
+    S.t0[l + 1] = S.t0[l] + ((L.out + 31) / 32) * ((L.in + 63) / 64);
+    S.poff[l + 1] = S.poff[l] + (long)L.out * L.in;
+  }
+  S.zoff[depth + 1] = (long)depth * width + n_out;
+  S.nw = S.poff[depth + 1];
+  return S;
+}
+
+MlpParams Surrogate::param_table() {
+  MlpParams Q = {};
+  for (int l = 0; l <= depth; ++l) {
+    Layer &L = layers[l];
+    Q.W[l] = L.W.p;
+    Q.b[l] = L.b.p;
+    Q.mW[l] = L.mW.p;
+    Q.vW[l] = L.vW.p;
+    Q.mb[l] = L.mb.p;
+    Q.vb[l] = L.vb.p;
+    Q.gW[l] = L.gW.p;
+    Q.gb[l] = L.gb.p;
+    Q.Wb[l] = L.Wb.p;
+    Q.Wt[l] = L.Wt.p;
+    Q.in_pad[l] = L.in_pad;
+    Q.out32[l] = L.out32;
+  }
+  return Q;
+}
+
+// batch splits of the weight gradients: 512 rows each, at most 4 (12 -> 256 x 4
+// -> 641 at a batch of 2 048, gradient + update launch: 1 split 51 + 8 us, 2 28
+// + 8, 4 17 + 8, 8 17 + 9, 16 15 + 11)
+int Surrogate::rows_splits(int B) const { return std::max(1, std::min(4, B / 512)); }
+
+void Surrogate::ensure_rows(int B) {
+  if (B <= cap_rows) return;
+  const long Bp = rows_pitch(B), nb = (B + 31) / 32 * 2;
+  actT.alloc((size_t)(n_in + depth * width) * Bp);
+  dzT.alloc((size_t)(depth * width + n_out) * Bp);
+  db.alloc((size_t)(depth * width + n_out) * nb);
+  slab.alloc((size_t)rows_splits(B) * shape().nw);
+  part.alloc(1024);
+  cap_rows = B;
+}
+
+int Surrogate::rows_step(int B, const bf16_t *X, const float *T, const int *idx, float *loss, const MlpAdam *h) {
+  ensure_rows(B);
+  MlpRows P = rows_args(B, X, T, idx);
+  P.loss = loss;
+  const MlpShape S = shape();
+  const int nb = mlp_rows(P, width, true, stream()), ns = rows_splits(B);
+  mlp_wgrad(S, ns, (B + 31) / 32, P.Bp, actT.p, dzT.p, slab.p, stream());
+  mlp_update(S, param_table(), h, ns, nb, slab.p, db.p, stream());
+  return nb;
+}
+
+MlpAdam Surrogate::next_adam() {
+  ++adam_t;
+  MlpAdam h;
+  h.lr = (float)lr;
+  h.b1 = (float)beta1;
+  h.b2 = (float)beta2;
+  h.eps = (float)eps;
+  h.c1 = (float)(1.0 - std::pow(beta1, (double)adam_t));
+  h.c2 = (float)(1.0 - std::pow(beta2, (double)adam_t));
+  return h;
 }
 
 void Surrogate::ensure_batch(int B) {
@@ -164,6 +281,12 @@ void Surrogate::ensure_batch(int B) {
 }
 
 void Surrogate::forward(int B, const bf16_t *x) {
+  if (use_rows(B)) {
+    MlpRows P = rows_args(B, x, nullptr, nullptr);
+    P.y = y.p;
+    mlp_rows(P, width, false, stream());
+    return;
+  }
   for (int l = 0; l <= depth; ++l) {
     const Layer &L = layers[l];
     GemmArgs g;
@@ -250,21 +373,25 @@ int Surrogate::backward(int B, float *partials) {
 }
 
 double Surrogate::loss_and_grad(int B) {
-  const int nb = backward(B, part.p);
+  int nb;
+  if (use_rows(B)) {
+    nb = rows_step(B, xb.p, t.p, nullptr, part.p, nullptr);
+  } else {
+    forward(B, xb.p);
+    nb = backward(B, part.p);
+  }
   std::vector<float> hp(nb);
   part.download(hp.data(), nb);
   return mlp_fold(hp.data(), nb) / B;
 }
 
 void Surrogate::adam_step() {
-  ++adam_t;
-  const float c1 = (float)(1.0 - std::pow(beta1, (double)adam_t)), c2 = (float)(1.0 - std::pow(beta2, (double)adam_t));
+  const MlpAdam h = next_adam();
   for (Layer &L : layers) {
-    mlp_adam(L.W.n, L.W.p, L.gW.p, L.mW.p, L.vW.p, L.Wb.p, (float)lr, (float)beta1, (float)beta2, (float)eps, c1, c2,
-             stream());
-    mlp_adam(L.b.n, L.b.p, L.gb.p, L.mb.p, L.vb.p, nullptr, (float)lr, (float)beta1, (float)beta2, (float)eps, c1,
-             c2, stream());
+    mlp_adam(L.W.n, L.W.p, L.gW.p, L.mW.p, L.vW.p, L.Wb.p, h.lr, h.b1, h.b2, h.eps, h.c1, h.c2, stream());
+    mlp_adam(L.b.n, L.b.p, L.gb.p, L.mb.p, L.vb.p, nullptr, h.lr, h.b1, h.b2, h.eps, h.c1, h.c2, stream());
   }
+  if (rows_ok) copy_weights();  // (a batch beyond the row-block kernels: their transposed copies follow)
 }
 
 void Surrogate::upload_inputs(int n, const double *x, DevBuf<bf16_t> &dst) const {
@@ -309,7 +436,6 @@ double Surrogate::loss_grad_host(int n, const double *x, const double *yv, doubl
   ensure_batch(n);
   upload_inputs(n, x, xb);
   upload_targets(n, yv, t);
-  forward(n, xb.p);
   const double loss = loss_and_grad(n);
   if (grad) {
     size_t k = 0;
@@ -332,14 +458,17 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
   DevBuf<float> T;
   upload_inputs(n, x, X);
   upload_targets(n, yv, T);
-  ensure_batch(batch);
+  if (!use_rows(batch)) ensure_batch(batch);
   const int steps = n / batch;  // full batches only: every step sees the same batch size
   std::vector<int> idx(n);
   std::iota(idx.begin(), idx.end(), 0);
   std::mt19937_64 g(seed);
+  // the losses of up to 64 epochs (64 MB of partials) stay on the device before the host waits
+  const size_t per_epoch = (size_t)std::max(steps, 1) * 1024;
+  const int group = (int)std::max<size_t>(1, std::min<size_t>({64, (size_t)epochs, (size_t(16) << 20) / per_epoch}));
   DevBuf<int> didx(n);
-  DevBuf<float> eparts((size_t)std::max(steps, 1) * 1024);
-  std::vector<int> nbs(std::max(steps, 1));
+  DevBuf<float> eparts(per_epoch * (size_t)group);
+  std::vector<int> nbs((size_t)std::max(steps, 1) * group);
   std::vector<float> hp;
   std::vector<double> hist;
   double ms_total = 0.0;
@@ -347,31 +476,43 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
   hipEvent_t e0, e1;
   ED_HIP(hipEventCreate(&e0));
   ED_HIP(hipEventCreate(&e1));
-  for (int ep = 0; ep < epochs; ++ep) {
-    check_cancel();
-    for (int i = n - 1; i > 0; --i) std::swap(idx[i], idx[(size_t)(g() % (uint64_t)(i + 1))]);
-    didx.upload(idx);
+  for (int ep0 = 0; ep0 < epochs; ep0 += group) {
+    const int ne = std::min(group, epochs - ep0);
     ED_HIP(hipEventRecord(e0, stream()));
-    for (int s = 0; s < steps; ++s) {
-      const int *bi = didx.p + (size_t)s * batch;
-      mlp_gather_bf16(batch, ip, bi, X.p, xb.p, stream());
-      mlp_gather_f32(batch, op, bi, T.p, t.p, stream());
-      forward(batch, xb.p);
-      nbs[s] = backward(batch, eparts.p + (size_t)s * 1024);
-      adam_step();
+    for (int ep = 0; ep < ne; ++ep) {
+      check_cancel();
+      for (int i = n - 1; i > 0; --i) std::swap(idx[i], idx[(size_t)(g() % (uint64_t)(i + 1))]);
+      didx.upload(idx);
+      for (int s = 0; s < steps; ++s) {
+        const int *bi = didx.p + (size_t)s * batch;
+        float *lp = eparts.p + per_epoch * (size_t)ep + (size_t)s * 1024;
+        int &nb = nbs[(size_t)ep * steps + s];
+        if (use_rows(batch)) {
+          const MlpAdam h = next_adam();
+          nb = rows_step(batch, X.p, T.p, bi, lp, &h);
+          continue;
+        }
+        mlp_gather_bf16(batch, ip, bi, X.p, xb.p, stream());
+        mlp_gather_f32(batch, op, bi, T.p, t.p, stream());
+        forward(batch, xb.p);
+        nb = backward(batch, lp);
+        adam_step();
+      }
     }
     ED_HIP(hipEventRecord(e1, stream()));
     ED_HIP(hipEventSynchronize(e1));
-    // the epoch's losses, read once the epoch has run
-    hp.resize((size_t)std::max(steps, 1) * 1024);
-    if (steps) eparts.download(hp.data(), (size_t)steps * 1024);
-    double sum = 0.0;
-    for (int s = 0; s < steps; ++s) sum += mlp_fold(hp.data() + (size_t)s * 1024, nbs[s]) / batch;
+    hp.resize(per_epoch * (size_t)ne);
+    if (steps) eparts.download(hp.data(), per_epoch * (size_t)ne);
+    for (int ep = 0; ep < ne; ++ep) {
+      double sum = 0.0;
+      for (int s = 0; s < steps; ++s)
+        sum += mlp_fold(hp.data() + per_epoch * (size_t)ep + (size_t)s * 1024, nbs[(size_t)ep * steps + s]) / batch;
+      hist.push_back(steps ? sum / steps : 0.0);
+    }
     float ms = 0.f;
     ED_HIP(hipEventElapsedTime(&ms, e0, e1));
     ms_total += ms;
-    nsteps += steps;
-    hist.push_back(steps ? sum / steps : 0.0);
+    nsteps += (long)steps * ne;
   }
   ED_HIP(hipEventDestroy(e0));
   ED_HIP(hipEventDestroy(e1));
@@ -390,15 +531,20 @@ void Surrogate::time(int batch, int nrep, double *ms_fwd, double *ms_fb) {
   ED_HIP(hipEventCreate(&e0));
   ED_HIP(hipEventCreate(&e1));
   ED_HIP(hipEventCreate(&e2));
+  auto both = [&] {
+    if (use_rows(batch)) {
+      rows_step(batch, xb.p, t.p, nullptr, part.p, nullptr);
+    } else {
+      forward(batch, xb.p);
+      backward(batch, part.p);
+    }
+  };
   forward(batch, xb.p);
-  backward(batch, part.p);
+  both();
   ED_HIP(hipEventRecord(e0, stream()));
   for (int r = 0; r < nrep; ++r) forward(batch, xb.p);
   ED_HIP(hipEventRecord(e1, stream()));
-  for (int r = 0; r < nrep; ++r) {
-    forward(batch, xb.p);
-    backward(batch, part.p);
-  }
+  for (int r = 0; r < nrep; ++r) both();
   ED_HIP(hipEventRecord(e2, stream()));
   ED_HIP(hipEventSynchronize(e2));
   float a = 0.f, b = 0.f;

@@ -204,6 +204,353 @@ __global__ __launch_bounds__(256) void k_gather(int n, int ld, const int *idx, c
   }
 }
 
+// ---------------------------------------------------------------------------
+// Row-block kernels (widths 64, 128, 256).  A layer at a batch of 2 048 is 0.3
+// GFLOP, a fraction of a microsecond of matrix-core time, so separate GEMM,
+// loss, column-sum and optimizer launches were all launch and load latency (30
+// launches, 290 us a step).  Rows of the batch are independent through the
+// forward pass, the loss and the input gradients: k_mlp_rows takes 16 of them
+// through all layers and back with activations, pre-activations (fp32) and
+// gradients in LDS, and reads the weights as MFMA fragments straight from
+// L2 (16 bytes a lane, from W forward and from a transposed copy backward).  It
+// leaves activations and gradients feature-major, so that k_mlp_wgrad reads
+// both operands of dW = dZ^T A as fragments too, all layers in one launch; k_mlp_update
+// folds the batch splits and applies Adam.  A step of 12 -> 256 x 4 -> 641 at
+// 2 048 rows: 290 us -> 73 (rows 48, bound by the instructions of 128
+// workgroups' GELUs and by load latency; weight gradients 17; update 8); a
+// forward pass of 1 000 rows 26 us.
+// ---------------------------------------------------------------------------
+constexpr int kRows = 16, kRowThreads = 1024, kRowWaves = kRowThreads / 64;
+
+// KS k-steps of one weight row per lane (w: the lane's row at its 8-element
+// offset).  No lane is masked, a masked load is a branch: rows are clamped by
+// the caller, and steps past a row's end read on (the copies are allocated
+// with a layer width to spare) to meet zeros of A or no product at all.
+template <int KS>
+__device__ __forceinline__ void mlp_load(bf16x8 (&x)[KS], const bf16_t *w) {
+#pragma unroll
+  for (int i = 0; i < KS; ++i) x[i] = *(const bf16x8 *)(w + 32 * i);
+}
+// c += A(16 x 32 KS) x^T, a: the lane's LDS row at its 8-element offset
+template <int KS>
+__device__ __forceinline__ void mlp_mma(const bf16_t *a, const bf16x8 (&x)[KS], f32x4 &c) {
+#pragma unroll
+  for (int i = 0; i < KS; ++i)
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(a + 32 * i), x[i], c, 0, 0, 0);
+}
+template <int KS>
+__device__ __forceinline__ void mlp_take(bf16x8 (&x)[KS], const bf16x8 (&y)[KS]) {
+#pragma unroll
+  for (int i = 0; i < KS; ++i) x[i] = y[i];
+}
+
+// columns f < nf of a 16-row LDS matrix to feature-major memory (row pitch
+// Bp), and their sums over the rows to db (when not null)
+__device__ __forceinline__ void mlp_store_t(const bf16_t *buf, int pitch, int nf, bf16_t *dst, long Bp, int b0,
+                                            float *db) {
+  for (int t = threadIdx.x; t < 2 * nf; t += kRowThreads) {
+    const int f = t >> 1, h = t & 1;
+    bf16x8 v;
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = buf[(8 * h + i) * pitch + f];
+      s += (float)v[i];
+    }
+    *(bf16x8 *)(dst + (long)f * Bp + b0 + 8 * h) = v;
+    if (db) {
+      s += __shfl_xor(s, 1, 64);
+      if (h == 0) db[f] = s;
+    }
+  }
+}
+
+template <int KS, bool TRAIN>
+__global__ __launch_bounds__(kRowThreads) void k_mlp_rows(MlpRows P) {
+  constexpr int WD = 32 * KS, PA = WD + 8, ZP = WD + 4, NT = WD / 16;
+  extern __shared__ __attribute__((aligned(16))) char sm[];
+  __shared__ float red[kRowWaves];
+  bf16_t *a0 = (bf16_t *)sm, *a1 = a0 + kRows * PA;
+  float *gg = (float *)(a1 + kRows * PA);                    // gelu'(Z): depth x 16 x ZP (TRAIN)
+  const int PO = P.out32 + 8, nbias = P.depth * WD + P.n_out;
+  // biases, and (TRAIN) loss weights and the output gradients, 16 x PO
+  float *sb = TRAIN ? gg + (long)P.depth * kRows * ZP : gg, *slw = sb + nbias;
+  bf16_t *dy = (bf16_t *)(slw + (P.n_out + nbias + 7) / 8 * 8 - nbias);
+  const int b0 = blockIdx.x * kRows;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, lc = l & 15, lk = 8 * (l >> 4);
+  // wave w owns 16 columns of a hidden layer (waves beyond NT idle there);
+  // the weights of the next product are loaded before the current one is used
+  const bool own = w < NT;
+  const int n = 16 * w + lc, nh = 16 * (w % NT) + lc;
+  bf16x8 x[KS], nx[KS] = {};
+  mlp_load(x, P.W[0] + (long)nh * P.in_pad + lk);
+  // the sample of each of this lane's four output rows (the last row repeated
+  // past the batch; its results are dropped), and everything else a wave will
+  // want from memory one value at a time: each would be a full latency later
+  long sample[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int b = min(b0 + 4 * (l >> 4) + r, P.B - 1);
+    sample[r] = P.idx ? P.idx[b] : b;
+  }
+  float tv[4] = {};
+  if (TRAIN)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tv[r] = P.T[sample[r] * P.out_pad + min(n, P.n_out - 1)];
+  for (int y = 0; y <= P.depth; ++y)
+    for (int e = threadIdx.x; e < (y < P.depth ? WD : P.n_out); e += kRowThreads) sb[y * WD + e] = P.bias[y][e];
+  if (TRAIN)
+    for (int e = threadIdx.x; e < P.n_out; e += kRowThreads) slw[e] = P.lw[e];
+  for (int e = threadIdx.x; e < kRows * PA; e += kRowThreads) {
+    const int r = e / PA, c = e - r * PA, b = b0 + r;
+    bf16_t v = (bf16_t)0.f;
+    if (b < P.B && c < P.in_pad) v = P.X[(long)(P.idx ? P.idx[b] : b) * P.in_pad + c];
+    a0[e] = v;
+  }
+  if (TRAIN)
+    for (int e = threadIdx.x; e < kRows * PO; e += kRowThreads) dy[e] = (bf16_t)0.f;
+  __syncthreads();
+  if (TRAIN) mlp_store_t(a0, PA, P.n_in, P.actT, P.Bp, b0, nullptr);
+  for (int y = 0; y < P.depth; ++y) {
+    const bf16_t *src = y & 1 ? a1 : a0;
+    bf16_t *dst = y & 1 ? a0 : a1;
+    const bool hid = y + 1 < P.depth;  // else the first output tile of the wave follows
+    mlp_load(nx, P.W[y + 1] + (long)(hid ? nh : min(n, P.n_out - 1)) * WD + lk);
+    if (own) {
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+      mlp_mma(src + lc * PA + lk, x, c);
+      const float bias = sb[y * WD + n];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (l >> 4) + r;
+        const float z = c[r] + bias, h = 0.5f * (1.f + erff(z * 0.70710678118654752f));
+        dst[row * PA + n] = (bf16_t)(z * h);
+        if (TRAIN) gg[((long)y * kRows + row) * ZP + n] = h + z * 0.39894228040143268f * expf(-0.5f * z * z);
+      }
+    }
+    mlp_take(x, nx);
+    __syncthreads();
+    if (TRAIN) mlp_store_t(dst, PA, WD, P.actT + (long)(P.n_in + y * WD) * P.Bp, P.Bp, b0, nullptr);
+  }
+  // output layer: tiles w, w + kRowWaves, ...
+  float loss = 0.f;
+  {
+    const bf16_t *a = (P.depth & 1 ? a1 : a0) + lc * PA + lk;
+    for (int m = n; m - lc < P.n_out; m += 16 * kRowWaves) {
+      const int m2 = m + 16 * kRowWaves, mc = min(m, P.n_out - 1);
+      mlp_load(nx, P.W[P.depth] + (long)min(m2, P.n_out - 1) * WD + lk);
+      float tn[4] = {};
+      if (TRAIN)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tn[r] = P.T[sample[r] * P.out_pad + min(m2, P.n_out - 1)];
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+      mlp_mma(a, x, c);
+      mlp_take(x, nx);
+      const float bias = sb[P.depth * WD + mc], wo = TRAIN ? slw[mc] : 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (l >> 4) + r, b = b0 + row;
+        const bool in = b < P.B && m < P.n_out;
+        const float yv = c[r] + bias;
+        if (!TRAIN) {
+          if (in) P.y[(long)b * P.out_pad + m] = yv;
+        } else {
+          const float rr = in ? yv - tv[r] : 0.f;
+          loss += wo * rr * rr;
+          if (m < P.n_out) dy[row * PO + m] = (bf16_t)(P.scale * wo * rr);
+          tv[r] = tn[r];
+        }
+      }
+    }
+  }
+  if (!TRAIN) return;
+  const int ko = P.out32;  // row pitch of the transposed output weights
+  mlp_load(x, P.Wt[P.depth] + (long)nh * ko + lk);
+  loss = wave_sum_f(loss);
+  if (l == 0) red[w] = loss;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float sum = 0.f;
+    for (int i = 0; i < kRowWaves; ++i) sum += red[i];
+    P.loss[b0 / kRows] = sum;
+  }
+  float *db = P.db + (long)(b0 / kRows) * (P.depth * WD + P.n_out);
+  mlp_store_t(dy, PO, P.n_out, P.dzT + (long)P.depth * WD * P.Bp, P.Bp, b0, db + P.depth * WD);
+  // dZ_{y-1} = (dZ_y W_y) gelu'(Z_{y-1}); the activation buffers are free again
+  const bf16_t *src = dy;
+  int spitch = PO;
+  for (int y = P.depth; y >= 1; --y) {
+    bf16_t *dst = (P.depth - y) & 1 ? a1 : a0;
+    const bf16_t *a = src + lc * spitch + lk;
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+    if (y == P.depth) {
+      // the output layer's k range in groups of KS steps (steps past its end
+      // meet zero weights; their LDS reads stay inside the row)
+      for (int k = WD; k < ko; k += WD) {
+        mlp_load(nx, P.Wt[y] + (long)nh * ko + lk + k);
+        mlp_mma(a + k - WD, x, c);
+        mlp_take(x, nx);
+      }
+      const int kl = (ko - 1) / WD * WD;
+      if (y > 1) mlp_load(nx, P.Wt[y - 1] + (long)nh * WD + lk);
+#pragma unroll
+      for (int i = 0; i < KS; ++i)
+        if (kl + 32 * i < ko)
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(a + kl + 32 * i), x[i], c, 0, 0, 0);
+    } else {
+      if (y > 1) mlp_load(nx, P.Wt[y - 1] + (long)nh * WD + lk);
+      mlp_mma(a, x, c);
+    }
+    mlp_take(x, nx);
+    if (own) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (l >> 4) + r;
+        dst[row * PA + n] = (bf16_t)(c[r] * gg[((long)(y - 1) * kRows + row) * ZP + n]);
+      }
+    }
+    __syncthreads();
+    mlp_store_t(dst, PA, WD, P.dzT + (long)(y - 1) * WD * P.Bp, P.Bp, b0, db + (y - 1) * WD);
+    src = dst;
+    spitch = PA;
+  }
+}
+
+// dW of every layer, one 32 x 64 tile and one split of the batch per wave;
+// both operands are read feature-major (K, the batch, contiguous)
+__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpShape S, int ntile, int nsplit, int nk, long Bp,
+                                                   const bf16_t *__restrict__ actT, const bf16_t *__restrict__ dzT,
+                                                   float *__restrict__ part) {
+  const int l = threadIdx.x & 63, lc = l & 15, lk = 8 * (l >> 4);
+  const int tile = (int)(blockIdx.x / nsplit) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sp = (int)(blockIdx.x % nsplit);
+  if (tile >= ntile) return;
+  int y = 0;
+  while (tile >= S.t0[y + 1]) ++y;
+  const int in = S.in[y], out = S.out[y], ntn = (in + 63) / 64, q = tile - S.t0[y];
+  const int m0 = 32 * (q / ntn), n0 = 64 * (q % ntn);
+  const int per = (nk + nsplit - 1) / nsplit, k0 = sp * per, k1 = min(nk, k0 + per);
+  const bf16_t *A[2], *Bv[4];
+  bool ma[2], nb[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int m = m0 + 16 * i + lc;
+    ma[i] = m < out;
+    A[i] = dzT + (S.zoff[y] + (ma[i] ? m : 0)) * Bp + lk;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int n = n0 + 16 * j + lc;
+    nb[j] = n < in;
+    Bv[j] = actT + (S.aoff[y] + (nb[j] ? n : 0)) * Bp + lk;
+  }
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // four k-steps' fragments are loaded together, 24 loads in flight a wave: a
+  // round takes ~3 us (sixteen rows a load, written by other XCDs)
+  constexpr int KB = 4;
+  for (int k = k0; k < k1; k += KB) {
+    bf16x8 a[KB][2], b[KB][4];
+#pragma unroll
+    for (int q = 0; q < KB; ++q) {
+      const long at = 32L * min(k + q, k1 - 1);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[q][i] = *(const bf16x8 *)(A[i] + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[q][j] = *(const bf16x8 *)(Bv[j] + at);
+    }
+#pragma unroll
+    for (int q = 0; q < KB; ++q)
+      if (k + q < k1)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][i], b[q][j], acc[i][j], 0, 0, 0);
+  }
+  // (rows and columns past the layer read row 0 and are not stored)
+  float *C = part + (long)sp * S.nw + S.poff[y];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + 16 * j + lc;
+      if (n >= in) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + 16 * i + 4 * (l >> 4) + r;
+        if (m < out) C[(long)m * in + n] = acc[i][j][r];
+      }
+    }
+}
+
+__device__ __forceinline__ float adam_one(float p, float g, float &m, float &v, const MlpAdam &h) {
+  m = h.b1 * m + (1.f - h.b1) * g;
+  v = h.b2 * v + (1.f - h.b2) * g * g;
+  return p - h.lr * (m / h.c1) / (sqrtf(v / h.c2) + h.eps);
+}
+
+// gradients folded over the batch splits (weights) and row blocks (biases, one
+// wave each), both in a fixed order, then one Adam step on the fp32 masters
+// and the two bf16 copies (ADAM), or the gradients stored
+// (grid y: the layer, uniform, so that the tables are scalar loads)
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_mlp_update(MlpShape S, MlpParams Q, MlpAdam h, int nsplit, int nrow,
+                                                    const float *part, const float *db) {
+  const int y = blockIdx.y, in = S.in[y], out = S.out[y], wblk = (out * in + 255) / 256;
+  if ((int)blockIdx.x < wblk) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= out * in) return;
+    const int o = e / in, i = e - o * in;
+    float g = 0.f;
+    for (int z = 0; z < nsplit; ++z) g += part[(long)z * S.nw + S.poff[y] + e];
+    const long at = (long)o * Q.in_pad[y] + i;
+    if (!ADAM) {
+      Q.gW[y][at] = g;
+      return;
+    }
+    float m = Q.mW[y][at], v = Q.vW[y][at];
+    const float x = adam_one(Q.W[y][at], g, m, v, h);
+    Q.mW[y][at] = m;
+    Q.vW[y][at] = v;
+    Q.W[y][at] = x;
+    Q.Wb[y][at] = (bf16_t)x;
+    Q.Wt[y][(long)i * Q.out32[y] + o] = (bf16_t)x;
+    return;
+  }
+  const int o = ((int)blockIdx.x - wblk) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (o >= out) return;
+  const long nbias = S.zoff[S.nl];
+  float g = 0.f;
+  for (int r = l; r < nrow; r += 64) g += db[r * nbias + S.zoff[y] + o];
+  g = wave_sum_f(g);
+  if (l) return;
+  if (!ADAM) {
+    Q.gb[y][o] = g;
+    return;
+  }
+  float m = Q.mb[y][o], v = Q.vb[y][o];
+  Q.b[y][o] = adam_one(Q.b[y][o], g, m, v, h);
+  Q.mb[y][o] = m;
+  Q.vb[y][o] = v;
+}
+
+// the bf16 copies of one layer's weights: row-major, and transposed with a
+// pitch of 32-element groups (padding zero from the allocation)
+__global__ __launch_bounds__(256) void k_mlp_copies(int out, int in, int in_pad, int out32, const float *W, bf16_t *Wb,
+                                                    bf16_t *Wt) {
+  const size_t n = (size_t)out * in;
+  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
+    const int o = (int)(e / in), i = (int)(e - (size_t)o * in);
+    const bf16_t v = (bf16_t)W[(size_t)o * in_pad + i];
+    Wb[(size_t)o * in_pad + i] = v;
+    Wt[(size_t)i * out32 + o] = v;
+  }
+}
+
 int grid1(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 4096)); }
 
 }  // namespace
@@ -285,6 +632,64 @@ void mlp_gather_bf16(int n, int ld, const int *idx, const bf16_t *src, bf16_t *d
 void mlp_gather_f32(int n, int ld, const int *idx, const float *src, float *dst, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_gather<float>, dim3(grid1((size_t)n * ld)), dim3(256), 0, s, n, ld, idx, src, dst);
+  ED_HIP(hipGetLastError());
+}
+
+size_t mlp_rows_lds(int width, int depth, int n_out, bool train) {
+  const size_t act = 2 * (size_t)kRows * (width + 8) * sizeof(bf16_t), nbias = (size_t)depth * width + n_out;
+  const int out32 = (n_out + 31) / 32 * 32;
+  if (!train) return act + (nbias + 8) * sizeof(float);
+  return act + (size_t)depth * kRows * (width + 4) * sizeof(float) + (n_out + nbias + 7) / 8 * 8 * sizeof(float) +
+         (size_t)kRows * (out32 + 8) * sizeof(bf16_t);
+}
+
+int mlp_rows(const MlpRows &P, int width, bool train, hipStream_t s) {
+  if (P.B <= 0) return 0;
+  const size_t lds = mlp_rows_lds(width, P.depth, P.n_out, train);
+  if (lds > kMlpRowsLds || P.depth > kMlpLayers - 1 || P.in_pad > width || P.Bp % 32 || P.Bp < P.B ||
+      (P.in_pad % 8) || (reinterpret_cast<uintptr_t>(P.actT) & 15) || (reinterpret_cast<uintptr_t>(P.dzT) & 15))
+    fail(ED_ERR_INTERNAL, "mlp_rows: network outside the row-block kernel's range");
+  // a training step's blocks cover the padded batch: the padding of the
+  // feature-major matrices is written too (gradients zero)
+  const int nb = train ? (P.B + 31) / 32 * 2 : (P.B + kRows - 1) / kRows;
+#define ED_ROWS(KS)                                                                                          \
+  do {                                                                                                       \
+    auto kern = train ? k_mlp_rows<KS, true> : k_mlp_rows<KS, false>;                                        \
+    if (lds > 64 * 1024)                                                                                     \
+      ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),                                       \
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                     \
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(kRowThreads), lds, s, P);                                        \
+  } while (0)
+  if (width == 64) ED_ROWS(2);
+  else if (width == 128) ED_ROWS(4);
+  else if (width == 256) ED_ROWS(8);
+  else fail(ED_ERR_INTERNAL, "mlp_rows: width");
+#undef ED_ROWS
+  ED_HIP(hipGetLastError());
+  return nb;
+}
+
+void mlp_wgrad(const MlpShape &S, int nsplit, int nk, long Bp, const bf16_t *actT, const bf16_t *dzT, float *part,
+               hipStream_t s) {
+  const int nt = S.t0[S.nl];
+  hipLaunchKernelGGL(k_mlp_wgrad, dim3((nt + 3) / 4 * nsplit), dim3(256), 0, s, S, nt, nsplit, nk, Bp, actT, dzT, part);
+  ED_HIP(hipGetLastError());
+}
+
+void mlp_update(const MlpShape &S, const MlpParams &Q, const MlpAdam *h, int nsplit, int nrow, const float *part,
+                const float *db, hipStream_t s) {
+  int nx = 1;
+  for (int y = 0; y < S.nl; ++y) nx = std::max(nx, (S.out[y] * S.in[y] + 255) / 256 + (S.out[y] + 3) / 4);
+  const dim3 grid((unsigned)nx, (unsigned)S.nl);
+  if (h)
+    hipLaunchKernelGGL((k_mlp_update<true>), grid, dim3(256), 0, s, S, Q, *h, nsplit, nrow, part, db);
+  else
+    hipLaunchKernelGGL((k_mlp_update<false>), grid, dim3(256), 0, s, S, Q, MlpAdam(), nsplit, nrow, part, db);
+  ED_HIP(hipGetLastError());
+}
+
+void mlp_copies(int out, int in, int in_pad, int out32, const float *W, bf16_t *Wb, bf16_t *Wt, hipStream_t s) {
+  hipLaunchKernelGGL(k_mlp_copies, dim3(grid1((size_t)out * in)), dim3(256), 0, s, out, in, in_pad, out32, W, Wb, Wt);
   ED_HIP(hipGetLastError());
 }
 

@@ -63,15 +63,59 @@ void mlp_adam(size_t n, float *p, const float *g, float *m, float *v, bf16_t *pb
 // dst rows r < n: dst[r * ld + c] = src[idx[r] * ld + c]
 void mlp_gather_bf16(int n, int ld, const int *idx, const bf16_t *src, bf16_t *dst, hipStream_t s);
 void mlp_gather_f32(int n, int ld, const int *idx, const float *src, float *dst, hipStream_t s);
+// ---- row-block kernels (widths 64, 128, 256), see ed_surrogate.hip ----
+constexpr int kMlpLayers = 9;              // at most 8 hidden layers
+constexpr size_t kMlpRowsLds = 150 * 1024;
+constexpr size_t kMlpSpare = 512;          // elements past a weight copy's last row
+// One pass of B rows (rows idx[b] of X and T, or b when idx is null) through
+// the network.  Forward only: y (pitch out_pad).  Training: the activations
+// (inputs first) and output gradients feature-major (row pitch Bp, a multiple
+// of 32) in actT and dzT, the bias gradients' and the loss's partials per
+// block of 16 rows in db and loss.
+struct MlpRows {
+  int depth = 0, n_in = 0, n_out = 0, in_pad = 0, out_pad = 0, out32 = 0, B = 0;
+  long Bp = 0;
+  const bf16_t *W[kMlpLayers] = {}, *Wt[kMlpLayers] = {};
+  const float *bias[kMlpLayers] = {};
+  const bf16_t *X = nullptr;
+  const float *T = nullptr, *lw = nullptr;
+  const int *idx = nullptr;
+  float scale = 0.f;
+  bf16_t *actT = nullptr, *dzT = nullptr;
+  float *db = nullptr, *loss = nullptr, *y = nullptr;
+};
+// layer sizes; first row of each layer's input / gradient in actT / dzT, first
+// weight (rows of `in`, unpadded) and first 32 x 64 tile
+struct MlpShape {
+  int nl = 0;
+  int in[kMlpLayers] = {}, out[kMlpLayers] = {}, t0[kMlpLayers + 1] = {};
+  long aoff[kMlpLayers] = {}, zoff[kMlpLayers + 1] = {}, poff[kMlpLayers + 1] = {}, nw = 0;
+};
+struct MlpParams {
+  float *W[kMlpLayers], *b[kMlpLayers], *mW[kMlpLayers], *vW[kMlpLayers], *mb[kMlpLayers], *vb[kMlpLayers];
+  float *gW[kMlpLayers], *gb[kMlpLayers];
+  bf16_t *Wb[kMlpLayers], *Wt[kMlpLayers];
+  int in_pad[kMlpLayers], out32[kMlpLayers];
+};
+struct MlpAdam { float lr = 0.f, b1 = 0.f, b2 = 0.f, eps = 0.f, c1 = 1.f, c2 = 1.f; };
+size_t mlp_rows_lds(int width, int depth, int n_out, bool train);
+int mlp_rows(const MlpRows &P, int width, bool train, hipStream_t s);  // returns the blocks (partials)
+void mlp_wgrad(const MlpShape &S, int nsplit, int nk, long Bp, const bf16_t *actT, const bf16_t *dzT, float *part,
+               hipStream_t s);
+// h == nullptr: gradients to gW / gb; else one Adam step
+void mlp_update(const MlpShape &S, const MlpParams &Q, const MlpAdam *h, int nsplit, int nrow, const float *part,
+                const float *db, hipStream_t s);
+void mlp_copies(int out, int in, int in_pad, int out32, const float *W, bf16_t *Wb, bf16_t *Wt, hipStream_t s);
+
 // fold of float partials into one double (host): deterministic order
 double mlp_fold(const float *partials, int n);
 
 // ---- host model (ed_surrogate.cpp) ----
 struct Surrogate {
   struct Layer {
-    int in = 0, out = 0, in_pad = 0, out_pad = 0;
+    int in = 0, out = 0, in_pad = 0, out_pad = 0, out32 = 0;
     DevBuf<float> W, b, gW, gb, mW, vW, mb, vb;
-    DevBuf<bf16_t> Wb;
+    DevBuf<bf16_t> Wb, Wt;  // Wt: transposed copy, pitch out32 (row-block kernels)
   };
   int n_in = 0, n_out = 0, width = 0, depth = 0;
   std::vector<Layer> layers;
@@ -84,12 +128,28 @@ struct Surrogate {
   DevBuf<bf16_t> xb, act_b, dz_b, dz2_b;  // activations (depth x B x width), output gradients
   DevBuf<float> z, y, t, part, split;
   int split_S = 0;
+  // row-block kernels: whether the network is in their range, and their buffers
+  bool rows_ok = false;
+  int cap_rows = 0;
+  DevBuf<bf16_t> actT, dzT;
+  DevBuf<float> slab, db;
 
   Surrogate(int n_in, int n_out, int width, int depth, uint64_t seed);
   size_t n_params() const;
   void set_scaling(const double *xm, const double *xs, const double *ym, const double *ys, const double *w);
   void get_weights(double *w) const;
   void set_weights(const double *w);
+  void copy_weights();  // bf16 copies from the fp32 masters
+  // one launch from row idx[b] (b when null) of X and T, b < B, to gradients in
+  // dzT / actT / db and loss partials (returns their number)
+  bool use_rows(int B) const { return rows_ok && (B + 31) / 32 * 2 <= 1024; }
+  MlpRows rows_args(int B, const bf16_t *X, const float *T, const int *idx);
+  MlpShape shape() const;
+  MlpParams param_table();
+  int rows_splits(int B) const;
+  void ensure_rows(int B);
+  int rows_step(int B, const bf16_t *X, const float *T, const int *idx, float *loss, const MlpAdam *h);
+  MlpAdam next_adam();
   // device forward on normalized bf16 inputs (B rows, in_pad columns) -> y (fp32, normalized)
   void forward(int B, const bf16_t *x);
   // gradients (into gW / gb) of B rows already in xb / t after forward(B, xb):

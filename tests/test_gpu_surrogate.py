@@ -113,3 +113,30 @@ def test_bad_arguments_are_errors():
         net.set_scaling(x_std=np.array([1.0, 0.0, 1.0]))
     with pytest.raises(ValueError):
         net.set_weights(np.zeros(3))
+
+
+@pytest.mark.parametrize("n_in,n_out,width,depth,B", [(1, 1, 64, 1, 1), (3, 16, 64, 1, 15), (33, 17, 128, 2, 16),
+                                                      (64, 7, 64, 3, 17), (9, 300, 256, 2, 1037), (250, 33, 256, 1, 64),
+                                                      (12, 641, 256, 4, 31), (5, 40, 32, 2, 50), (7, 20, 256, 9, 20)])
+def test_row_block_kernels_at_their_edges(n_in, n_out, width, depth, B):
+    """Batches around a row block (16) and a k-step (32), several batch splits,
+    one to many output tiles, inputs as wide as a layer, one hidden layer, and
+    two networks outside the row-block kernels' range (width 32, nine hidden
+    layers): predictions, loss and gradients against the oracle with the same
+    bf16 roundings (as the tests above: 1e-3 of the scale, 1e-4, and 5e-3 per
+    layer; a bf16 rounding that falls the other way after a 1e-7 difference
+    moves a single gradient entry by 0.4 %, and few rows average less: 2e-2
+    below 64 rows)."""
+    net, P = _net(n_in, n_out, width, depth, seed=B)
+    rng = np.random.default_rng(B)
+    x = rng.normal(size=(B, n_in))
+    t = rng.normal(size=(B, n_out))
+    y = net.predict(x)
+    y_mim, _ = M.forward(P, x, mimic=True)
+    assert np.max(np.abs(y - y_mim)) <= 2e-3 * np.max(np.abs(y_mim))
+    loss, g = net.loss_grad(x, t)
+    loss_m, G_m = M.loss_grad(P, x, M.f32(t), np.ones(n_out), mimic=True)
+    assert abs(loss - loss_m) <= 1e-4 * loss_m
+    for (dW, db), (mW, mb) in zip(M.unflatten(g, n_in, n_out, width, depth), G_m):
+        for a, m in ((dW, mW), (db, mb)):
+            assert np.linalg.norm(a - m) <= (5e-3 if B >= 64 else 2e-2) * np.linalg.norm(m) + 1e-12
