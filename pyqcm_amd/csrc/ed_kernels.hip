@@ -22,9 +22,8 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Block-wide sum; result valid in thread 0.  sh must hold BS/64 doubles.
-template <int BS>
-__device__ __forceinline__ double block_sum(double v, double *sh) {
+// Block-wide sum over nw waves; result valid in thread 0.  sh must hold nw doubles.
+__device__ __forceinline__ double block_sum(double v, double *sh, int nw) {
   v = wave_sum(v);
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   __syncthreads();
@@ -32,10 +31,14 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
   __syncthreads();
   double r = 0.0;
   if (threadIdx.x < kWave) {
-    r = (threadIdx.x < BS / kWave) ? sh[threadIdx.x] : 0.0;
+    r = ((int)threadIdx.x < nw) ? sh[threadIdx.x] : 0.0;
     r = wave_sum(r);
   }
   return r;
+}
+template <int BS>
+__device__ __forceinline__ double block_sum(double v, double *sh) {
+  return block_sum(v, sh, BS / kWave);
 }
 
 __device__ __forceinline__ double half_entry(const DevHalf &h, const double *vtab, uint32_t e, uint32_t &col) {
@@ -406,6 +409,131 @@ __global__ __launch_bounds__(BS) void k_hv_rows_sell(FusedParams P) {
   }
   if (DOWN && P.part) {
     const double s = block_sum<BS>(dot, red);
+    if (threadIdx.x == 0) P.part[blockIdx.x] = s;
+  }
+}
+
+// Row kernel for short rows: RPT rows per workgroup, one column of all of them
+// per thread, so that a column's table entries, diagonal parts and the entry
+// values are read once for RPT rows, and the RPT rows' reads of a neighbour
+// are in flight together.  Bound by the latency and the L1 rate of those reads,
+// not by memory (the vector stays in the XCD's L2).  With one row per workgroup
+// of four waves, every row re-read the whole up table, 190 MB of vector memory
+// traffic for a 6.8 MB vector of 924 x 924 states, and each wave walked its
+// slices one latency after the other; rows below 512 states, several to a
+// workgroup, went state by state through the compressed rows.  The neighbour
+// lists are staged in LDS, padded to emax entries (own row, value 0).  The rows
+// of an XCD are one run of the breadth-first order, whose hops stay close: 924 x
+// 924 17.4 us with the rows dealt out to the XCDs in turn, 16.5 so.  Sizes and
+// times: short_row_count.
+template <int RPT, int TM>
+__global__ __launch_bounds__(1024) void k_hv_rows_multi(FusedParams P, uint32_t emax) {
+  extern __shared__ double smem[];
+  const uint32_t BS = blockDim.x;
+  __shared__ double Ush[32];
+  __shared__ double vtu[kVtabMax];
+  __shared__ double red[1024 / kWave];
+  const FactArgs &a = P.a;
+  const uint32_t du = a.up.dim, dd = a.dn.dim, pitch = du + 1;
+  double *xs = smem, *nval = smem + RPT * pitch;
+  uint32_t *ncol = reinterpret_cast<uint32_t *>(nval + RPT * emax);
+  if (threadIdx.x < 32) Ush[threadIdx.x] = a.Uc[threadIdx.x];
+  if (TM == 0)
+    for (uint32_t i = threadIdx.x; i < (uint32_t)P.ntab_up; i += BS) vtu[i] = a.up.val[i];
+  const double *vtab_u = P.ntab_up ? vtu : a.up.val;
+  const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  // XCD x (blocks b % 8) takes the x-th run of rows
+  const uint32_t blk = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  uint32_t d[RPT];
+#pragma unroll
+  for (int j = 0; j < RPT; ++j) {
+    const uint32_t i = min(blk * RPT + j, dd - 1);  // past the last row: repeated, not stored
+    d[j] = a.row_order ? a.dn.order[i] : i;
+  }
+#pragma unroll
+  for (int j = 0; j < RPT; ++j) {
+    const double *xr = P.x + (size_t)d[j] * du;
+    for (uint32_t f = threadIdx.x; f < pitch; f += BS) xs[j * pitch + f] = f < du ? xr[f] : 0.0;
+    const uint32_t g0 = a.dn.ptr[d[j]], nnb = a.dn.ptr[d[j] + 1] - g0;
+    for (uint32_t q = threadIdx.x; q < emax; q += BS) {
+      uint32_t c = d[j];
+      const double v = q < nnb ? half_entry(a.dn, a.dn.val, g0 + q, c) : 0.0;
+      ncol[q * RPT + j] = c;
+      nval[q * RPT + j] = v;
+    }
+  }
+  __syncthreads();
+  const SellTable &T = a.up.sell[0];
+  double dot = 0.0;
+  for (uint32_t s = blk * RPT < dd ? wave : T.nslice; s < T.nslice; s += BS / kWave) {
+    const uint32_t u = s * kWave + lane, uu = min(u, du - 1);
+    double acc[RPT];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j)
+      acc[j] = diag_value(a, Ush, (size_t)d[j] * du + uu, uu, d[j], a.diag_mode ? a.dn.states[d[j]] : 0u) *
+               xs[j * pitch + uu];
+    const size_t o0 = T.off[s], o1 = T.off[s + 1];
+    if (TM == 1) {
+      for (size_t e = o0 + lane; e < o1; e += kWave) {
+        const double v = T.val[e];
+        const uint32_t c = T.ent[e];
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) acc[j] += v * xs[j * pitch + c];
+      }
+    } else {
+      double up[RPT];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) up[j] = 0.0;
+      const uint32_t nq = (uint32_t)((o1 - o0) / (kWave * 4)), mask = (1u << a.up.colbits) - 1u;
+#pragma unroll 2
+      for (uint32_t q = 0; q < nq; ++q) {
+        uint32_t c[4];
+        double v[4];
+        if (TM == 2) {
+          const uint2 g = reinterpret_cast<const uint2 *>(T.e16 + o0)[(size_t)q * kWave + lane];
+          const uint32_t e[4] = {g.x & 0xffffu, g.x >> 16, g.y & 0xffffu, g.y >> 16};
+#pragma unroll
+          for (int h = 0; h < 4; ++h) {
+            c[h] = e[h] & 0x7fffu;
+            v[h] = e[h] & 0x8000u ? -1.0 : 1.0;
+          }
+        } else {
+          const uint4 g = reinterpret_cast<const uint4 *>(T.ent + o0)[(size_t)q * kWave + lane];
+          const uint32_t e[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+          for (int h = 0; h < 4; ++h) {
+            c[h] = e[h] & mask;
+            v[h] = vtab_u[e[h] >> a.up.colbits];
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+#pragma unroll
+          for (int j = 0; j < RPT; ++j) up[j] += v[h] * xs[j * pitch + c[h]];
+      }
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) acc[j] += TM == 2 ? a.up.t0 * up[j] : up[j];
+    }
+#pragma unroll 4
+    for (uint32_t q = 0; q < emax; ++q) {
+      double xv[RPT];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) xv[j] = P.x[(size_t)ncol[q * RPT + j] * du + uu];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) acc[j] += nval[q * RPT + j] * xv[j];
+    }
+    if (u < du)
+#pragma unroll
+      for (int j = 0; j < RPT; ++j)
+        if (blk * RPT + j < dd) {
+          const size_t I = (size_t)d[j] * du + u;
+          const double out = (P.beta != 0.0) ? P.ax * acc[j] + P.beta * P.y[I] : P.ax * acc[j];
+          P.y[I] = out;
+          dot += out * xs[j * pitch + u];
+        }
+  }
+  if (P.part) {
+    const double s = block_sum(dot, red, (int)BS / kWave);
     if (threadIdx.x == 0) P.part[blockIdx.x] = s;
   }
 }
@@ -1346,6 +1474,47 @@ static int fused_grid(const FactArgs &a, uint32_t R) {
   return (int)std::min<uint32_t>(nb, (uint32_t)kPartialsCap);
 }
 
+// Dynamic LDS of the short-row kernel (the CU's 160 KB less its static tables)
+constexpr size_t kShortRowLds = 140 * 1024;
+constexpr uint32_t kShortRow = 4096;
+static size_t short_row_lds(const FactArgs &a, int rpt) {
+  return rpt * (((size_t)a.up.dim + 1 + a.dn.maxrow) * sizeof(double) + a.dn.maxrow * sizeof(uint32_t));
+}
+
+// Rows per workgroup of the short-row kernel; 0: the general row kernels.
+// The rows that the fullest CU works on, each at the cost of a row among 1, 2
+// or 4: where the up table is heavy (20 bytes or more per state) the shared
+// read of it makes the rows of a larger group cheaper, with a light one it
+// does not.  us of one product against the general kernels:
+//   heavy  924 x 924 (4 rows) 20.8 -> 16.5, 1716^2 (4) 60 -> 48,
+//          1287^2 (2) 34.7 -> 33.6, 3432^2 (4) 230 -> 185, 364 rows of 3432 (2) 32 -> 27
+//   light  70 x 70 (1) 9.5 -> 4.7, 252 x 252 (1) 15.4 -> 5, 1001^2 (1) 17.2 -> 12.5,
+//          1287^2 (1) 24.7 -> 23.9, 3003^2 (1) 121 -> 101
+// With light tables 2 or 4 rows lose (1287^2: 27 and 30 us), with heavy ones 1
+// row does (924^2: 20 us).  From kShortRow states on a row is long enough to
+// keep a workgroup of 16 waves busy by itself, and the rows in flight no longer
+// fit the XCD's L2: 6435 x 5005 0.65 ms general, 0.77 here; 12870^2 3.8 and 5.6.
+// Rows of more than 64 neighbours, and blocks asked for by size, stay general.
+static int short_row_count(const FactArgs &a) {
+  if (a.block != 0 || a.up.dim >= kShortRow || a.up.sell[0].nslice == 0 || a.dn.maxrow > 64)
+    return 0;
+  const size_t entry = a.up.mode16 ? 2 : (a.up.packed ? 4 : 12);
+  const bool heavy = a.up.nnz * entry >= 20 * (size_t)a.up.dim;
+  const double cost[3] = {1.0, heavy ? 0.93 : 1.0, heavy ? 0.8 : 1.0};
+  int best = 0;
+  double least = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const uint32_t rpt = 1u << k, nb = (a.dn.dim + rpt - 1) / rpt;
+    if (nb > (uint32_t)kPartialsCap - 8 || short_row_lds(a, rpt) > kShortRowLds) continue;
+    const double t = cost[k] * (double)rpt * ((nb + 255) / 256);
+    if (!best || t < least) {
+      best = (int)rpt;
+      least = t;
+    }
+  }
+  return best;
+}
+
 int hv_factorized_max_partials(const FactArgs &a, int variant) { return kPartialsCap; }
 
 int hv_factorized_cfg(const FactArgs &a, const double *x, double *y, double ax, double beta, double *part, int variant,
@@ -1384,8 +1553,40 @@ int hv_factorized_cfg(const FactArgs &a, const double *x, double *y, double ax, 
     hipLaunchKernelGGL(kern, dim3(g), dim3(BS), lds, s, P);                     \
   } while (0)
     const uint32_t kneed = (du + BS - 1) / BS;
+    const int tm = a.up.mode16 ? 2 : (a.up.packed ? 0 : 1);
+    const int rpt = short_row_count(a);
+    if (down_here && rpt > 0) {
+      const int gm = 8 * (int)(((dd + rpt - 1) / rpt + 7) / 8);
+      const size_t lm = short_row_lds(a, rpt);
+      // About 16 waves in flight per CU (fewer hide no latency, more crowd the
+      // CU's L1), as many on each SIMD.  1716 x 1716 states, 4 rows, 2
+      // workgroups per CU: 8 waves each 49 us, 4 60, 16 53; 924 x 924, 4 rows,
+      // 1 per CU: 16 waves 16 us, 8 18, 4 25; 1287 x 1287, 2 rows, 3 per CU:
+      // 4 waves 33 us, 6 43, 8 34.
+      const size_t resident = std::min<size_t>((gm + 255) / 256, kShortRowLds / lm);
+      const int waves = resident == 1 ? 16 : (resident == 2 ? 8 : 4);
+      const int bs = kWave * std::min<int>(waves, (du + kWave - 1) / kWave);
+#define ED_MULTI(RP, T)                                                         \
+  do {                                                                          \
+    auto kern = k_hv_rows_multi<RP, T>;                                         \
+    allow_lds(kern, lm);                                                        \
+    hipLaunchKernelGGL(kern, dim3(gm), dim3(bs), lm, s, P, a.dn.maxrow);        \
+  } while (0)
+#define ED_MULTI_TM(RP)                                                         \
+  do {                                                                          \
+    if (tm == 2) ED_MULTI(RP, 2);                                               \
+    else if (tm == 1) ED_MULTI(RP, 1);                                          \
+    else ED_MULTI(RP, 0);                                                       \
+  } while (0)
+      if (rpt == 1) ED_MULTI_TM(1);
+      else if (rpt == 2) ED_MULTI_TM(2);
+      else ED_MULTI_TM(4);
+#undef ED_MULTI_TM
+#undef ED_MULTI
+      ED_HIP(hipGetLastError());
+      return gm;
+    }
     if (stage && R == 1 && a.up.sell[0].nslice > 0 && a.up.sell[1].nslice > 0) {
-      const int tm = a.up.mode16 ? 2 : (a.up.packed ? 0 : 1);
       // short rows: 4-wave blocks, so that all rows of a small sector are resident at once
       const bool small = a.block == 256 || (a.block == 0 && du < 2048);
 #define ED_SELL(BSZ, DOWN, TMV)                                               \

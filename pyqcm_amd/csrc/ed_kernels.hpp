@@ -37,6 +37,7 @@ struct DevHalf {
   int packed = 1;
   int colbits = 0;
   uint32_t nval = 0;               // size of the value table (packed == 1)
+  uint32_t nnz = 0, maxrow = 0;    // entries of all rows, of the longest row
   // the same operator as sliced-ELL tables (see SellTable): [0] in state
   // order (the fused kernel's down part needs lane u on column u), [1] with
   // the states sorted by row length, which removes most of the padding

@@ -875,6 +875,9 @@ struct DevHalfStore {
     view.packed = H.packed;
     view.colbits = H.colbits;
     view.nval = H.nval;
+    view.nnz = H.ptr[H.dim];
+    view.maxrow = 0;
+    for (uint32_t r = 0; r < H.dim; ++r) view.maxrow = std::max(view.maxrow, H.ptr[r + 1] - H.ptr[r]);
     view.sell[0] = sell_nat.view(true);
     view.sell[1] = sell_sorted.view(w <= 1);
     view.mode16 = t0 != 0.0 ? 1 : 0;

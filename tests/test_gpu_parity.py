@@ -126,6 +126,40 @@ def test_factorized_sliced_ell_modes(oracle, kind, variant, sell16, block, row_o
     assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("row_order", [0, 1])
+@pytest.mark.parametrize("kind,Nup,Ndw", [
+    ("chain", 12, 6), ("chain", 6, 12), ("chain", 11, 6),   # one up state, one row, 12 columns
+    ("chain", 2, 2), ("chain", 4, 6),                       # 66 columns: a slice of 64 and one of 2; 495 x 924
+    ("bath", 7, 4), ("bath", 6, 6),                         # two rows to a workgroup, the last one alone; four
+    ("random", 5, 5), ("random", 3, 6),                     # explicit values, full diagonal: two and four rows
+    ("random", 6, 1)])                                      # 12 rows
+def test_short_rows_at_their_edges(oracle, kind, Nup, Ndw, row_order):
+    """The short-row product, with 16-bit, packed and explicit tables, against
+    the oracle and the general row kernels: added to a vector and written over
+    one.  An element is a sum of at most 36 + 36 + 1 products; the module's bar
+    of 1e-12 of the largest is far above the rounding of that."""
+    wl = {"chain": lambda: W.hubbard_chain(12, U=4.0, mu=2.0), "bath": lambda: W.plaquette_bath(seed=2025),
+          "random": lambda: _random_workload(4, 12)}[kind]()
+    sec = "R0:N%d:S%d" % (Nup + Ndw, Nup - Ndw)
+    H = []
+    for block in (0, 256):
+        qcm.set_global_parameterC("hv_row_order", row_order)
+        qcm.set_global_parameterC("hv_block", block)
+        try:
+            H.append(qcm.Hamiltonian(_instance(wl, sec), sec, "G"))
+        finally:
+            qcm.set_global_parameterC("hv_block", 0)
+            qcm.set_global_parameterC("hv_row_order", 1)
+    rng = np.random.default_rng(Nup + 20 * Ndw)
+    x, y0 = rng.normal(size=(2, H[0].dim))
+    ref = oracle.Model(wl.L, wl.terms()).hv_factorized(Nup, Ndw, x)
+    scale = np.abs(ref).max()
+    for h in H:
+        h.set_variant(1)
+        assert np.abs(h.apply(x) - ref).max() <= 1e-12 * scale
+        assert np.abs(h.mult_add(x, y0.copy()) - y0 - ref).max() <= 1e-12 * (scale + np.abs(y0).max())
+
+
 def test_torus4x4_full_sector_hv_matches_oracle(oracle):
     """The 4x4 periodic cluster at half filling (dim 165 636 900): every kernel
     schedule against the oracle's OpenMP product, and symmetry of H."""
