@@ -756,6 +756,56 @@ __global__ __launch_bounds__(BS) void k_fact_diag(FactArgs a, double *d) {
 // ---------------------------------------------------------------------------
 // CSR SpMV (full symmetric matrix), G lanes per row.
 // ---------------------------------------------------------------------------
+// The same product from slices of 64 rows, one row per lane: 4 bytes per entry
+// instead of 12 and no sum across lanes, neighbouring lanes mostly reading
+// neighbouring x.  Bound by the entries' stream (853 776 states, 12 per row: 53
+// MB in 20 us; 48 us from the compressed rows) and, smaller, by the latency of a
+// slice.  XCD x (blocks b % 8) takes the x-th run of slices, so that its reads
+// of x stay in its own L2.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_hv_csr_slices(CsrArgs A, const double *x, double *y, double ax, double beta,
+                                                      double *part) {
+  __shared__ double red[BS / kWave];
+  __shared__ double tab[kCsrTabMax];
+  for (uint32_t i = threadIdx.x; i < A.ntab; i += BS) tab[i] = A.tab[i];
+  __syncthreads();
+  const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const size_t ns = (A.n + kWave - 1) / kWave, run = (ns + 7) / 8;
+  const size_t s0 = blockIdx.x % 8 * run, s1 = s0 + run < ns ? s0 + run : ns;
+  const uint32_t mask = (uint32_t)(((uint64_t)1 << A.colbits) - 1);
+  double dot = 0.0;
+  for (size_t s = s0 + (size_t)(blockIdx.x / 8) * (BS / kWave) + wave; s < s1; s += (size_t)(gridDim.x / 8) * (BS / kWave)) {
+    const size_t row = s * kWave + lane, own = row < A.n ? row : A.n - 1;
+    const double xo = x[own];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};  // short sums: no more rounding than from 8 lanes
+    const uint4 *g = reinterpret_cast<const uint4 *>(A.ent) + lane;
+    const uint32_t q1 = A.slice[s + 1];
+#pragma unroll 2
+    for (uint32_t q = A.slice[s]; q < q1; ++q) {
+      const uint4 w = g[(size_t)q * kWave];
+      const uint32_t e[4] = {w.x, w.y, w.z, w.w};
+      double xv[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) xv[h] = x[e[h] == kCsrPad ? own : (size_t)(e[h] & mask)];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const double t = acc[h] + tab[e[h] == kCsrPad ? 0u : e[h] >> A.colbits] * xv[h];
+        acc[h] = e[h] == kCsrPad ? acc[h] : t;
+      }
+    }
+    if (row < A.n) {
+      const double sum = (acc[0] + acc[1]) + (acc[2] + acc[3]) + A.diag[row] * xo;
+      const double out = (beta != 0.0) ? ax * sum + beta * y[row] : ax * sum;
+      y[row] = out;
+      dot += out * xo;
+    }
+  }
+  if (part) {
+    const double s = block_sum<BS>(dot, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+  }
+}
+
 template <int BS, int G>
 __global__ __launch_bounds__(BS) void k_hv_csr(CsrArgs A, const double *x, double *y, double ax, double beta,
                                                double *part) {
@@ -1720,6 +1770,13 @@ int hv_csr_max_partials(const CsrArgs &) { return kPartialsCap; }
 int hv_csr(const CsrArgs &A, const double *x, double *y, double ax, double beta, double *part, hipStream_t s) {
   if (!A.n) return 0;
   constexpr int BS = 256, G = 8;
+  if (A.ent) {
+    const size_t run = ((A.n + kWave - 1) / kWave + 7) / 8;  // slices of an XCD
+    const int gs = 8 * (int)std::min<size_t>((run + BS / kWave - 1) / (BS / kWave), kPartialsCap / 8);
+    hipLaunchKernelGGL((k_hv_csr_slices<BS>), dim3(gs), dim3(BS), 0, s, A, x, y, ax, beta, part);
+    ED_HIP(hipGetLastError());
+    return gs;
+  }
   const int g = grid_for(A.n * G, BS, 16);
   hipLaunchKernelGGL((k_hv_csr<BS, G>), dim3(g), dim3(BS), 0, s, A, x, y, ax, beta, part);
   ED_HIP(hipGetLastError());

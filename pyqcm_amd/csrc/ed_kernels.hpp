@@ -93,7 +93,17 @@ struct CsrArgs {
   const uint32_t *col = nullptr;
   const double *val = nullptr;
   const double *diag = nullptr;
+  // sliced form (null: the compressed rows): slices of 64 rows, lane l of slice
+  // s holding row 64 s + l, padded to whole groups of 4 entries that are stored
+  // group-major, lane-minor; an entry is col | id << colbits, kCsrPad padding
+  const uint32_t *slice = nullptr;  // (n + 63) / 64 + 1 offsets, in groups of 64 x 4 entries
+  const uint32_t *ent = nullptr;
+  const double *tab = nullptr;      // ntab values
+  uint32_t ntab = 0;
+  int colbits = 0;
 };
+constexpr uint32_t kCsrPad = 0xffffffffu;
+constexpr uint32_t kCsrTabMax = 256;  // values of a sliced matrix (its table is staged in LDS)
 int hv_csr(const CsrArgs &a, const double *x, double *y, double ax, double beta, double *dot_partials,
            hipStream_t s);
 int hv_csr_max_partials(const CsrArgs &a);

@@ -83,6 +83,36 @@ def test_csr_pattern_bit_exact(oracle):
     assert np.allclose(v, v2, rtol=0, atol=1e-15)
 
 
+@pytest.mark.parametrize("kind,L,Nup,Ndw", [
+    ("chain", 12, 3, 2), ("chain", 12, 4, 2),     # 14 520 states: compressed rows; 32 670: slices, the last of 30 rows
+    ("chain", 14, 4, 2), ("chain", 16, 8, 2),     # the last slice of 19 rows, of 16
+    ("bath", 12, 6, 4), ("random", 10, 3, 5),     # 19 and up to 180 values
+    ("random", 12, 2, 4)])                        # more values than the table holds
+def test_csr_slices_at_their_edges(oracle, kind, L, Nup, Ndw):
+    """The 'S' product from slices of 64 rows against the oracle, written over a
+    vector and added to one, and with an infinite element: only the rows that
+    read it (and itself) turn infinite or NaN."""
+    wl = {"chain": lambda: W.hubbard_chain(L, U=4.0, mu=1.7), "bath": lambda: W.plaquette_bath(seed=2025),
+          "random": lambda: _random_workload(4, L)}[kind]()
+    sec = "R0:N%d:S%d" % (Nup + Ndw, Nup - Ndw)
+    H = qcm.Hamiltonian(_instance(wl, sec), sec, "S")
+    rng = np.random.default_rng(L + Nup)
+    x, y0 = rng.normal(size=(2, H.dim))
+    M = oracle.Model(wl.L, wl.terms())
+    ref = M.hv_factorized(Nup, Ndw, x)
+    scale = np.abs(ref).max()
+    assert np.abs(H.apply(x) - ref).max() <= 1e-12 * scale
+    assert np.abs(H.mult_add(x, y0.copy()) - y0 - ref).max() <= 1e-12 * (scale + np.abs(y0).max())
+    for k in (63, H.dim - 1):
+        e = np.zeros(H.dim)
+        e[k] = 1.0
+        reads = M.hv_factorized(Nup, Ndw, e) != 0.0
+        reads[k] = True
+        x[k] = np.inf
+        assert np.array_equal(~np.isfinite(H.apply(x)), reads)
+        x[k] = 1.0
+
+
 @pytest.mark.parametrize("variant", [1, 2, 3])
 def test_factorized_variants_agree(oracle, variant):
     wl = W.plaquette_bath(n_bath=4)     # L = 8, dim(4,4) = 4900
