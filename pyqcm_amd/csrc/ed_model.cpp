@@ -1164,9 +1164,9 @@ void csr_lower(const TermList &T, int Nup, int Ndw, std::vector<int32_t> &Iptr, 
 // bytes than the 12 per entry of the compressed rows (the streams bound the
 // product); empty otherwise, and below kCsrSlicesMin states, where a row's
 // entries are read at once by 8 lanes (us of one product, compressed / sliced:
-// 2520 states 2.8 / 3.1, 4900 2.9 / 3.3, 63 504 5.1 / 4.8, 853 776 48 / 20,
-// 2 944 656 227 / 85).
-constexpr size_t kCsrSlicesMin = 16384;
+// 4900 states 2.9 / 3.3, 25 200 3.5 / 4.4, 54 450 4.8 / 4.6, 108 900 7.0 / 5.1,
+// 213 444 16 / 7.4, 853 776 48 / 20, 2 944 656 227 / 85).
+constexpr size_t kCsrSlicesMin = 49152;
 struct CsrSlices {
   std::vector<uint32_t> slice, ent;
   std::vector<double> tab;

@@ -84,10 +84,10 @@ def test_csr_pattern_bit_exact(oracle):
 
 
 @pytest.mark.parametrize("kind,L,Nup,Ndw", [
-    ("chain", 12, 3, 2), ("chain", 12, 4, 2),     # 14 520 states: compressed rows; 32 670: slices, the last of 30 rows
+    ("chain", 12, 3, 3), ("chain", 12, 5, 2),     # 48 400 states: compressed rows; 52 272: slices, the last of 48 rows
     ("chain", 14, 4, 2), ("chain", 16, 8, 2),     # the last slice of 19 rows, of 16
-    ("bath", 12, 6, 4), ("random", 10, 3, 5),     # 19 and up to 180 values
-    ("random", 12, 2, 4)])                        # more values than the table holds
+    ("bath", 12, 6, 4), ("random", 10, 4, 5),     # 19 and up to 180 values
+    ("random", 12, 2, 5)])                        # more values than the table holds
 def test_csr_slices_at_their_edges(oracle, kind, L, Nup, Ndw):
     """The 'S' product from slices of 64 rows against the oracle, written over a
     vector and added to one, and with an infinite element: only the rows that
