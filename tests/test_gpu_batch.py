@@ -3,6 +3,7 @@ the per-instance path on the same parameters and against dense
 diagonalization.  Bars: E0 1e-10 relative; G(z) 1e-8 on a Matsubara grid,
 both spin blocks."""
 import dataclasses
+import math
 
 import numpy as np
 import pytest
@@ -96,6 +97,17 @@ def test_batch_2x3_neel_points_continued_fractions():
 def test_batch_ground_states_with_band_lanczos_green_functions():
     """GF_method 'L': batched ground states, band-Lanczos Green functions per instance."""
     _compare(W.vca_cluster(2, 2), W.vca_points(3, seed=6), "L", W.matsubara(32, 20.0))
+
+
+@pytest.mark.parametrize("L,N,S,dim", [(2, 1, 1, 2), (4, 1, 1, 4), (5, 1, 1, 5), (3, 2, 0, 9), (5, 2, 2, 10),
+                                       (4, 4, 0, 36), (5, 4, 0, 100), (6, 4, 0, 225)])
+def test_ground_states_whose_krylov_space_ends_between_checks(L, N, S, dim):
+    """Ritz pairs are found every fourth step and wherever the Krylov space may
+    end: as many states as one, between one and two checks, and more, in the
+    one-wave and the four-wave workgroup."""
+    wl = dataclasses.replace(W.hubbard_chain(L, U=4.0, mu=1.3), sector="R0:N%d:S%d" % (N, S))
+    assert math.comb(L, (N + S) // 2) * math.comb(L, (N - S) // 2) == dim
+    _compare(wl, [{"t": 1.0, "U": 4.0, "mu": 1.3}, {"t": 1.0, "U": 7.0, "mu": 2.2}], "F", W.matsubara(16, 20.0))
 
 
 def test_batch_large_sector_four_wave_kernel():
