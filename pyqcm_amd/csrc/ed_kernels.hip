@@ -22,8 +22,9 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Block-wide sum over nw waves; result valid in thread 0.  sh must hold nw doubles.
-__device__ __forceinline__ double block_sum(double v, double *sh, int nw) {
+// Block-wide sum; result valid in thread 0.  sh must hold BS/64 doubles.
+template <int BS>
+__device__ __forceinline__ double block_sum(double v, double *sh) {
   v = wave_sum(v);
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   __syncthreads();
@@ -31,14 +32,10 @@ __device__ __forceinline__ double block_sum(double v, double *sh, int nw) {
   __syncthreads();
   double r = 0.0;
   if (threadIdx.x < kWave) {
-    r = ((int)threadIdx.x < nw) ? sh[threadIdx.x] : 0.0;
+    r = (threadIdx.x < BS / kWave) ? sh[threadIdx.x] : 0.0;
     r = wave_sum(r);
   }
   return r;
-}
-template <int BS>
-__device__ __forceinline__ double block_sum(double v, double *sh) {
-  return block_sum(v, sh, BS / kWave);
 }
 
 __device__ __forceinline__ double half_entry(const DevHalf &h, const double *vtab, uint32_t e, uint32_t &col) {
@@ -51,11 +48,12 @@ __device__ __forceinline__ double half_entry(const DevHalf &h, const double *vta
   return h.val[e];
 }
 
-__device__ __forceinline__ double diag_value(const FactArgs &a, const double *Ush, size_t I, uint32_t u,
-                                             uint32_t d, uint32_t sd) {
+// diagonal of state I = (u, d) from the down half state sd and its own diagonal ddiag
+__device__ __forceinline__ double diag_of_row(const FactArgs &a, const double *Ush, size_t I, uint32_t u,
+                                              double ddiag, uint32_t sd) {
   if (a.diag_mode == 0) return a.dg[I];
   const uint32_t su = a.up.states[u];
-  double s = a.up.diag[u] + a.dn.diag[d];
+  double s = a.up.diag[u] + ddiag;
   uint32_t m = su & sd;
   if (a.diag_mode == 2) return s + Ush[0] * (double)__popc(m);
   while (m) {
@@ -64,6 +62,10 @@ __device__ __forceinline__ double diag_value(const FactArgs &a, const double *Us
     m &= m - 1u;
   }
   return s;
+}
+__device__ __forceinline__ double diag_value(const FactArgs &a, const double *Ush, size_t I, uint32_t u,
+                                             uint32_t d, uint32_t sd) {
+  return diag_of_row(a, Ush, I, u, a.dn.diag[d], sd);
 }
 
 struct FusedParams {
@@ -413,128 +415,234 @@ __global__ __launch_bounds__(BS) void k_hv_rows_sell(FusedParams P) {
   }
 }
 
-// Row kernel for short rows: RPT rows per workgroup, one column of all of them
-// per thread, so that a column's table entries, diagonal parts and the entry
-// values are read once for RPT rows, and the RPT rows' reads of a neighbour
-// are in flight together.  Bound by the latency and the L1 rate of those reads,
-// not by memory (the vector stays in the XCD's L2).  With one row per workgroup
-// of four waves, every row re-read the whole up table, 190 MB of vector memory
-// traffic for a 6.8 MB vector of 924 x 924 states, and each wave walked its
-// slices one latency after the other; rows below 512 states, several to a
-// workgroup, went state by state through the compressed rows.  The neighbour
-// lists are staged in LDS, padded to emax entries (own row, value 0).  The rows
-// of an XCD are one run of the breadth-first order, whose hops stay close: 924 x
-// 924 17.4 us with the rows dealt out to the XCDs in turn, 16.5 so.  Sizes and
-// times: short_row_count.
-template <int RPT, int TM>
-__global__ __launch_bounds__(1024) void k_hv_rows_multi(FusedParams P, uint32_t emax) {
+// Row kernel for short rows: RPT rows per workgroup, one column of all of them per
+// thread, so that a column's table entries, diagonal parts and the entry values are
+// read once for RPT rows, and the RPT rows' reads of a neighbour are in flight
+// together.  Bound by the latency and the L1 rate of those reads, not by memory (the
+// vector stays in the XCD's L2).  With one row per workgroup of four waves, every row
+// re-read the whole up table, 190 MB of vector memory traffic for a 6.8 MB vector of
+// 924 x 924 states, and each wave walked its slices one latency after the other; rows
+// below 512 states, several to a workgroup, went state by state through the compressed
+// rows.  The neighbour lists are staged in LDS, padded to emax entries (own row, value
+// 0).  The rows of an XCD are one run of the breadth-first order, whose hops stay
+// close.  Sizes and times: short_row_plan.
+//
+// Every sum is that of the general kernels, term by term: a Krylov run that stops at
+// its lowest Ritz value leaves a Green function that rounding moves by up to 1e-5, so
+// a product whose sums ran in another order gave other results.  SEQ (rows below 512
+// states, k_hv_rows): diagonal, up entries, down entries in one chain; else
+// (k_hv_rows_sell) the up entries in two chains, the diagonal on their sum, then the
+// down entries.  The partials of <y, x> are those of the general kernel's workgroup of
+// nvw waves, one per row or (SEQ) one per ng rows in label order, which are this
+// workgroup's then, side by side with one row per thread.  Its wave w walks the
+// 64-column pieces w, w + nvw, ... in one chain.  Here a wave walks nvw / waves chains
+// by turns (DOT 1), or a chain passes through LDS from wave to wave (DOT 2, nvw = 4 and
+// a multiple of four waves); DOT 0 forms no partials.
+template <int RPT, int TM, bool SEQ, int DOT>
+__global__ __launch_bounds__(1024) void k_hv_rows_multi(FusedParams P, uint32_t emax, uint32_t ng, uint32_t nvw) {
   extern __shared__ double smem[];
-  const uint32_t BS = blockDim.x;
+  constexpr uint32_t kPass = 4;  // nvw of DOT 2
+  constexpr bool FLAT = SEQ && DOT;  // G = ng rows side by side, one per thread; else G = RPT
+  const uint32_t BS = blockDim.x, NW = BS / kWave;
   __shared__ double Ush[32];
-  __shared__ double vtu[kVtabMax];
-  __shared__ double red[1024 / kWave];
+  __shared__ double vtu[TM == 0 ? kVtabMax : 1];
+  __shared__ uint32_t rows[RPT];
+  __shared__ double red[DOT ? RPT * 16 : 1];
+  __shared__ double chain[DOT == 2 ? kPass : 1][RPT][kWave];
   const FactArgs &a = P.a;
-  const uint32_t du = a.up.dim, dd = a.dn.dim, pitch = du + 1;
-  double *xs = smem, *nval = smem + RPT * pitch;
-  uint32_t *ncol = reinterpret_cast<uint32_t *>(nval + RPT * emax);
+  const uint32_t du = a.up.dim, dd = a.dn.dim, pitch = du + 1, G = FLAT ? ng : RPT;
+  double *xs = smem, *nval = smem + G * pitch;
+  uint32_t *ncol = reinterpret_cast<uint32_t *>(nval + G * emax);
   if (threadIdx.x < 32) Ush[threadIdx.x] = a.Uc[threadIdx.x];
   if (TM == 0)
     for (uint32_t i = threadIdx.x; i < (uint32_t)P.ntab_up; i += BS) vtu[i] = a.up.val[i];
   const double *vtab_u = P.ntab_up ? vtu : a.up.val;
   const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   // XCD x (blocks b % 8) takes the x-th run of rows
-  const uint32_t blk = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const uint32_t blk = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8, i0 = blk * G;
+  if (i0 >= dd) return;
+  // (rows past the last one repeat it and are not stored)
   uint32_t d[RPT];
+  if (FLAT) {
+    for (uint32_t f = threadIdx.x; f < G * pitch; f += BS) {
+      const uint32_t r = f / pitch, c = f - r * pitch;
+      xs[f] = c < du ? P.x[(size_t)min(i0 + r, dd - 1) * du + c] : 0.0;
+    }
+    for (uint32_t f = threadIdx.x; f < G * emax; f += BS) {
+      const uint32_t r = f % G, i = min(i0 + r, dd - 1), e = a.dn.ptr[i] + f / G;
+      uint32_t c = i;
+      const double v = e < a.dn.ptr[i + 1] ? half_entry(a.dn, a.dn.val, e, c) : 0.0;
+      ncol[f] = c;
+      nval[f] = v;
+    }
+  } else {
 #pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    const uint32_t i = min(blk * RPT + j, dd - 1);  // past the last row: repeated, not stored
-    d[j] = a.row_order ? a.dn.order[i] : i;
+    for (int j = 0; j < RPT; ++j) {
+      const uint32_t i = min(i0 + j, dd - 1);
+      d[j] = a.row_order ? a.dn.order[i] : i;
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const double *xr = P.x + (size_t)d[j] * du;
+      for (uint32_t f = threadIdx.x; f < pitch; f += BS) xs[j * pitch + f] = f < du ? xr[f] : 0.0;
+    }
+    // (the rows' lists in one pass, and the row numbers read back from LDS: 924 x
+    // 924 14.6 us; list after list, row numbers in registers: 15.4)
+    for (uint32_t f = threadIdx.x; f < RPT * emax; f += BS) {
+      const uint32_t r = min(i0 + f % RPT, dd - 1), i = a.row_order ? a.dn.order[r] : r;
+      const uint32_t e = a.dn.ptr[i] + f / RPT;
+      uint32_t c = i;
+      const double v = e < a.dn.ptr[i + 1] ? half_entry(a.dn, a.dn.val, e, c) : 0.0;
+      ncol[f] = c;
+      nval[f] = v;
+    }
+    if (RPT > 1 && threadIdx.x < RPT) {
+      const uint32_t r = min(i0 + threadIdx.x, dd - 1);
+      rows[threadIdx.x] = a.row_order ? a.dn.order[r] : r;
+    }
   }
+  if (DOT == 2 && wave < kPass)
 #pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    const double *xr = P.x + (size_t)d[j] * du;
-    for (uint32_t f = threadIdx.x; f < pitch; f += BS) xs[j * pitch + f] = f < du ? xr[f] : 0.0;
-    const uint32_t g0 = a.dn.ptr[d[j]], nnb = a.dn.ptr[d[j] + 1] - g0;
-    for (uint32_t q = threadIdx.x; q < emax; q += BS) {
-      uint32_t c = d[j];
-      const double v = q < nnb ? half_entry(a.dn, a.dn.val, g0 + q, c) : 0.0;
-      ncol[q * RPT + j] = c;
-      nval[q * RPT + j] = v;
+    for (int j = 0; j < RPT; ++j) chain[wave][j][lane] = 0.0;
+  constexpr uint32_t kOwn = 4 / RPT;  // chains of a wave, at most
+  double own[kOwn][RPT] = {};
+  uint32_t turn = 0;
+  __syncthreads();
+  const SellTable &T = a.up.sell[0];
+  const uint32_t n = FLAT ? ng * du : du, nf = DOT == 2 ? (n + BS - 1) / BS * BS : n;  // DOT 2: all waves meet in each round
+  for (uint32_t f = threadIdx.x; f - lane < nf; f += BS) {
+    double out[RPT], xo[RPT];
+    if (f - lane < n) {
+      const uint32_t fc = min(f, n - 1), r0 = FLAT ? fc / du : 0u, u = fc - r0 * du;
+      const uint32_t s = u / kWave, sl = u % kWave;  // slice of the table and lane in it
+      const double *xg = xs + r0 * pitch;
+      double acc[RPT];
+      if (FLAT) d[0] = min(i0 + r0, dd - 1);
+      if (RPT > 1)
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) d[j] = rows[j];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        acc[j] = diag_value(a, Ush, (size_t)d[j] * du + u, u, d[j], a.diag_mode ? a.dn.states[d[j]] : 0u);
+        if (SEQ) acc[j] *= xg[j * pitch + u];
+      }
+      // SEQ: acc is the running sum; else e and o are the up part's two chains
+      double e[RPT], o[RPT];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) e[j] = o[j] = 0.0;
+      const size_t o0 = T.off[s], o1 = T.off[s + 1];
+      if (TM == 1) {
+        for (size_t q = o0 + sl; q < o1; q += kWave) {
+          const double v = T.val[q];
+          const uint32_t c = T.ent[q];
+#pragma unroll
+          for (int j = 0; j < RPT; ++j) {
+            double &sum = SEQ ? acc[j] : e[j];
+            sum = fma(v, xg[j * pitch + c], sum);
+          }
+        }
+      } else {
+        const uint32_t nq = (uint32_t)((o1 - o0) / (kWave * 4)), mask = (1u << a.up.colbits) - 1u;
+#pragma unroll 2
+        for (uint32_t q = 0; q < nq; ++q) {
+          uint32_t c[4];
+          double v[4];
+          if (TM == 2) {
+            const uint2 w2 = reinterpret_cast<const uint2 *>(T.e16 + o0)[(size_t)q * kWave + sl];
+            const uint32_t w[4] = {w2.x & 0xffffu, w2.x >> 16, w2.y & 0xffffu, w2.y >> 16};
+            const double t = SEQ ? a.up.t0 : 1.0;
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+              c[h] = w[h] & 0x7fffu;
+              v[h] = w[h] & 0x8000u ? -t : t;
+            }
+          } else {
+            const uint4 w4 = reinterpret_cast<const uint4 *>(T.ent + o0)[(size_t)q * kWave + sl];
+            const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+              c[h] = w[h] & mask;
+              v[h] = vtab_u[w[h] >> a.up.colbits];
+            }
+          }
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+              double &sum = SEQ ? acc[j] : (h & 1 ? o[j] : e[j]);
+              sum = fma(v[h], xg[j * pitch + c[h]], sum);
+            }
+        }
+      }
+      if (!SEQ)
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+          double up = TM == 1 ? e[j] : e[j] + o[j];
+          if (TM == 2) up *= a.up.t0;
+          acc[j] = fma(acc[j], xg[j * pitch + u], up);
+        }
+#pragma unroll 4
+      for (uint32_t q = 0; q < emax; ++q) {
+        double xv[RPT];
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) xv[j] = P.x[(size_t)ncol[q * G + r0 + j] * du + u];
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) acc[j] = fma(nval[q * G + r0 + j], xv[j], acc[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        const size_t I = (size_t)d[j] * du + u;
+        out[j] = P.ax * acc[j];
+        xo[j] = 0.0;
+        if (f < n && i0 + r0 + j < dd) {
+          if (P.beta != 0.0) out[j] = fma(P.beta, P.y[I], out[j]);
+          P.y[I] = out[j];
+          if (DOT) xo[j] = xg[j * pitch + u];
+        } else if (DOT) {
+          out[j] = 0.0;  // adds nothing to a chain
+        }
+      }
+    }
+    if (DOT == 1) {
+#pragma unroll
+      for (uint32_t k = 0; k < kOwn; ++k)
+        if (k == turn)
+#pragma unroll
+          for (int j = 0; j < RPT; ++j) own[k][j] = fma(out[j], xo[j], own[k][j]);
+      if (++turn * NW == nvw) turn = 0;
+    }
+    if (DOT == 2)
+      for (uint32_t k = 0; k < NW / kPass; ++k) {
+        if (wave / kPass == k && f < n)
+#pragma unroll
+          for (int j = 0; j < RPT; ++j) {
+            double &c = chain[wave % kPass][j][lane];
+            c = fma(out[j], xo[j], c);
+          }
+        __syncthreads();
+      }
+  }
+  if (!DOT) return;
+  const uint32_t nres = SEQ ? 1u : min(G, dd - i0);
+  if (DOT == 1) {
+#pragma unroll
+    for (uint32_t k = 0; k < kOwn; ++k)
+#pragma unroll
+      for (int j = 0; j < RPT; ++j)
+        if (wave + k * NW < nvw) {
+          const double s = wave_sum(own[k][j]);
+          if (lane == 0) red[j * nvw + wave + k * NW] = s;
+        }
+  } else {
+    for (uint32_t v = wave; v < nres * nvw; v += NW) {
+      const double s = wave_sum(chain[v % nvw][v / nvw][lane]);
+      if (lane == 0) red[v] = s;
     }
   }
   __syncthreads();
-  const SellTable &T = a.up.sell[0];
-  double dot = 0.0;
-  for (uint32_t s = blk * RPT < dd ? wave : T.nslice; s < T.nslice; s += BS / kWave) {
-    const uint32_t u = s * kWave + lane, uu = min(u, du - 1);
-    double acc[RPT];
-#pragma unroll
-    for (int j = 0; j < RPT; ++j)
-      acc[j] = diag_value(a, Ush, (size_t)d[j] * du + uu, uu, d[j], a.diag_mode ? a.dn.states[d[j]] : 0u) *
-               xs[j * pitch + uu];
-    const size_t o0 = T.off[s], o1 = T.off[s + 1];
-    if (TM == 1) {
-      for (size_t e = o0 + lane; e < o1; e += kWave) {
-        const double v = T.val[e];
-        const uint32_t c = T.ent[e];
-#pragma unroll
-        for (int j = 0; j < RPT; ++j) acc[j] += v * xs[j * pitch + c];
-      }
-    } else {
-      double up[RPT];
-#pragma unroll
-      for (int j = 0; j < RPT; ++j) up[j] = 0.0;
-      const uint32_t nq = (uint32_t)((o1 - o0) / (kWave * 4)), mask = (1u << a.up.colbits) - 1u;
-#pragma unroll 2
-      for (uint32_t q = 0; q < nq; ++q) {
-        uint32_t c[4];
-        double v[4];
-        if (TM == 2) {
-          const uint2 g = reinterpret_cast<const uint2 *>(T.e16 + o0)[(size_t)q * kWave + lane];
-          const uint32_t e[4] = {g.x & 0xffffu, g.x >> 16, g.y & 0xffffu, g.y >> 16};
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            c[h] = e[h] & 0x7fffu;
-            v[h] = e[h] & 0x8000u ? -1.0 : 1.0;
-          }
-        } else {
-          const uint4 g = reinterpret_cast<const uint4 *>(T.ent + o0)[(size_t)q * kWave + lane];
-          const uint32_t e[4] = {g.x, g.y, g.z, g.w};
-#pragma unroll
-          for (int h = 0; h < 4; ++h) {
-            c[h] = e[h] & mask;
-            v[h] = vtab_u[e[h] >> a.up.colbits];
-          }
-        }
-#pragma unroll
-        for (int h = 0; h < 4; ++h)
-#pragma unroll
-          for (int j = 0; j < RPT; ++j) up[j] += v[h] * xs[j * pitch + c[h]];
-      }
-#pragma unroll
-      for (int j = 0; j < RPT; ++j) acc[j] += TM == 2 ? a.up.t0 * up[j] : up[j];
-    }
-#pragma unroll 4
-    for (uint32_t q = 0; q < emax; ++q) {
-      double xv[RPT];
-#pragma unroll
-      for (int j = 0; j < RPT; ++j) xv[j] = P.x[(size_t)ncol[q * RPT + j] * du + uu];
-#pragma unroll
-      for (int j = 0; j < RPT; ++j) acc[j] += nval[q * RPT + j] * xv[j];
-    }
-    if (u < du)
-#pragma unroll
-      for (int j = 0; j < RPT; ++j)
-        if (blk * RPT + j < dd) {
-          const size_t I = (size_t)d[j] * du + u;
-          const double out = (P.beta != 0.0) ? P.ax * acc[j] + P.beta * P.y[I] : P.ax * acc[j];
-          P.y[I] = out;
-          dot += out * xs[j * pitch + u];
-        }
-  }
-  if (P.part) {
-    const double s = block_sum(dot, red, (int)BS / kWave);
-    if (threadIdx.x == 0) P.part[blockIdx.x] = s;
+  for (uint32_t r = wave; r < nres; r += NW) {
+    const double s = wave_sum(lane < nvw ? red[r * nvw + lane] : 0.0);
+    if (lane == 0) P.part[SEQ ? blk : i0 + r] = s;
   }
 }
 
@@ -1527,42 +1635,64 @@ static int fused_grid(const FactArgs &a, uint32_t R) {
 // Dynamic LDS of the short-row kernel (the CU's 160 KB less its static tables)
 constexpr size_t kShortRowLds = 140 * 1024;
 constexpr uint32_t kShortRow = 4096;
-static size_t short_row_lds(const FactArgs &a, int rpt) {
-  return rpt * (((size_t)a.up.dim + 1 + a.dn.maxrow) * sizeof(double) + a.dn.maxrow * sizeof(uint32_t));
+static size_t short_row_lds(const FactArgs &a, uint32_t rows) {
+  return rows * (((size_t)a.up.dim + 1 + a.dn.maxrow) * sizeof(double) + a.dn.maxrow * sizeof(uint32_t));
 }
 
-// Rows per workgroup of the short-row kernel; 0: the general row kernels.
+// The short-row kernel's schedule: rpt rows per thread (0: the general row
+// kernels), ng rows side by side per workgroup.
 // The rows that the fullest CU works on, each at the cost of a row among 1, 2
 // or 4: where the up table is heavy (20 bytes or more per state) the shared
 // read of it makes the rows of a larger group cheaper, with a light one it
-// does not.  us of one product against the general kernels:
-//   heavy  924 x 924 (4 rows) 20.8 -> 16.5, 1716^2 (4) 60 -> 48,
-//          1287^2 (2) 34.7 -> 33.6, 3432^2 (4) 230 -> 185, 364 rows of 3432 (2) 32 -> 27
-//   light  70 x 70 (1) 9.5 -> 4.7, 252 x 252 (1) 15.4 -> 5, 1001^2 (1) 17.2 -> 12.5,
-//          1287^2 (1) 24.7 -> 23.9, 3003^2 (1) 121 -> 101
+// does not.  us of one product, general kernels -> this one (clusters: open
+// chains, plaquette + bath, periodic 4 x 3 and 4 x 4):
+//   heavy  924^2 plaquette (4 rows) 19.8 -> 14.5, periodic 18.3 -> 16.7; 1716^2 (4)
+//          57 -> 43; 1820^2 periodic (4) 58 -> 49; 3432^2 (4) 217 -> 169; 364
+//          columns of 3432 rows (2) 40 -> 23
+//   light  70^2 (1) 8.9 -> 4.3, 252^2 (1) 14.5 -> 4.6, 1287^2 (1) 23.0 -> 22.2,
+//          1716^2 (1) 43 -> 35, 3003^2 (1) 118 -> 97
 // With light tables 2 or 4 rows lose (1287^2: 27 and 30 us), with heavy ones 1
-// row does (924^2: 20 us).  From kShortRow states on a row is long enough to
-// keep a workgroup of 16 waves busy by itself, and the rows in flight no longer
-// fit the XCD's L2: 6435 x 5005 0.65 ms general, 0.77 here; 12870^2 3.8 and 5.6.
-// Rows of more than 64 neighbours, and blocks asked for by size, stay general.
-static int short_row_count(const FactArgs &a) {
-  if (a.block != 0 || a.up.dim >= kShortRow || a.up.sell[0].nslice == 0 || a.dn.maxrow > 64)
-    return 0;
+// row does (924^2: 20 us), and 1 row in four waves is the general kernel over
+// again, a little slower (560^2 periodic 8.6 -> 9.0, 715^2 plaquette 12.0 -> 12.5):
+// those stay general.  From kShortRow states on a row is long enough to keep a
+// workgroup of 16 waves busy by itself, and the rows in flight no longer fit the
+// XCD's L2: 6435 x 5005 0.65 ms general, 0.77 here; 12870^2 3.8 and 5.6.  Rows of
+// more than 64 neighbours, and blocks asked for by size, stay general, as do
+// sectors whose general kernels walk more rows than they have partials.
+// With partials (dot) rows below 512 states take the general kernel's R rows per
+// workgroup, one per thread, since each such group has one partial; and a chain
+// that passes between waves costs most where workgroups follow one another on a
+// CU, so that 4 rows are left to sectors whose workgroups run at once (1820 x 4368
+// periodic, with the fold: general 149 us, 4 rows 167, 2 rows 141; 1716^2, which
+// runs at once: 73 and 63).
+struct ShortRows {
+  int rpt = 0;
+  uint32_t ng = 1;
+};
+static ShortRows short_row_plan(const FactArgs &a, bool dot) {
+  ShortRows S;
+  const uint32_t R = rows_per_block(a.up.dim);
+  if (a.block != 0 || a.up.dim >= kShortRow || R == 0 || a.up.sell[0].nslice == 0 || a.up.sell[1].nslice == 0 ||
+      a.dn.maxrow > 64 || (a.dn.dim + R - 1) / R > (uint32_t)kPartialsCap)
+    return S;
   const size_t entry = a.up.mode16 ? 2 : (a.up.packed ? 4 : 12);
-  const bool heavy = a.up.nnz * entry >= 20 * (size_t)a.up.dim;
+  const bool heavy = a.up.nnz * entry >= 20 * (size_t)a.up.dim, fixed = dot && R > 1;
   const double cost[3] = {1.0, heavy ? 0.93 : 1.0, heavy ? 0.8 : 1.0};
-  int best = 0;
   double least = 0.0;
   for (int k = 0; k < 3; ++k) {
     const uint32_t rpt = 1u << k, nb = (a.dn.dim + rpt - 1) / rpt;
-    if (nb > (uint32_t)kPartialsCap - 8 || short_row_lds(a, rpt) > kShortRowLds) continue;
+    const size_t lds = short_row_lds(a, fixed ? R : rpt);
+    if ((fixed && k > 0) || lds > kShortRowLds) continue;
+    if (dot && R == 1 && a.up.dim < 2048 && nb > 512 && kShortRowLds / lds == 2) continue;
     const double t = cost[k] * (double)rpt * ((nb + 255) / 256);
-    if (!best || t < least) {
-      best = (int)rpt;
+    if (!S.rpt || t < least) {
+      S.rpt = (int)rpt;
+      S.ng = fixed ? R : 1;
       least = t;
     }
   }
-  return best;
+  if (heavy && R == 1 && S.rpt == 1 && a.dn.dim > 512) S.rpt = 0;
+  return S;
 }
 
 int hv_factorized_max_partials(const FactArgs &a, int variant) { return kPartialsCap; }
@@ -1604,37 +1734,56 @@ int hv_factorized_cfg(const FactArgs &a, const double *x, double *y, double ax, 
   } while (0)
     const uint32_t kneed = (du + BS - 1) / BS;
     const int tm = a.up.mode16 ? 2 : (a.up.packed ? 0 : 1);
-    const int rpt = short_row_count(a);
-    if (down_here && rpt > 0) {
-      const int gm = 8 * (int)(((dd + rpt - 1) / rpt + 7) / 8);
-      const size_t lm = short_row_lds(a, rpt);
+    const ShortRows sr = down_here ? short_row_plan(a, part != nullptr) : ShortRows();
+    if (sr.rpt > 0) {
+      const uint32_t G = sr.rpt * sr.ng, items = (sr.ng * du + kWave - 1) / kWave;
+      const int gm = 8 * (int)(((dd + G - 1) / G + 7) / 8);
+      const size_t lm = short_row_lds(a, G);
       // About 16 waves in flight per CU (fewer hide no latency, more crowd the
       // CU's L1), as many on each SIMD.  1716 x 1716 states, 4 rows, 2
       // workgroups per CU: 8 waves each 49 us, 4 60, 16 53; 924 x 924, 4 rows,
       // 1 per CU: 16 waves 16 us, 8 18, 4 25; 1287 x 1287, 2 rows, 3 per CU:
       // 4 waves 33 us, 6 43, 8 34.
       const size_t resident = std::min<size_t>((gm + 255) / 256, kShortRowLds / lm);
-      const int waves = resident == 1 ? 16 : (resident == 2 ? 8 : 4);
-      const int bs = kWave * std::min<int>(waves, (du + kWave - 1) / kWave);
-#define ED_MULTI(RP, T)                                                         \
-  do {                                                                          \
-    auto kern = k_hv_rows_multi<RP, T>;                                         \
-    allow_lds(kern, lm);                                                        \
-    hipLaunchKernelGGL(kern, dim3(gm), dim3(bs), lm, s, P, a.dn.maxrow);        \
+      int waves = resident == 1 ? 16 : (resident == 2 ? 8 : 4);
+      // with partials: a divisor of the sixteen waves of the general kernel (at
+      // most 4 / rpt chains each), or a multiple of its four
+      const int nvw = du < 2048 ? 4 : 16;
+      if (!part) waves = std::min<int>(waves, items);
+      else waves = std::max(waves, nvw * sr.rpt / 4);
+      const int bs = kWave * waves, dot = !part ? 0 : (waves <= nvw ? 1 : 2);
+#define ED_MULTI(RP, T, SQ, DT)                                                           \
+  do {                                                                                    \
+    auto kern = k_hv_rows_multi<RP, T, SQ, DT>;                                           \
+    allow_lds(kern, lm);                                                                  \
+    hipLaunchKernelGGL(kern, dim3(gm), dim3(bs), lm, s, P, a.dn.maxrow, sr.ng, (uint32_t)nvw); \
   } while (0)
-#define ED_MULTI_TM(RP)                                                         \
-  do {                                                                          \
-    if (tm == 2) ED_MULTI(RP, 2);                                               \
-    else if (tm == 1) ED_MULTI(RP, 1);                                          \
-    else ED_MULTI(RP, 0);                                                       \
+#define ED_MULTI_TM(RP, SQ, DT)                                                           \
+  do {                                                                                    \
+    if (tm == 2) ED_MULTI(RP, 2, SQ, DT);                                                 \
+    else if (tm == 1) ED_MULTI(RP, 1, SQ, DT);                                            \
+    else ED_MULTI(RP, 0, SQ, DT);                                                         \
   } while (0)
-      if (rpt == 1) ED_MULTI_TM(1);
-      else if (rpt == 2) ED_MULTI_TM(2);
-      else ED_MULTI_TM(4);
+#define ED_MULTI_DOT(RP, SQ)                                                              \
+  do {                                                                                    \
+    if (dot == 2) ED_MULTI_TM(RP, SQ, 2);                                                 \
+    else if (dot == 1) ED_MULTI_TM(RP, SQ, 1);                                            \
+    else ED_MULTI_TM(RP, SQ, 0);                                                          \
+  } while (0)
+      if (R > 1) {
+        if (sr.rpt == 1) ED_MULTI_DOT(1, true);
+        else if (sr.rpt == 2) ED_MULTI_TM(2, true, 0);
+        else ED_MULTI_TM(4, true, 0);
+      } else {
+        if (sr.rpt == 1) ED_MULTI_DOT(1, false);
+        else if (sr.rpt == 2) ED_MULTI_DOT(2, false);
+        else ED_MULTI_DOT(4, false);
+      }
+#undef ED_MULTI_DOT
 #undef ED_MULTI_TM
 #undef ED_MULTI
       ED_HIP(hipGetLastError());
-      return gm;
+      return g;
     }
     if (stage && R == 1 && a.up.sell[0].nslice > 0 && a.up.sell[1].nslice > 0) {
       // short rows: 4-wave blocks, so that all rows of a small sector are resident at once

@@ -1,11 +1,14 @@
 """GPU parity of the HIP path against the CPU oracle (and, for tiny sectors, the
 dense Jordan-Wigner Hamiltonian).  Bars: bit-exact for bases / patterns /
 sign tables; 1e-12 relative for H.x; 1e-10 relative for E0; 1e-8 for G(z)."""
+import math
+
 import numpy as np
 import pytest
 
 from pyqcm_amd import qcm, workloads as W, _lib
 from tests.dense_ref import dense_hamiltonian
+from tests.test_zz_no_alloc import _Dev
 
 pytestmark = pytest.mark.gpu
 
@@ -188,6 +191,57 @@ def test_short_rows_at_their_edges(oracle, kind, Nup, Ndw, row_order):
         h.set_variant(1)
         assert np.abs(h.apply(x) - ref).max() <= 1e-12 * scale
         assert np.abs(h.mult_add(x, y0.copy()) - y0 - ref).max() <= 1e-12 * (scale + np.abs(y0).max())
+
+
+@pytest.mark.parametrize("row_order", [0, 1])
+@pytest.mark.parametrize("kind,L,Nup,Ndw", [
+    # below 512 columns: 8, 16 and 4 rows to a partial sum, one column, 12, 495 (two rows)
+    ("chain", 8, 4, 4), ("chain", 8, 3, 4), ("chain", 10, 5, 5), ("chain", 12, 12, 6), ("chain", 12, 11, 6),
+    ("chain", 12, 4, 6), ("bath", 12, 4, 5), ("bath", 12, 2, 3), ("bath", 12, 1, 1), ("random", 12, 3, 6),
+    ("random", 10, 3, 4),
+    # the same with four waves
+    ("chain", 13, 3, 6), ("bath", 13, 3, 6), ("random", 13, 3, 6),
+    # from 512 columns on: one, two and four rows, sixteen, eight and four waves
+    ("chain", 12, 6, 6), ("chain", 13, 6, 6), ("bath", 12, 6, 6), ("bath", 12, 7, 4), ("bath", 13, 6, 6),
+    ("bath", 14, 5, 6), ("random", 12, 5, 5), ("random", 12, 6, 1),
+    # from 2 048 columns on, where the general kernel has sixteen waves
+    ("chain", 14, 5, 1), ("chain", 14, 6, 2), ("chain", 14, 6, 3), ("chain", 14, 6, 4), ("bath", 14, 6, 2),
+    ("bath", 14, 6, 3), ("bath", 14, 6, 4), ("random", 14, 6, 2)])
+def test_short_rows_sum_as_the_general_kernels(kind, L, Nup, Ndw, row_order):
+    """The short-row product is the general row kernels', bit for bit, and so is
+    <x, y> from its partial sums: a Krylov run that ends on its lowest Ritz value
+    leaves a Green function that another order of the sums moves by up to 1e-5."""
+    wl = {"chain": lambda: W.hubbard_chain(L, U=4.0, mu=2.0), "bath": lambda: W.plaquette_bath(n_bath=L - 4),
+          "random": lambda: _random_workload(4, L)}[kind]()
+    sec = "R0:N%d:S%d" % (Nup + Ndw, Nup - Ndw)
+    H = []
+    for block in (0, 256 if math.comb(L, Nup) < 2048 else 1024):
+        qcm.set_global_parameterC("hv_row_order", row_order)
+        qcm.set_global_parameterC("hv_block", block)
+        try:
+            H.append(qcm.Hamiltonian(_instance(wl, sec), sec, "G"))
+        finally:
+            qcm.set_global_parameterC("hv_block", 0)
+            qcm.set_global_parameterC("hv_row_order", 1)
+    n = H[0].dim
+    x, y0 = np.random.default_rng(Nup + 20 * Ndw).normal(size=(2, n))
+    for beta in (0.0, -0.75):
+        out = []
+        for h in H:
+            h.set_variant(1)
+            dx, dy, dd = _Dev(n), _Dev(n), _Dev(1)
+            try:
+                dx.put(x)
+                dy.put(y0)
+                h.apply_dot_noalloc(dx.p, dy.p, dd.p, beta)
+                out.append([dy.get(), dd.get()])
+                h.apply_device(dx.p, dy.p, 0.0)  # without the dot product: other groups of rows
+                out[-1].append(dy.get())
+            finally:
+                for q in (dx, dy, dd):
+                    q.free()
+        for a, b in zip(*out):
+            assert np.array_equal(a, b), (beta, np.abs(a - b).max())
 
 
 def test_torus4x4_full_sector_hv_matches_oracle(oracle):
