@@ -228,10 +228,10 @@ void Surrogate::ensure_rows(int B) {
   dzT.alloc((size_t)(depth * width + n_out) * Bp);
   db.alloc((size_t)(depth * width + n_out) * nb);
   slab.alloc((size_t)rows_splits(B) * shape().nw);
-  part.alloc(1024);
   cap_rows = B;
 }
 
+// (loss is the caller's, part of ensure_batch among them: nothing here may move it)
 int Surrogate::rows_step(int B, const bf16_t *X, const float *T, const int *idx, float *loss, const MlpAdam *h) {
   ensure_rows(B);
   MlpRows P = rows_args(B, X, T, idx);

@@ -7,6 +7,8 @@ gradients 5e-3 relative per tensor, the loss 1e-4); against the unrounded
 FP64 network, to bfloat16 level (3e-2 / 6e-2).  One Adam step moves every
 parameter with a clear gradient by -lr sign(g), as the oracle's step does.
 Training lowers the loss of a smooth regression by more than 10x."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -140,3 +142,39 @@ def test_row_block_kernels_at_their_edges(n_in, n_out, width, depth, B):
     for (dW, db), (mW, mb) in zip(M.unflatten(g, n_in, n_out, width, depth), G_m):
         for a, m in ((dW, mW), (db, mb)):
             assert np.linalg.norm(a - m) <= (5e-3 if B >= 64 else 2e-2) * np.linalg.norm(m) + 1e-12
+
+
+def test_loss_from_a_second_thread():
+    """predict on one thread, then the first loss_grad and the first time() of
+    larger batches on another, both threads alive: the loss is that of a network
+    used on one thread, to the last bit.  (The loss partials' buffer belongs to
+    the stream that allocated it; a step that replaced it handed the kernel the
+    old one.)"""
+    n_in, n_out, width, depth = 12, 40, 64, 2
+    rng = np.random.default_rng(21)
+    x, t = rng.normal(size=(700, n_in)), rng.normal(size=(700, n_out))
+    nets = [_net(n_in, n_out, width, depth, seed=5)[0] for _ in range(2)]
+    want = [nets[0].loss_grad(x[:n], t[:n]) for n in (64, 700)]
+    got, first, done = [], threading.Event(), threading.Event()
+
+    def predicts():
+        nets[1].predict(x[:64])
+        first.set()
+        done.wait(60)
+
+    def learns():
+        first.wait(60)
+        for n in (64, 700):
+            got.append(nets[1].loss_grad(x[:n], t[:n]))
+        got.append(nets[1].time(900, 2))
+        done.set()
+
+    th = [threading.Thread(target=f) for f in (predicts, learns)]
+    for q in th:
+        q.start()
+    for q in th:
+        q.join(120)
+    assert len(got) == 3 and min(got[2]) > 0.0
+    for (loss, g), (loss_w, g_w) in zip(got, want):
+        assert loss == loss_w
+        assert np.array_equal(g, g_w)
