@@ -449,6 +449,40 @@ double Surrogate::loss_grad_host(int n, const double *x, const double *yv, doubl
   return loss;
 }
 
+namespace {
+// Device time of the steps of sampled epochs, without the shuffles and index
+// uploads between epochs.  One pair of events; a record costs 4 us of the
+// stream's time, so not every short epoch has one.
+struct EpochClock {
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  double ms = 0.0;
+  long steps = 0, pending = 0;
+  EpochClock() {
+    ED_HIP(hipEventCreate(&e0));
+    ED_HIP(hipEventCreate(&e1));
+  }
+  EpochClock(const EpochClock &) = delete;
+  ~EpochClock() {
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+  }
+  void wait() {
+    if (!pending) return;
+    ED_HIP(hipEventSynchronize(e1));
+    float t = 0.f;
+    ED_HIP(hipEventElapsedTime(&t, e0, e1));
+    ms += t;
+    steps += pending;
+    pending = 0;
+  }
+  void start() { ED_HIP(hipEventRecord(e0, stream())); }
+  void stop(long n) {
+    ED_HIP(hipEventRecord(e1, stream()));
+    pending = n;
+  }
+};
+}  // namespace
+
 std::vector<double> Surrogate::train(int n, const double *x, const double *yv, int epochs, int batch, uint64_t seed,
                                      double *ms_per_step) {
   if (n < 1 || epochs < 0 || batch < 1) fail(ED_ERR_INVALID, "surrogate: bad training arguments");
@@ -463,7 +497,7 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
   std::vector<int> idx(n);
   std::iota(idx.begin(), idx.end(), 0);
   std::mt19937_64 g(seed);
-  // the losses of up to 64 epochs (64 MB of partials) stay on the device before the host waits
+  // the losses of up to 64 epochs (64 MB of partials) stay on the device before the host reads them
   const size_t per_epoch = (size_t)std::max(steps, 1) * 1024;
   const int group = (int)std::max<size_t>(1, std::min<size_t>({64, (size_t)epochs, (size_t(16) << 20) / per_epoch}));
   DevBuf<int> didx(n);
@@ -471,18 +505,17 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
   std::vector<int> nbs((size_t)std::max(steps, 1) * group);
   std::vector<float> hp;
   std::vector<double> hist;
-  double ms_total = 0.0;
-  long nsteps = 0;
-  hipEvent_t e0, e1;
-  ED_HIP(hipEventCreate(&e0));
-  ED_HIP(hipEventCreate(&e1));
+  const int every = group;  // one sampled epoch per group
+  EpochClock clock;
   for (int ep0 = 0; ep0 < epochs; ep0 += group) {
     const int ne = std::min(group, epochs - ep0);
-    ED_HIP(hipEventRecord(e0, stream()));
     for (int ep = 0; ep < ne; ++ep) {
-      check_cancel();
       for (int i = n - 1; i > 0; --i) std::swap(idx[i], idx[(size_t)(g() % (uint64_t)(i + 1))]);
       didx.upload(idx);
+      const bool sample = (ep0 + ep) % every == 0;
+      if (sample) clock.wait();
+      check_cancel();
+      if (sample) clock.start();
       for (int s = 0; s < steps; ++s) {
         const int *bi = didx.p + (size_t)s * batch;
         float *lp = eparts.p + per_epoch * (size_t)ep + (size_t)s * 1024;
@@ -498,9 +531,8 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
         nb = backward(batch, lp);
         adam_step();
       }
+      if (sample) clock.stop(steps);
     }
-    ED_HIP(hipEventRecord(e1, stream()));
-    ED_HIP(hipEventSynchronize(e1));
     hp.resize(per_epoch * (size_t)ne);
     if (steps) eparts.download(hp.data(), per_epoch * (size_t)ne);
     for (int ep = 0; ep < ne; ++ep) {
@@ -509,14 +541,9 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
         sum += mlp_fold(hp.data() + per_epoch * (size_t)ep + (size_t)s * 1024, nbs[(size_t)ep * steps + s]) / batch;
       hist.push_back(steps ? sum / steps : 0.0);
     }
-    float ms = 0.f;
-    ED_HIP(hipEventElapsedTime(&ms, e0, e1));
-    ms_total += ms;
-    nsteps += (long)steps * ne;
   }
-  ED_HIP(hipEventDestroy(e0));
-  ED_HIP(hipEventDestroy(e1));
-  if (ms_per_step) *ms_per_step = nsteps ? ms_total / nsteps : 0.0;
+  clock.wait();
+  if (ms_per_step) *ms_per_step = clock.steps ? clock.ms / clock.steps : 0.0;
   return hist;
 }
 

@@ -178,3 +178,17 @@ def test_loss_from_a_second_thread():
     for (loss, g), (loss_w, g_w) in zip(got, want):
         assert loss == loss_w
         assert np.array_equal(g, g_w)
+
+
+def test_step_time_is_that_of_the_steps():
+    """train's ms per step is the device's: an epoch of one step on one eighth of
+    the rows' worth of shuffling costs as much per step as one without."""
+    n_in, n_out = 4, 8
+    rng = np.random.default_rng(23)
+    x, t = rng.normal(size=(30000, n_in)), rng.normal(size=(30000, n_out))
+    net = MLP(n_in, n_out, 64, 1, seed=2)
+    ms = []
+    for rows in (16384, 30000):  # both one step of 16 384 rows an epoch
+        net.train(x[:rows], t[:rows], epochs=2, batch=16384)
+        ms.append(min(net.train(x[:rows], t[:rows], epochs=64, batch=16384)[1] for _ in range(3)))
+    assert ms[1] < 1.5 * ms[0], ms
