@@ -450,9 +450,10 @@ double Surrogate::loss_grad_host(int n, const double *x, const double *yv, doubl
 }
 
 namespace {
-// Device time of the steps of sampled epochs, without the shuffles and index
-// uploads between epochs.  One pair of events; a record costs 4 us of the
-// stream's time, so not every short epoch has one.
+// Device time of the steps of sampled epochs (without the shuffles and index
+// uploads between epochs), and with it the bound on how far the host queues
+// ahead: a sample begins once the last one has run.  One pair of events; a
+// record costs 4 us of the stream's time, so not every short epoch has one.
 struct EpochClock {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   double ms = 0.0;
@@ -505,7 +506,9 @@ std::vector<double> Surrogate::train(int n, const double *x, const double *yv, i
   std::vector<int> nbs((size_t)std::max(steps, 1) * group);
   std::vector<float> hp;
   std::vector<double> hist;
-  const int every = group;  // one sampled epoch per group
+  // a sampled epoch every 32 steps: the host is at most 64 steps (or two epochs)
+  // ahead, and sees a cancellation within as many
+  const int every = std::max(1, 32 / std::max(steps, 1));
   EpochClock clock;
   for (int ep0 = 0; ep0 < epochs; ep0 += group) {
     const int ne = std::min(group, epochs - ep0);

@@ -8,6 +8,7 @@ FP64 network, to bfloat16 level (3e-2 / 6e-2).  One Adam step moves every
 parameter with a clear gradient by -lr sign(g), as the oracle's step does.
 Training lowers the loss of a smooth regression by more than 10x."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -178,6 +179,33 @@ def test_loss_from_a_second_thread():
     for (loss, g), (loss_w, g_w) in zip(got, want):
         assert loss == loss_w
         assert np.array_equal(g, g_w)
+
+
+def test_training_sees_a_cancellation():
+    """A cancellation that arrives when most of a run's steps have been executed
+    still ends it (the host does not queue the whole run and leave), and the
+    network goes on afterwards."""
+    n_in, n_out, batch = 12, 33, 2048
+    rng = np.random.default_rng(22)
+    x, t = rng.normal(size=(16 * batch, n_in)), rng.normal(size=(16 * batch, n_out))
+    net = MLP(n_in, n_out, 256, 8, seed=2)
+    net.train(x, t, epochs=1, batch=batch)
+    # 64 epochs of 16 steps; the steps alone take most of the time
+    _, ms = net.train(x, t, epochs=2, batch=batch)
+    w0 = net.get_weights()
+    t0 = time.perf_counter()
+    net.train(x, t, epochs=64, batch=batch)
+    wall = time.perf_counter() - t0
+    net.set_weights(w0)
+    timer = threading.Timer(wall - 0.35e-3 * 64 * 16 * ms, _lib.lib().ed_request_cancel)
+    timer.start()
+    try:
+        with pytest.raises(_lib.EDError, match="interrupted"):
+            net.train(x, t, epochs=64, batch=batch)
+    finally:
+        timer.join()
+    hist, _ = net.train(x, t, epochs=1, batch=batch)
+    assert np.isfinite(hist[0]) and np.all(np.isfinite(net.get_weights()))
 
 
 def test_step_time_is_that_of_the_steps():
