@@ -4,7 +4,7 @@
 // recurrence from LDS, so that a sweep over hundreds of parameter points x
 // sectors is a single launch.  Larger ("wide") items keep their vectors in
 // memory and advance in lockstep, two launches per Lanczos step for all items
-// of a shape.  The projected tridiagonal problem is solved on the device by
+// of a shape (ground states three).  The projected tridiagonal problem is solved on the device by
 // one wave per item; every reduction has a fixed order.
 #include "ed_batch.hpp"
 
@@ -685,6 +685,7 @@ constexpr double kRunning = -2.0;
 constexpr int kWideBlock = 256;
 constexpr int kXcd = 8;
 constexpr size_t kWideLdsMax = 144 * 1024;  // longest row staged in LDS
+constexpr size_t kTriLdsMax = 144 * 1024;   // largest tridiagonal in LDS (3 072 steps)
 
 // item and workgroup of a block (grid: kXcd * ceil(n / kXcd) * nwg blocks)
 __device__ __forceinline__ bool wide_place(int n, int nwg, int &item, int &w) {
@@ -937,31 +938,40 @@ __global__ __launch_bounds__(kWideBlock) void k_wide_gs_init(const WideItem *ite
 }
 
 // after step k: the Ritz pair of the (k + 1) x (k + 1) tridiagonal and the
-// stop rule of the ground state, one wave per item
+// stop rule of the ground state, one wave per item.  LDS: the tridiagonal in
+// LDS, since the Sturm counts and the inverse iteration walk it serially; else
+// (more steps than fit) on the item's own arrays.
+template <bool LDS>
 __global__ __launch_bounds__(kW) void k_wide_ritz(const WideItem *items, int nwg, int M, int k, int max_iter,
                                                   double accur) {
   extern __shared__ double smem[];
   __shared__ double s_lam, s_zl, s_hi;
   const WideItem it = items[blockIdx.x];
   if (it.sc[SC_N] != kRunning) return;
-  // the tridiagonal in LDS: the Sturm counts and the inverse iteration walk it serially
-  double *al = smem, *be = al + k + 1, *bb = be + k + 1, *z = bb + k + 1, *D = z + k + 1, *l = D + k + 1;
+  const size_t len = LDS ? (size_t)k + 1 : (size_t)M;
+  double *al = LDS ? smem : it.a;
+  double *be = al + len, *bb = be + len, *z = bb + len, *D = z + len, *l = D + len;
   double *be_g = it.a + M, *z_g = it.a + 3 * (size_t)M;
   const double beta = sqrt(wide_fold(it.part + nwg, nwg));
-  for (int i = threadIdx.x; i <= k; i += kW) {
-    const double bi = i < k ? be_g[i] : beta;
-    al[i] = it.a[i];
-    be[i] = bi;
-    bb[i] = bi * bi;
-  }
+  if (LDS)
+    for (int i = threadIdx.x; i <= k; i += kW) {
+      const double bi = i < k ? be_g[i] : beta;
+      al[i] = it.a[i];
+      be[i] = bi;
+      bb[i] = bi * bi;
+    }
+  else
+    for (int i = threadIdx.x; i < k; i += kW) bb[i] = be[i] * be[i];  // (the LDS form leaves none)
   if (threadIdx.x == 0) {
     be_g[k] = beta;
+    if (!LDS) bb[k] = beta * beta;
     s_hi = it.sc[SC_HI];
   }
   __syncthreads();
   tri_lowest_wave(k + 1, al, be, bb, &s_hi, z, D, l, &s_lam, &s_zl);
   __syncthreads();
-  for (int i = threadIdx.x; i <= k; i += kW) z_g[i] = z[i];
+  if (LDS)
+    for (int i = threadIdx.x; i <= k; i += kW) z_g[i] = z[i];
   if (threadIdx.x == 0) {
     it.sc[SC_HI] = s_hi;
     it.sc[SC_LAM] = s_lam;
@@ -1149,10 +1159,14 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
     wide_hv<1>(W, items, n, k, 0, 0.0, s);
     wide_upd(W, items, n, k, s);
     const size_t tri = (size_t)kTriArrays * (k + 1) * sizeof(double);
-    if (tri > 64 * 1024)
-      ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_wide_ritz),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri));
-    hipLaunchKernelGGL(k_wide_ritz, dim3(n), dim3(kW), tri, s, items, W.nwg, M, k, max_iter, accur);
+    if (tri <= kTriLdsMax) {
+      if (tri > 64 * 1024)
+        ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_wide_ritz<true>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri));
+      hipLaunchKernelGGL((k_wide_ritz<true>), dim3(n), dim3(kW), tri, s, items, W.nwg, M, k, max_iter, accur);
+    } else {
+      hipLaunchKernelGGL((k_wide_ritz<false>), dim3(n), dim3(kW), 0, s, items, W.nwg, M, k, max_iter, accur);
+    }
     // (k_wide_ritz ends every item by step max_iter)
     if ((k >= max_iter || (k + 1) % kWideCheck == 0) && !wide_running(items, n, count, s)) break;
   }

@@ -110,6 +110,31 @@ def test_ground_states_whose_krylov_space_ends_between_checks(L, N, S, dim):
     _compare(wl, [{"t": 1.0, "U": 4.0, "mu": 1.3}, {"t": 1.0, "U": 7.0, "mu": 2.2}], "F", W.matsubara(16, 20.0))
 
 
+def test_lockstep_ground_states_beyond_the_steps_that_fit_in_lds():
+    """3 100 Lanczos steps of a 4 900-state sector that may not converge (a stop
+    bar below zero): the tridiagonal outgrows LDS at step 3 072 and the run ends
+    as not converged at its own limit, with the batch usable afterwards."""
+    wl = W.hubbard_chain(8, U=4.0, mu=2.0)
+    name = _model(wl)
+    label = _new_label()
+    qcm.new_model_instanceC(name, wl.values, wl.sector, label)
+    try:
+        qcm.set_global_parameterC("max_iter_lanczos", 3100)
+        qcm.set_global_parameterC("accur_lanczos", -1.0)
+        with pytest.raises(_lib.EDError, match="exceeded 3100 iterations"):
+            qcm.solve_batch([label], green_function=False)
+    finally:
+        qcm.set_global_parameterC("max_iter_lanczos", 1000)
+        qcm.set_global_parameterC("accur_lanczos", 1e-12)
+    qcm.solve_batch([label], green_function=False)
+    E0 = qcm.ground_state_solve(label)[0]
+    qcm.erase_model_instance(label)
+    label = _new_label()
+    qcm.new_model_instanceC(name, wl.values, wl.sector, label)
+    assert abs(E0 - qcm.ground_state_solve(label)[0]) <= 1e-10 * abs(E0)
+    qcm.erase_model_instance(label)
+
+
 def test_batch_large_sector_four_wave_kernel():
     """A 10-site chain at half filling (dim 63 504; N +- 1 sectors 52 920) runs
     in the four-wave workgroup."""
