@@ -120,10 +120,11 @@ void wide_coefficients(const BatchGSItem &, double *tri, size_t M, WideItem &w) 
   w.b = tri + M - 1;
 }
 
-// execution class of an item: from LDS with one or four waves, with the other
-// items of its shape in lockstep, or (fractions) from registers
-enum Cls { kLds = 0, kLdsFour = 1, kWide = 2, kTile = 3 };
-constexpr int kLdsClasses = 2;
+// execution class of an item: from LDS with one or four waves, the same with a
+// ground state's tridiagonal arrays in memory, with the other items of its shape
+// in lockstep, or (fractions) from registers
+enum Cls { kLds = 0, kLdsFour = 1, kLdsTri = 2, kLdsTriFour = 3, kWide = 4, kTile = 5 };
+constexpr int kLdsClasses = 4;
 // Both halves up to two tiles of 16: the register kernel at any size (512
 // points of the 2x3 sweep, 225-400 states: 67 ms of LDS kernels -> 31 ms; 2x2
 // with 2 bath orbitals 34.3 -> 26.5 ms a whole sweep, with 1 23.6 -> 20.7; 24 -
@@ -159,9 +160,20 @@ Cls classify(size_t lds, uint32_t dim) {
   return kWide;
 }
 
+// A ground state: many steps allowed (max_iter_lanczos 5 000: 240 KB of
+// tridiagonal arrays) do not send a small sector to the lockstep kernels, whose
+// three launches a step are for sectors that fill them (512 points of 2x2, 16 to
+// 36 states: 4.4 ms, from LDS 2.4; of 2x3, 300 to 400 states: 23.0 and 9.5).
+Cls classify_gs(size_t lds, size_t lds_without_tri, uint32_t dim) {
+  const Cls c = classify(lds, dim);
+  if (c != kWide || lds_without_tri > kBatchLdsCap) return c;
+  return dim >= kFourWaveDim ? kLdsTriFour : kLdsTri;
+}
+
 // one launch per LDS class
 template <typename Item, typename Launch>
-void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls, size_t lds_max, Launch launch) {
+void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls, const size_t (&lds_max)[kLdsClasses / 2],
+                    Launch launch) {
   std::vector<Item> part[kLdsClasses];
   for (size_t k = 0; k < items.size(); ++k)
     if (cls[k] < kLdsClasses) part[cls[k]].push_back(items[k]);
@@ -169,7 +181,7 @@ void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls,
   for (int c = 0; c < kLdsClasses; ++c) {
     if (part[c].empty()) continue;
     d[c].upload(part[c]);
-    launch(d[c].p, (int)part[c].size(), c == kLdsFour ? 256 : 64, lds_max);
+    launch(d[c].p, (int)part[c].size(), c & 1 ? 256 : 64, lds_max[c / 2], c < kLdsTri);
   }
   sync();
 }
@@ -370,7 +382,7 @@ void append_pairs(std::vector<BatchCFItem> &items, MapCache &maps, int L, const 
 void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::vector<int> &tab, int max_cf,
                    double acc, DevBuf<double> &av, DevBuf<double> &bv, DevBuf<double> &out) {
   std::vector<Cls> cls(items.size());
-  size_t lds_max = 0;
+  size_t lds_max[2] = {0, 0};
   for (size_t k = 0; k < items.size(); ++k) {
     const TablePack::Off &o = tabs.offs[tab[k]];
     if (o.du <= kTileDim && o.dd <= kTileDim) {
@@ -380,7 +392,7 @@ void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::
     const size_t b = tabs.lds(tab[k], kCfVectors, 0);
     cls[k] = classify(b, tabs.offs[tab[k]].du * tabs.offs[tab[k]].dd);
     if (cls[k] == kWide) tabs.use_wide(tab[k]);
-    else lds_max = std::max(lds_max, b);
+    else lds_max[0] = std::max(lds_max[0], b);
   }
   tabs.upload();
   vlog("batch: %zu continued-fraction items, tables and maps built", items.size());
@@ -394,7 +406,7 @@ void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::
     it.b = bv.p + (size_t)(max_cf + 1) * k;
     it.out = out.p + 2 * k;
   }
-  launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds) {
+  launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds, bool) {
     batch_cf(d, n, block, lds, max_cf, acc, stream());
   });
   launch_tiles(tabs, items, cls, tab, max_cf, acc);
@@ -453,21 +465,27 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
     const size_t ntri = (size_t)kTriArrays * (max_iter + 2);
     std::vector<Cls> cls(refs.size());
     std::vector<int> tab(refs.size());
-    size_t lds_max = 0;
+    size_t lds_max[2] = {0, 0}, ntri_mem = 0;
     for (size_t k = 0; k < refs.size(); ++k) {
-      const size_t b = tabs.lds(refs[k].tab, kGsVectors, ntri);
-      cls[k] = classify(b, refs[k].dim);
+      const size_t b = tabs.lds(refs[k].tab, kGsVectors, ntri), b0 = tabs.lds(refs[k].tab, kGsVectors, 0);
+      cls[k] = classify_gs(b, b0, refs[k].dim);
       tab[k] = refs[k].tab;
-      if (cls[k] == kWide) tabs.use_wide(tab[k]);
-      else lds_max = std::max(lds_max, b);
+      if (cls[k] == kWide) {
+        tabs.use_wide(tab[k]);
+      } else if (cls[k] >= kLdsTri) {
+        lds_max[1] = std::max(lds_max[1], b0);
+        ++ntri_mem;
+      } else {
+        lds_max[0] = std::max(lds_max[0], b);
+      }
     }
     tabs.upload();
     vlog("batch: %zu ground-state tables built and uploaded", refs.size());
     // the ground states stay here; each state's vector is a view kept alive by it
     auto gsv = std::make_shared<DevBuf<double>>(std::max<size_t>(gs_len, 1));
-    DevBuf<double> out(std::max<size_t>(3 * refs.size(), 1));
+    DevBuf<double> out(std::max<size_t>(3 * refs.size(), 1)), tri(std::max<size_t>(ntri * ntri_mem, 1));
     std::vector<BatchGSItem> items(refs.size());
-    size_t go = 0;
+    size_t go = 0, to = 0;
     for (size_t k = 0; k < refs.size(); ++k) {
       BatchGSItem &it = items[k];
       it.S = tabs.view(refs[k].tab);
@@ -475,9 +493,10 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
       it.gs = gsv->p + go;
       it.out = out.p + 3 * k;
       go += refs[k].dim;
+      if (cls[k] == kLdsTri || cls[k] == kLdsTriFour) it.tri = tri.p + ntri * to++;
     }
-    launch_classes(items, cls, lds_max, [&](const BatchGSItem *d, int n, int block, size_t lds) {
-      batch_gs(d, n, block, lds, max_iter, accur, stream());
+    launch_classes(items, cls, lds_max, [&](const BatchGSItem *d, int n, int block, size_t lds, bool tri_lds) {
+      batch_gs(d, n, block, lds, tri_lds, max_iter, accur, stream());
     });
     launch_wide(tabs, items, cls, tab, 3, ntri, [&](const WideShape &W, const WideItem *w, const BatchGSItem *q, int n) {
       wide_gs(W, w, q, n, max_iter, accur, stream());

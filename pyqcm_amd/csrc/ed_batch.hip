@@ -296,7 +296,9 @@ __device__ __forceinline__ void tri_lowest_wave(int n, const double *a, const do
 }
 
 constexpr int kRitzEvery = 4;
-template <int BS>
+// TRI: the tridiagonal arrays in LDS too; else (more steps allowed than fit
+// beside the sector) the item's own in memory
+template <int BS, bool TRI>
 __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int max_iter, double accur) {
   extern __shared__ double smem[];
   __shared__ double sh[BS / kW];
@@ -306,9 +308,9 @@ __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int m
   const uint32_t dim = G.du * G.dd;
   const double rdu = 1.0 / (double)G.du;
   const int M = max_iter + 2;
-  double *v = smem, *vp = v + dim, *gs = vp + dim, *tri = gs + dim;
+  double *v = smem, *vp = v + dim, *gs = vp + dim, *tri = TRI ? gs + dim : it.tri;
   const uint32_t nu = G.up_ptr[G.du], nd = G.dn_ptr[G.dd];
-  double *sd = tri + (size_t)kTriArrays * M;
+  double *sd = gs + dim + (TRI ? (size_t)kTriArrays * M : 0);
   const BatchSector S = stage_sector<BS>(G, sd, reinterpret_cast<uint32_t *>(sd + dim + nu + nd));
   double *al = tri, *be = al + M, *bb = be + M, *z = bb + M, *D = z + M, *l = D + M;
   // start vector (the same draws as the single-sector path)
@@ -1053,13 +1055,20 @@ __global__ void k_cf_store(int nitems, int max_cf, const double *out, const doub
 
 }  // namespace
 
-void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, int max_iter, double accur, hipStream_t s) {
+void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, bool tri_lds, int max_iter, double accur,
+              hipStream_t s) {
   if (n <= 0) return;
   if (lds > kBatchLdsCap) fail(ED_ERR_INVALID, "batch_gs: LDS request above the cap");
-  if (block == 256)
-    hipLaunchKernelGGL((k_batch_gs<256>), dim3(n), dim3(256), lds, s, d_items, max_iter, accur);
-  else
-    hipLaunchKernelGGL((k_batch_gs<64>), dim3(n), dim3(64), lds, s, d_items, max_iter, accur);
+#define ED_GS(BS, TRI) \
+  hipLaunchKernelGGL((k_batch_gs<BS, TRI>), dim3(n), dim3(BS), lds, s, d_items, max_iter, accur)
+  if (block == 256) {
+    if (tri_lds) ED_GS(256, true);
+    else ED_GS(256, false);
+  } else {
+    if (tri_lds) ED_GS(64, true);
+    else ED_GS(64, false);
+  }
+#undef ED_GS
   ED_HIP(hipGetLastError());
 }
 

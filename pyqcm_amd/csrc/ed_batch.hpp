@@ -29,6 +29,7 @@ struct BatchGSItem {
   BatchSector S;
   uint64_t seed = 0;
   double *gs = nullptr;   // dim: normalized ground state (output)
+  double *tri = nullptr;  // kTriArrays (max_iter + 2), for items whose arrays are not in LDS
   double *out = nullptr;  // E0, iterations, status (0 ok, 1 not converged)
 };
 
@@ -101,7 +102,9 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
              hipStream_t s);
 
 // items run from LDS, lds dynamic bytes each; block: 64 or 256 threads per item
-void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, int max_iter, double accur, hipStream_t s);
+// (tri_lds: the tridiagonal arrays among them, else in each item's tri)
+void batch_gs(const BatchGSItem *d_items, int n, int block, size_t lds, bool tri_lds, int max_iter, double accur,
+              hipStream_t s);
 void batch_cf(const BatchCFItem *d_items, int n, int block, size_t lds, int max_cf, double acc, hipStream_t s);
 
 // fractions of sectors of at most 16 rt down and 16 ct up half states (rt, ct

@@ -135,6 +135,35 @@ def test_lockstep_ground_states_beyond_the_steps_that_fit_in_lds():
     qcm.erase_model_instance(label)
 
 
+@pytest.mark.parametrize("steps", [1350, 5000])
+def test_many_allowed_steps_change_nothing_in_small_sectors(steps):
+    """Ground states of small sectors with more Lanczos steps allowed than their
+    tridiagonal arrays fit beside them in LDS (1 350: in some sectors only): the
+    energies and ground states are those of the default, to the last bit."""
+    wl = W.vca_cluster(2, 2)
+    wl6 = dataclasses.replace(W.hubbard_chain(6, U=4.0, mu=1.3), sector="R0:N6:S0/R0:N5:S1/R0:N2:S0/R0:N1:S1")
+    out = []
+    try:
+        for n in (1000, steps):
+            qcm.set_global_parameterC("max_iter_lanczos", n)
+            got = []
+            for w, pts in ((wl, W.vca_points(6, seed=9)), (wl6, [{"t": 1.0, "U": u, "mu": 1.0} for u in (2.0, 8.0)])):
+                labels = [_new_label() for _ in pts]
+                for lab, vals in zip(labels, pts):
+                    qcm.new_model_instanceC(_model(w), vals, w.sector, lab)
+                qcm.set_global_parameterC("GF_method", "F")
+                qcm.solve_batch(labels, green_function=True)
+                got += [qcm.ground_state_solve(lab)[0] for lab in labels]
+                got += [qcm.Green_function_grid(W.matsubara(8, 20.0), label=lab) for lab in labels]
+                for lab in labels:
+                    qcm.erase_model_instance(lab)
+            out.append(got)
+    finally:
+        qcm.set_global_parameterC("max_iter_lanczos", 1000)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_batch_large_sector_four_wave_kernel():
     """A 10-site chain at half filling (dim 63 504; N +- 1 sectors 52 920) runs
     in the four-wave workgroup."""
