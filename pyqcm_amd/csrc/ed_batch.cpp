@@ -149,6 +149,9 @@ constexpr size_t kWideBytes = size_t(192) << 20;
 // from there on one product fills the chip and its tuned kernels win (+ 9
 // bath, 2.9 M states: 1.24 s against 1.81 together).
 constexpr size_t kTogetherDim = size_t(1) << 20;
+// The same for a single fraction a part (one orbital): 213 444 states 46 ms alone
+// against 35 here, 731 808 states 24.9 against 26.1; three of them 75 and 45.
+constexpr size_t kAloneDim = size_t(1) << 19;
 
 // LDS decides between one workgroup an item and lockstep: a workgroup with
 // vectors in memory, the only other way to keep an item by itself, took 1.3 to
@@ -627,14 +630,15 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
   vlog("batch: continued fractions stored");
 }
 
-bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin) {
+bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin, size_t npairs) {
   Params &P = params();
   if ((I.format != 'G' && I.format != 'F') || P.geti("lanczos_block") == 0 || P.getb("lanczos_reorth") ||
       P.geti("max_iter_CF") <= 0 || !terms_factorizable(T))
     return false;
+  const size_t limit = npairs > 1 ? kTogetherDim : kAloneDim;
   for (int pm = -1; pm <= 1; pm += 2) {
     const Sector tgt = shift_sector(st.sec, pm, spin);
-    if (sector_valid(I.model->L, tgt) && sector_dim(I.model->L, tgt) > kTogetherDim) return false;
+    if (sector_valid(I.model->L, tgt) && sector_dim(I.model->L, tgt) > limit) return false;
   }
   return true;
 }

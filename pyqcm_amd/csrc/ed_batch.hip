@@ -677,8 +677,8 @@ __global__ __launch_bounds__(kW) void k_tile_cf(const BatchCFItem *items, int ma
 // all take the same branch when the stop rule ends the item; workgroup 0
 // stores the scalars, which other workgroups read from the next launch on.
 // Memory bound: 6 vector accesses a step plus the neighbour rows, which hit
-// the XCD's L2 because an item's workgroups are numbered onto one XCD
-// (block b runs on XCD b % 8).  Rows of U_k are staged in LDS for the lane
+// the XCD's L2 because an item's workgroups are numbered onto one XCD or a run
+// of them (wide_place).  Rows of U_k are staged in LDS for the lane
 // part; a lane's table entries are loaded once for RPT rows, since they are
 // 12 bytes a hop against 8 of the vector.
 // ---------------------------------------------------------------------------
@@ -686,14 +686,32 @@ enum { SC_N = 0, SC_NN = 1, SC_PROD = 2 /* two, by parity */, SC_HI = 4, SC_LAM 
 constexpr double kRunning = -2.0;
 constexpr int kWideBlock = 256;
 constexpr int kXcd = 8;
+constexpr size_t kWideSpread = size_t(1) << 17;
 constexpr size_t kWideLdsMax = 144 * 1024;  // longest row staged in LDS
 constexpr size_t kTriLdsMax = 144 * 1024;   // largest tridiagonal in LDS (3 072 steps)
 
-// item and workgroup of a block (grid: kXcd * ceil(n / kXcd) * nwg blocks)
-__device__ __forceinline__ bool wide_place(int n, int nwg, int &item, int &w) {
+// Item and workgroup of a block.  Block b runs on XCD b % 8.  Items are dealt out
+// to the XCDs whole (grid: kXcd * ceil(n / kXcd) * nwg blocks), so that what one
+// launch writes the next finds in its own L2, or (kWideSpread states or more, nwg
+// negated) XCD x takes the x-th run of all items' workgroups (kXcd * ceil(n nwg /
+// kXcd) blocks), so that fewer than 8 items, or 9, fill the chip too.  ms of a
+// Green function, whole / in runs / one fraction after the other:
+//   3 920 states    1 fraction a part  4.8 /  5.4 /  17    10 fractions   5.0 /  5.5 / 180
+//   15 876          1                 17.6 / 20.5 /  39     6            19.9 / 22.7 / 250
+//   52 920          1                  6.5 /  6.2 /  21    10            10.1 / 10.7 / 228
+//   213 444         1                 47   / 35   /  46     6            52.9 / 47.4 / 295
+//   731 808         1                 44.9 / 26.1 /  24.9  10           150   / 108  / 252
+__device__ __forceinline__ bool wide_place(int n, int &nwg, int &item, int &w) {
   const int b = blockIdx.x, j = b / kXcd;
-  item = (j / nwg) * kXcd + b % kXcd;
-  w = j % nwg;
+  if (nwg < 0) {
+    nwg = -nwg;
+    const int t = (int)(b % kXcd * (gridDim.x / kXcd)) + j;
+    item = t / nwg;
+    w = t - item * nwg;
+  } else {
+    item = (j / nwg) * kXcd + b % kXcd;
+    w = j % nwg;
+  }
   return item < n;
 }
 
@@ -1104,7 +1122,13 @@ WideShape wide_shape(uint32_t du, uint32_t dd, uint32_t emax) {
 }
 
 namespace {
-unsigned wide_grid(const WideShape &W, int n) { return (unsigned)(kXcd * ((n + kXcd - 1) / kXcd) * W.nwg); }
+bool wide_spread(const WideShape &W) { return (size_t)W.nl * W.nr >= kWideSpread; }
+// the kernels' nwg (negated: workgroups in runs, see wide_place) and their grid
+int wide_nwg(const WideShape &W) { return wide_spread(W) ? -W.nwg : W.nwg; }
+unsigned wide_grid(const WideShape &W, int n) {
+  if (wide_spread(W)) return (unsigned)(((size_t)n * W.nwg + kXcd - 1) / kXcd * kXcd);
+  return (unsigned)(kXcd * ((n + kXcd - 1) / kXcd) * W.nwg);
+}
 
 template <int MODE>
 void wide_hv(const WideShape &W, const WideItem *items, int n, int k, int max_k, double acc, hipStream_t s) {
@@ -1115,7 +1139,7 @@ void wide_hv(const WideShape &W, const WideItem *items, int n, int k, int max_k,
       ED_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_wide_hv<MODE, RPT, RG1, STG>),                  \
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)W.lds));                        \
     hipLaunchKernelGGL((k_wide_hv<MODE, RPT, RG1, STG>), dim3(wide_grid(W, n)), dim3(kWideBlock), W.lds, s,       \
-                       items, n, W.nwg, W.nl, W.nr, rg, W.emax, k, max_k, acc);                                          \
+                       items, n, wide_nwg(W), W.nl, W.nr, rg, W.emax, k, max_k, acc);                            \
   } while (0)
   if (!W.stage) ED_WIDE(1, true, false);
   else if (rg > 1) ED_WIDE(2, false, true);
@@ -1126,7 +1150,7 @@ void wide_hv(const WideShape &W, const WideItem *items, int n, int k, int max_k,
 }
 
 void wide_upd(const WideShape &W, const WideItem *items, int n, int k, hipStream_t s) {
-  hipLaunchKernelGGL(k_wide_upd, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, n, W.nwg,
+  hipLaunchKernelGGL(k_wide_upd, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, n, wide_nwg(W),
                      (size_t)W.nl * W.nr, k);
 }
 
@@ -1144,7 +1168,7 @@ void wide_cf(const WideShape &W, const WideItem *items, const BatchCFItem *src, 
              hipStream_t s) {
   if (n <= 0) return;
   DevBuf<int> count(1);
-  hipLaunchKernelGGL(k_wide_cf_init, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr,
+  hipLaunchKernelGGL(k_wide_cf_init, dim3(wide_grid(W, n)), dim3(kWideBlock), 0, s, items, src, n, wide_nwg(W), W.nl, W.nr,
                      W.swap);
   for (int k = 0; k <= max_cf; ++k) {
     wide_hv<0>(W, items, n, k, max_cf, acc, s);  // k == max_cf only ends the items
@@ -1162,7 +1186,7 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
   DevBuf<int> count(1);
   const int M = max_iter + 2;
   const unsigned g = wide_grid(W, n);
-  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap, M, 0);
+  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, wide_nwg(W), W.nl, W.nr, W.swap, M, 0);
   int k = 0;
   for (;; ++k) {
     wide_hv<1>(W, items, n, k, 0, 0.0, s);
@@ -1179,10 +1203,10 @@ void wide_gs(const WideShape &W, const WideItem *items, const BatchGSItem *src, 
     // (k_wide_ritz ends every item by step max_iter)
     if ((k >= max_iter || (k + 1) % kWideCheck == 0) && !wide_running(items, n, count, s)) break;
   }
-  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap, M, 1);
+  hipLaunchKernelGGL(k_wide_gs_init, dim3(g), dim3(kWideBlock), 0, s, items, src, n, wide_nwg(W), W.nl, W.nr, W.swap, M, 1);
   for (int j = 1; j <= k; ++j) wide_hv<2>(W, items, n, j, M, 0.0, s);
   for (int scale = 0; scale < 2; ++scale)
-    hipLaunchKernelGGL(k_wide_gs_out, dim3(g), dim3(kWideBlock), 0, s, items, src, n, W.nwg, W.nl, W.nr, W.swap,
+    hipLaunchKernelGGL(k_wide_gs_out, dim3(g), dim3(kWideBlock), 0, s, items, src, n, wide_nwg(W), W.nl, W.nr, W.swap,
                        scale);
   ED_HIP(hipGetLastError());
 }
