@@ -152,6 +152,9 @@ constexpr size_t kTogetherDim = size_t(1) << 20;
 // The same for a single fraction a part (one orbital): 213 444 states 46 ms alone
 // against 35 here, 731 808 states 24.9 against 26.1; three of them 75 and 45.
 constexpr size_t kAloneDim = size_t(1) << 19;
+// Room for the levels that the fractions of a part may have (each 32 bytes, both
+// parts): a level limit meant as none would ask for it at once.
+constexpr size_t kTogetherLevels = size_t(1) << 22;
 
 // LDS decides between one workgroup an item and lockstep: a workgroup with
 // vectors in memory, the only other way to keep an item by itself, took 1.3 to
@@ -630,10 +633,10 @@ void solve_batch(const std::vector<Instance *> &insts, bool want_gf) {
   vlog("batch: continued fractions stored");
 }
 
-bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin, size_t npairs) {
+bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin, size_t npairs, long max_cf) {
   Params &P = params();
   if ((I.format != 'G' && I.format != 'F') || P.geti("lanczos_block") == 0 || P.getb("lanczos_reorth") ||
-      P.geti("max_iter_CF") <= 0 || !terms_factorizable(T))
+      max_cf <= 0 || (size_t)max_cf > kTogetherLevels / std::max<size_t>(npairs, 1) || !terms_factorizable(T))
     return false;
   const size_t limit = npairs > 1 ? kTogetherDim : kAloneDim;
   for (int pm = -1; pm <= 1; pm += 2) {

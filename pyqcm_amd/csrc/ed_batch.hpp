@@ -131,9 +131,10 @@ struct Fraction {
 };
 struct State;
 struct TermList;
-// whether an instance's fractions of npairs orbital pairs from state st run as a
-// batch (the same recurrence and stop rule as lanczos_green, all pairs together)
-bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin, size_t npairs);
+// whether an instance's fractions of npairs orbital pairs from state st, at most
+// max_cf levels each, run as a batch (the same recurrence and stop rule as
+// lanczos_green, all pairs together)
+bool fractions_together(const Instance &I, const TermList &T, const State &st, int spin, size_t npairs, long max_cf);
 // the fractions of c^{pm}_o1 (+ c^{pm}_o2) |st> for the given pairs, at most
 // max_cf levels: entry 2 k + (pm < 0) for pair k; the hole and the electron
 // part run together.  Empty where the target sector is invalid or empty.

@@ -1084,7 +1084,7 @@ static void build_gf(Instance &I, State &st, int spin) {
     ee.swap(e.first);
     Ve.swap(e.second);
   }
-  if (G.kind == 'F' && fractions_together(I, T, st, spin, np)) {
+  if (G.kind == 'F' && fractions_together(I, T, st, spin, np, params().geti("max_iter_CF"))) {
     // build_cf (src_ed/model_instance.cpp:35-100) for all pairs at once
     check_cancel();
     std::vector<std::pair<int, int>> pairs;
@@ -1266,7 +1266,7 @@ void cf_pairs(Instance &I, int spin, const std::vector<std::pair<int, int>> &pai
   const TermList T = I.terms();
   a.assign(2 * pairs.size(), {});
   b.assign(2 * pairs.size(), {});
-  if (cap > 0 && fractions_together(I, T, st, sp, pairs.size())) {
+  if (fractions_together(I, T, st, sp, pairs.size(), cap)) {
     check_cancel();
     std::vector<Fraction> fr = state_fractions(I, T, st, sp, pairs, cap);
     for (size_t k = 0; k < fr.size(); ++k) {

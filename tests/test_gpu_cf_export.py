@@ -47,3 +47,26 @@ def test_export_import_round_trip(oracle):
     assert np.abs(b[0, :m] - br[:m]).max() < 1e-9
     qcm.erase_model_instance(9701)
     qcm.erase_model_instance(9702)
+
+
+def test_a_level_limit_meant_as_none():
+    """max_iter_CF far above the levels that the stop rule allows: the fractions
+    are those of the default limit (nothing is sized by the limit)."""
+    wl = W.hubbard_chain(4, U=4.0, mu=2.0)
+    name = W.setup(wl, label=9703, model_name="cfx_limit4")
+    z = W.matsubara(64, 20.0)
+    G = []
+    try:
+        for label, limit in ((9703, 400), (9704, 2000000000)):
+            qcm.set_global_parameterC("max_iter_CF", limit)
+            if label != 9703:
+                qcm.new_model_instanceC(name, dict(wl.values), wl.sector, label)
+            qcm.ground_state_solve(label)
+            qcm.Green_function_solveC(label)
+            assert qcm.continued_fractions(label, 0)[2].max() < 400
+            G.append(qcm.Green_function_grid(z, 0, label))
+    finally:
+        qcm.set_global_parameterC("max_iter_CF", 400)
+    assert np.abs(G[0] - G[1]).max() < 1e-12
+    qcm.erase_model_instance(9703)
+    qcm.erase_model_instance(9704)
