@@ -215,10 +215,12 @@ __global__ __launch_bounds__(64) void k_lattice_reg(Arg A, int nz, int zc, const
           }
         }
         if (MODE == 0) {
-          prod *= q2;
           // the product of the squared pivots is kept within range
-          if (!(prod < 1e100 && prod > 1e-100)) {
-            logdet += log(prod);
+          const double p2 = prod * q2;
+          if (p2 < 1e100 && p2 > 1e-100) {
+            prod = p2;
+          } else {
+            logdet += log(prod) + log(q2);
             prod = 1.0;
           }
           if (c == D - 1) break;

@@ -241,3 +241,26 @@ def test_lattice_sums_for_every_matrix_size(d, kgrid, nz):
         _, per = qcm.SEF_grid(w, np.ones(nz), sl, kgrid, sl, lab)
         refl = LR.sef_logdet(Gs[0], sl, kgrid) + LR.sef_logdet(Gs[1], sl, kgrid)
         assert np.abs(per - refl).max() < 1e-11 * max(1.0, np.abs(refl).max())
+
+
+@pytest.mark.parametrize("d", [2, 3, 6])
+def test_log_determinants_of_far_apart_pivots(d):
+    """Pivots of 1e45 and 1e125 (squared 1e90 and 1e250: their product is beyond
+    a double, their logarithms are not) in either order: numpy's slogdet of the
+    same matrices, whose rows are scaled to 1 first."""
+    ops = {"t": ("one-body", [(i, i + 1, -1.0) for i in range(d - 1)] + [(i + d, i + d + 1, -1.0) for i in range(d - 1)]),
+           "U": ("interaction", [(i, i + d, 1.0) for i in range(d)]),
+           "mu": ("one-body", [(a, a, -1.0) for a in range(2 * d)])}
+    lab = _instance("latfar%d" % d, d, 0, ops, {"t": 1.0, "U": 3.0, "mu": 0.2}, "R0:N1:S1")
+    w = np.linspace(0.2, 5.0, 7)
+    G = [_natural(qcm.Green_function_grid(1j * w, spin_down=s, label=lab)) for s in (0, 1)]
+    for order in (1, -1):
+        s = np.array(([1e45, 1e125] + [1.0] * (d - 2))[::order])
+        sl = {"V0": np.diag(s).astype(complex), "elements": [], "R": np.array([[1.0, 0, 0]])}
+        _, per = qcm.SEF_grid(w, np.ones(len(w)), sl, (1, (3, 1, 1), 0.0), sl, lab)
+        ref = np.zeros(len(w))
+        for g in G:
+            M = np.einsum("a,zab->zab", s / np.maximum(s, 1.0), g) - np.diag(1.0 / np.maximum(s, 1.0))
+            ref += np.linalg.slogdet(M)[1] + np.log(np.maximum(s, 1.0)).sum()
+        assert np.all(np.isfinite(per))
+        assert np.abs(per - ref).max() < 1e-11 * np.abs(ref).max()
