@@ -1,7 +1,9 @@
-"""Batched solves (one workgroup per sector or per continued fraction) against
-the per-instance path on the same parameters and against dense
-diagonalization.  Bars: E0 1e-10 relative; G(z) 1e-8 on a Matsubara grid,
-both spin blocks."""
+"""Batched solves against the per-instance path on the same parameters and
+against dense diagonalization.  Bars: E0 1e-10 relative; G(z) 1e-8 on a
+Matsubara grid, both spin blocks.  An instance's own continued fractions run
+through the batch kernels too, so the reference instances are solved with
+lanczos_block 0: the host-driven recurrence, one fraction at a time, on the
+sector's own product."""
 import dataclasses
 import math
 
@@ -60,9 +62,13 @@ def _compare(wl, points, gf_method, z, dense=True):
         qcm.new_model_instanceC(name, vals, wl.sector, lb)
         single.append(la)
         batch.append(lb)
-    for la in single:
-        qcm.ground_state_solve(la)
-        qcm.Green_function_solveC(la)
+    try:
+        qcm.set_global_parameterC("lanczos_block", 0 if gf_method == "F" else 12)
+        for la in single:
+            qcm.ground_state_solve(la)
+            qcm.Green_function_solveC(la)
+    finally:
+        qcm.set_global_parameterC("lanczos_block", 12)
     qcm.solve_batch(batch, green_function=True)
     for vals, la, lb in zip(points, single, batch):
         Ea, sa = qcm.ground_state_solve(la)
@@ -165,8 +171,8 @@ def test_many_allowed_steps_change_nothing_in_small_sectors(steps):
 
 
 def test_batch_large_sector_four_wave_kernel():
-    """A 10-site chain at half filling (dim 63 504; N +- 1 sectors 52 920) runs
-    in the four-wave workgroup."""
+    """A 10-site chain at half filling (dim 63 504; N +- 1 sectors 52 920): all
+    items advance in lockstep, four rows of 252 to 210 states a thread."""
     wl = W.hubbard_chain(10, U=4.0, mu=2.0)
     _compare(wl, [{"t": 1.0, "U": 4.0, "mu": 2.0}, {"t": 1.0, "U": 6.0, "mu": 3.1}], "F", W.matsubara(16, 20.0),
              dense=False)
@@ -175,8 +181,8 @@ def test_batch_large_sector_four_wave_kernel():
 def test_batch_48400_state_sector_global_memory(oracle):
     """The 2x3 cluster with 6 bath orbitals at N = 6 (220 x 220 = 48 400
     states; the fractions run in the N +- 1 sectors of 14 520 and 108 900
-    states): every item goes through the global-memory workgroups.  E0 against
-    the oracle's Lanczos, E0 and G against the per-instance path."""
+    states): every item advances in lockstep with its vectors in memory.  E0
+    against the oracle's Lanczos, E0 and G against the per-instance path."""
     wl = W.vca_cluster_bath(2, 3, 6)
     pts = [{**wl.values, **v} for v in W.vca_points(2, seed=4)]   # bath values kept
     _compare(wl, pts, "F", W.matsubara(16, 20.0), dense=False)
@@ -227,15 +233,19 @@ def test_batch_mixed_formats_and_empty():
 
 @pytest.mark.parametrize("nx,ny,nb,N,S,npts", [(2, 2, 4, 8, 0, 1), (2, 2, 4, 7, -1, 5), (2, 2, 5, 8, 0, 2),
                                                (2, 3, 4, 6, 0, 2), (2, 2, 8, 4, 0, 3), (2, 2, 8, 6, 0, 1),
-                                               (2, 1, 16, 8, 8, 1)])
+                                               (2, 1, 12, 7, 5, 1), (2, 1, 12, 7, -5, 2), (2, 1, 14, 7, 5, 1),
+                                               (2, 1, 14, 7, -5, 1), (2, 1, 16, 8, 8, 1), (2, 1, 16, 8, -8, 1)])
 def test_items_beyond_lds_match_single_solves(nx, ny, nb, N, S, npts):
     """Sectors too large for LDS advance in lockstep: shapes with several rows
-    per workgroup pass (larger half basis up to 128 states), with one, and with
-    the spin-down half the larger (N odd or the fractions' targets), one item
-    and several per shape, ragged row counts.  Against the instance's own
-    solve: E0 to 1e-11 relative, G on the Matsubara axis to 1e-8 (the fractions
-    are 400 steps without reorthogonalization, which drift apart on the real
-    axis only)."""
+    side by side (larger half basis up to 128 states), with four, two and one
+    rows a thread (up to 2 048, 4 096 and 18 432 states) and with rows beyond
+    LDS (43 758), each with either spin the larger half; one item and several
+    per shape, ragged row counts, sectors on both sides of the 131 072 states
+    from which items are spread over the XCDs.  Against the instance's own
+    solve with lanczos_block 0 (the host-driven recurrence on the row product):
+    E0 to 1e-11 relative, G on the Matsubara axis to 1e-8 (the fractions are 400
+    steps without reorthogonalization, which drift apart on the real axis
+    only)."""
     wl = W.vca_cluster_bath(nx, ny, nb, N=N)
     sector = "R0:N%d:S%d" % (N, S)
     name = "wide_%d%d%d_%d" % (nx, ny, nb, N)
@@ -255,13 +265,17 @@ def test_items_beyond_lds_match_single_solves(nx, ny, nb, N, S, npts):
             E = qcm.ground_state_solve(lab)[0]
             G = [qcm.Green_function_grid(z, s, lab) for s in (0, 1)]
             qcm.new_model_instanceC(name, v, sector, lab + 500)
+            qcm.set_global_parameterC("lanczos_block", 0)
             E1 = qcm.ground_state_solve(lab + 500)[0]
+            qcm.Green_function_solveC(lab + 500)
+            qcm.set_global_parameterC("lanczos_block", 12)
             assert abs(E - E1) < 1e-11 * abs(E1)
             for s in (0, 1):
                 assert np.abs(G[s] - qcm.Green_function_grid(z, s, lab + 500)).max() < 1e-8
             qcm.erase_model_instance(lab)
             qcm.erase_model_instance(lab + 500)
     finally:
+        qcm.set_global_parameterC("lanczos_block", 12)
         qcm.set_global_parameterC("GF_method", "L")
         qcm.set_global_parameterC("hv_variant", 0)
 
