@@ -1641,29 +1641,35 @@ static size_t short_row_lds(const FactArgs &a, uint32_t rows) {
 
 // The short-row kernel's schedule: rpt rows per thread (0: the general row
 // kernels), ng rows side by side per workgroup.
-// The rows that the fullest CU works on, each at the cost of a row among 1, 2
-// or 4: where the up table is heavy (20 bytes or more per state) the shared
-// read of it makes the rows of a larger group cheaper, with a light one it
-// does not.  us of one product, general kernels -> this one (clusters: open
-// chains, plaquette + bath, periodic 4 x 3 and 4 x 4):
-//   heavy  924^2 plaquette (4 rows) 19.8 -> 14.5, periodic 18.3 -> 16.7; 1716^2 (4)
-//          57 -> 43; 1820^2 periodic (4) 58 -> 49; 3432^2 (4) 217 -> 169; 364
-//          columns of 3432 rows (2) 40 -> 23
-//   light  70^2 (1) 8.9 -> 4.3, 252^2 (1) 14.5 -> 4.6, 1287^2 (1) 23.0 -> 22.2,
-//          1716^2 (1) 43 -> 35, 3003^2 (1) 118 -> 97
-// With light tables 2 or 4 rows lose (1287^2: 27 and 30 us), with heavy ones 1
-// row does (924^2: 20 us), and 1 row in four waves is the general kernel over
-// again, a little slower (560^2 periodic 8.6 -> 9.0, 715^2 plaquette 12.0 -> 12.5):
-// those stay general.  From kShortRow states on a row is long enough to keep a
-// workgroup of 16 waves busy by itself, and the rows in flight no longer fit the
-// XCD's L2: 6435 x 5005 0.65 ms general, 0.77 here; 12870^2 3.8 and 5.6.  Rows of
-// more than 64 neighbours, and blocks asked for by size, stay general, as do
-// sectors whose general kernels walk more rows than they have partials.
+//
+// One row where the up table is light (under 20 bytes per state).  us of one
+// product, general kernels -> this one (open chains): 70^2 8.9 -> 4.3, 252^2 14.5
+// -> 4.6, 924^2 15.7 -> 13.5, 1716^2 43 -> 34, 3003^2 118 -> 97; 2 or 4 rows lose
+// (1287^2: 23.0 general, 22.2, 27 and 30).  From 1 025 to 1 536 rows the general
+// kernel has all its rows on the chip at once too, and its deeper table reads win
+// with a cold table (1716 x 1287, whole call: 39.7 us general, 40.5 here).
+//
+// Where it is heavy the shared read of it makes the rows of a larger group cheaper:
+// the fullest CU's rows, in whole rounds of the workgroups that fit, each at the
+// cost of a row among 1, 2 or 4, against the general kernel's rows (clusters:
+// plaquette + bath, periodic 4 x 3 and 4 x 4): 924^2 plaquette (4 rows) 19.8 ->
+// 14.5, periodic 18.7 -> 17.2; 1716^2 (4) 57 -> 43; 1820^2 periodic (4) 58 -> 49;
+// 3432^2 (4) 217 -> 169; 364 columns of 3432 rows (4) 40 -> 23.  1 row in four
+// waves is the general kernel over again (560^2 8.6 -> 9.0), as are nearly 2 rows
+// (1287^2, whole call: 43.7 general, 44.3), and a last round of few workgroups
+// costs what they gain (1820 x 4368 periodic, 4 rows, whole call: 144 and 150).
+//
+// From kShortRow states on a row is long enough to keep a workgroup of 16 waves
+// busy by itself, and the rows in flight no longer fit the XCD's L2: 6435 x 5005
+// 0.65 ms general, 0.77 here; 12870^2 3.8 and 5.6.  Rows of more than 64
+// neighbours, and blocks asked for by size, stay general, as do sectors whose
+// general kernels walk more rows than they have partials.
+//
 // With partials (dot) rows below 512 states take the general kernel's R rows per
 // workgroup, one per thread, since each such group has one partial; and a chain
 // that passes between waves costs most where workgroups follow one another on a
-// CU, so that 4 rows are left to sectors whose workgroups run at once (1820 x 4368
-// periodic, with the fold: general 149 us, 4 rows 167, 2 rows 141; 1716^2, which
+// CU, so that 4 rows are left to sectors whose workgroups run at once (1820 x 8008
+// periodic, with the fold: general 276 us, 4 rows 282, 2 rows 262; 1716^2, which
 // runs at once: 73 and 63).
 struct ShortRows {
   int rpt = 0;
@@ -1671,27 +1677,35 @@ struct ShortRows {
 };
 static ShortRows short_row_plan(const FactArgs &a, bool dot) {
   ShortRows S;
-  const uint32_t R = rows_per_block(a.up.dim);
+  const uint32_t R = rows_per_block(a.up.dim), dd = a.dn.dim;
   if (a.block != 0 || a.up.dim >= kShortRow || R == 0 || a.up.sell[0].nslice == 0 || a.up.sell[1].nslice == 0 ||
-      a.dn.maxrow > 64 || (a.dn.dim + R - 1) / R > (uint32_t)kPartialsCap)
+      a.dn.maxrow > 64 || (dd + R - 1) / R > (uint32_t)kPartialsCap)
     return S;
   const size_t entry = a.up.mode16 ? 2 : (a.up.packed ? 4 : 12);
-  const bool heavy = a.up.nnz * entry >= 20 * (size_t)a.up.dim, fixed = dot && R > 1;
-  const double cost[3] = {1.0, heavy ? 0.93 : 1.0, heavy ? 0.8 : 1.0};
-  double least = 0.0;
+  const bool heavy = a.up.nnz * entry >= 20 * (size_t)a.up.dim;
+  if (dot && R > 1) {
+    S.rpt = short_row_lds(a, R) <= kShortRowLds ? 1 : 0;
+    S.ng = R;
+    return S;
+  }
+  if (!heavy) {
+    S.rpt = (R == 1 && dd > 1024 && dd <= 1536) || short_row_lds(a, 1) > kShortRowLds ? 0 : 1;
+    return S;
+  }
+  // the general kernel's cost (rows below 512 states, or up to two a CU: never)
+  double least = R > 1 || dd <= 512 ? 1e30 : (double)((dd + 255) / 256);
   for (int k = 0; k < 3; ++k) {
-    const uint32_t rpt = 1u << k, nb = (a.dn.dim + rpt - 1) / rpt;
-    const size_t lds = short_row_lds(a, fixed ? R : rpt);
-    if ((fixed && k > 0) || lds > kShortRowLds) continue;
-    if (dot && R == 1 && a.up.dim < 2048 && nb > 512 && kShortRowLds / lds == 2) continue;
-    const double t = cost[k] * (double)rpt * ((nb + 255) / 256);
-    if (!S.rpt || t < least) {
+    const uint32_t rpt = 1u << k, nb = (dd + rpt - 1) / rpt, cu = (nb + 255) / 256;
+    const size_t lds = short_row_lds(a, rpt);
+    if (lds > kShortRowLds || (dot && a.up.dim < 2048 && nb > 512 && kShortRowLds / lds == 2)) continue;
+    const uint32_t fit = (uint32_t)std::min<size_t>(std::min<uint32_t>(cu, 8), kShortRowLds / lds);
+    const double cost = k == 0 ? 1.05 : (k == 2 ? 0.8 : (R == 1 && cu > 2 && !dot ? 1.05 : 0.93));
+    const double t = cost * (double)rpt * ((cu + fit - 1) / fit * fit);
+    if (t < least) {
       S.rpt = (int)rpt;
-      S.ng = fixed ? R : 1;
       least = t;
     }
   }
-  if (heavy && R == 1 && S.rpt == 1 && a.dn.dim > 512) S.rpt = 0;
   return S;
 }
 
