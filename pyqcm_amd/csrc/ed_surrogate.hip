@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void k_gather(int n, int ld, const int *idx, c
 // ---------------------------------------------------------------------------
 // Row-block kernels (widths 64, 128, 256).  A layer at a batch of 2 048 is 0.3
 // GFLOP, a fraction of a microsecond of matrix-core time, so separate GEMM,
-// loss, column-sum and optimizer launches were all launch and load latency (30
+// loss, column-sum and optimizer launches were all launch and load latency (42
 // launches, 290 us a step).  Rows of the batch are independent through the
 // forward pass, the loss and the input gradients: k_mlp_rows takes 16 of them
 // through all layers and back with activations, pre-activations (fp32) and
@@ -225,7 +225,7 @@ constexpr int kRows = 16, kRowThreads = 1024, kRowWaves = kRowThreads / 64;
 // KS k-steps of one weight row per lane (w: the lane's row at its 8-element
 // offset).  No lane is masked, a masked load is a branch: rows are clamped by
 // the caller, and steps past a row's end read on (the copies are allocated
-// with a layer width to spare) to meet zeros of A or no product at all.
+// with a layer width to spare) to be zeroed by the caller or used in no product.
 template <int KS>
 __device__ __forceinline__ void mlp_load(bf16x8 (&x)[KS], const bf16_t *w) {
 #pragma unroll
@@ -284,6 +284,11 @@ __global__ __launch_bounds__(kRowThreads) void k_mlp_rows(MlpRows P) {
   const int n = 16 * w + lc, nh = 16 * (w % NT) + lc;
   bf16x8 x[KS], nx[KS] = {};
   mlp_load(x, P.W[0] + (long)nh * P.in_pad + lk);
+  // (past the inputs the load reads other neurons' weights: their products with
+  // the zeros of A are dropped here, an infinite one would not be zero)
+#pragma unroll
+  for (int i = 0; i < KS; ++i)
+    if (lk + 32 * i >= P.in_pad) x[i] = bf16x8{};
   // the sample of each of this lane's four output rows (the last row repeated
   // past the batch; its results are dropped), and everything else a wave will
   // want from memory one value at a time: each would be a full latency later

@@ -220,3 +220,17 @@ def test_step_time_is_that_of_the_steps():
         net.train(x[:rows], t[:rows], epochs=2, batch=16384)
         ms.append(min(net.train(x[:rows], t[:rows], epochs=64, batch=16384)[1] for _ in range(3)))
     assert ms[1] < 1.5 * ms[0], ms
+
+
+def test_an_infinite_weight_stays_in_its_neuron():
+    """One infinite first-layer weight of neuron 5: z and the activation of that
+    neuron are infinite, those of its neighbours are not touched (their rows are
+    read in one run with its), so that an output with positive weights is
+    infinite and not NaN."""
+    n_in, n_out, width = 3, 4, 64
+    net, P = _net(n_in, n_out, width, 1, seed=9)
+    w = np.abs(net.get_weights()) + 0.01
+    w[5 * n_in + 1] = np.inf
+    net.set_weights(w)
+    x = np.abs(np.random.default_rng(3).normal(size=(20, n_in))) + 0.1
+    assert np.all(net.predict(x) == np.inf)
