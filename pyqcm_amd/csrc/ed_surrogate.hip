@@ -225,7 +225,7 @@ constexpr int kRows = 16, kRowThreads = 1024, kRowWaves = kRowThreads / 64;
 // KS k-steps of one weight row per lane (w: the lane's row at its 8-element
 // offset).  No lane is masked, a masked load is a branch: rows are clamped by
 // the caller, and steps past a row's end read on (the copies are allocated
-// with a layer width to spare) to be zeroed by the caller or used in no product.
+// with a layer width to spare) and are used in no product.
 template <int KS>
 __device__ __forceinline__ void mlp_load(bf16x8 (&x)[KS], const bf16_t *w) {
 #pragma unroll
@@ -283,12 +283,13 @@ __global__ __launch_bounds__(kRowThreads) void k_mlp_rows(MlpRows P) {
   const bool own = w < NT;
   const int n = 16 * w + lc, nh = 16 * (w % NT) + lc;
   bf16x8 x[KS], nx[KS] = {};
-  mlp_load(x, P.W[0] + (long)nh * P.in_pad + lk);
-  // (past the inputs the load reads other neurons' weights: their products with
-  // the zeros of A are dropped here, an infinite one would not be zero)
+  // (past the inputs a row would read on into other neurons' weights, of which an
+  // infinite one times a zero of A is not zero: these lanes read the zeros behind
+  // the last row.  Zeroing the registers instead cost 1 to 2 of a forward pass's
+  // 26 us, a copy of the weights in rows of a layer width 2.5)
+  const bf16_t *w0 = P.W[0] + (long)nh * P.in_pad + lk, *none = P.W[0] + (long)WD * P.in_pad;
 #pragma unroll
-  for (int i = 0; i < KS; ++i)
-    if (lk + 32 * i >= P.in_pad) x[i] = bf16x8{};
+  for (int i = 0; i < KS; ++i) x[i] = *(const bf16x8 *)(lk + 32 * i < P.in_pad ? w0 + 32 * i : none);
   // the sample of each of this lane's four output rows (the last row repeated
   // past the batch; its results are dropped), and everything else a wave will
   // want from memory one value at a time: each would be a full latency later
