@@ -280,8 +280,22 @@ void Surrogate::ensure_batch(int B) {
   cap_B = B;
 }
 
+// A forward pass alone through the row-block kernel: 4 096 rows a round of 256
+// workgroups, each of which reads all weights (about 4 us and 1 us per 17 000
+// weights), against a GEMM per layer, about 10 us each at these sizes.  us at
+// width, hidden layers, outputs and rows, GEMMs / row blocks: 256 4 641 4 096 45 /
+// 26, 8 192 56 / 49, 9 000 66 / 72, 16 384 75 / 97; 256 2 641 4 096 26 / 19, 8 192
+// 33 / 35; 256 4 64 12 288 56 / 46, 16 384 61 / 62; 128 8 641 16 384 91 / 80; 128 1
+// 641 8 192 18 / 16, 12 288 23 / 23; 64 8 641 16 384 72 / 46.  A training step is
+// the faster in row blocks at every size (256 2 641 16 384: 430 / 228).
+bool Surrogate::forward_rows(int B) const {
+  const long weights = (long)(depth - 1) * width * width + (long)width * n_out;
+  const long rounds = (B + 4095) / 4096;
+  return use_rows(B) && (rounds == 1 || rounds * (4 + weights / 17000) <= 10L * (depth + 1));
+}
+
 void Surrogate::forward(int B, const bf16_t *x) {
-  if (use_rows(B)) {
+  if (forward_rows(B)) {
     MlpRows P = rows_args(B, x, nullptr, nullptr);
     P.y = y.p;
     mlp_rows(P, width, false, stream());

@@ -143,6 +143,7 @@ struct Surrogate {
   // one launch from row idx[b] (b when null) of X and T, b < B, to gradients in
   // dzT / actT / db and loss partials (returns their number)
   bool use_rows(int B) const { return rows_ok && (B + 31) / 32 * 2 <= 1024; }
+  bool forward_rows(int B) const;
   MlpRows rows_args(int B, const bf16_t *X, const float *T, const int *idx);
   MlpShape shape() const;
   MlpParams param_table();

@@ -234,3 +234,17 @@ def test_an_infinite_weight_stays_in_its_neuron():
     net.set_weights(w)
     x = np.abs(np.random.default_rng(3).normal(size=(20, n_in))) + 0.1
     assert np.all(net.predict(x) == np.inf)
+
+
+def test_forward_passes_on_both_sides_of_the_row_block_line():
+    """Two hidden layers of 256 and 641 outputs: 4 096 rows go through the row
+    blocks, 4 097 layer by layer.  The same operands in another summation order
+    (fp32, and a bf16 rounding that may fall the other way): 2e-3 of the scale, as
+    above; three of the rows also against the oracle."""
+    net, P = _net(12, 641, 256, 2, seed=4)
+    x = np.random.default_rng(5).normal(size=(4097, 12))
+    a, b = net.predict(x[:4096]), net.predict(x)
+    scale = np.abs(b).max()
+    assert np.abs(a - b[:4096]).max() <= 2e-3 * scale
+    rows = [0, 2048, 4096]
+    assert np.abs(b[rows] - M.forward(P, x[rows], mimic=True)[0]).max() <= 2e-3 * scale
