@@ -18,21 +18,24 @@ long KGrid::count() const {
   return n;
 }
 
-// The elements go to the device grouped by neighbor vector (one phase serves
-// a group), all parts in one block of doubles: V0, the values, R, then the
-// integer lists.
+// The elements go to the device grouped as the kernel for this d reads them, all
+// parts in one block of doubles: V0, the values, R, then the integer lists.  Up
+// to kRegDim by neighbor vector (one phase serves a group); above by position,
+// since there a lane owns one.
 SuperlatticeDev::SuperlatticeDev(const Superlattice &S) : d(S.d), nnbr((int)S.R.size() / 3) {
   const int dd = d * d;
-  const size_t ne = S.nbr.size();
-  std::vector<int> eptr(nnbr + 1, 0), epos(std::max<size_t>(ne, 1), 0);
+  const bool reg = d <= kRegDim;
+  const size_t ne = S.nbr.size(), ng = reg ? (size_t)nnbr : (size_t)dd;
+  const auto group = [&](size_t r) { return reg ? S.nbr[r] : S.row[r] + d * S.col[r]; };
+  std::vector<int> eptr(ng + 1, 0), epos(std::max<size_t>(ne, 1), 0);
   std::vector<double> ev(2 * std::max<size_t>(ne, 1), 0.0);
   std::vector<char> used(dd, 0);
   for (int e = 0; e < dd; ++e) used[e] = S.V0[2 * e] != 0.0 || S.V0[2 * e + 1] != 0.0;
   for (size_t r = 0; r < ne; ++r) {
-    ++eptr[S.nbr[r] + 1];
+    ++eptr[group(r) + 1];
     used[S.row[r] + d * S.col[r]] = 1;
   }
-  for (int n = 0; n < nnbr; ++n) eptr[n + 1] += eptr[n];
+  for (size_t n = 0; n < ng; ++n) eptr[n + 1] += eptr[n];
   std::vector<int> fill(eptr.begin(), eptr.end() - 1), plist, slot(dd, 0);
   for (int e = 0; e < dd; ++e)
     if (used[e]) {
@@ -42,8 +45,8 @@ SuperlatticeDev::SuperlatticeDev(const Superlattice &S) : d(S.d), nnbr((int)S.R.
     }
   npos = (int)plist.size();
   for (size_t r = 0; r < ne; ++r) {
-    const int at = fill[S.nbr[r]]++, e = S.row[r] + d * S.col[r];
-    epos[at] = slot[e] | e << 16;
+    const int at = fill[group(r)]++;
+    epos[at] = reg ? slot[S.row[r] + d * S.col[r]] : S.nbr[r];
     ev[2 * at] = S.val[2 * r];
     ev[2 * at + 1] = S.val[2 * r + 1];
   }
@@ -71,7 +74,6 @@ SuperlatticeDev::SuperlatticeDev(const Superlattice &S) : d(S.d), nnbr((int)S.R.
 
 namespace {
 
-constexpr int kRegDim = 6;          // largest matrix kept in one lane's registers
 constexpr long kLatticeWaves = 4096;  // waves a launch is cut into (1024 SIMDs x 4)
 
 struct Arg {
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(64) void k_lattice_reg(Arg A, int nz, int zc, const
       double cs, sn;
       phase(A, kk, n, cs, sn);
       for (int r = A.eptr[n]; r < A.eptr[n + 1]; ++r) {
-        double2 &v = sV[(A.epos[r] & 0xffff) * 64 + lane];
+        double2 &v = sV[A.epos[r] * 64 + lane];
         double tr, ti;
         cmul(A.val[2 * r], A.val[2 * r + 1], cs, sn, tr, ti);
         v.x += tr;
@@ -345,14 +347,13 @@ __global__ __launch_bounds__(64) void k_lattice(Arg A, const double *Gz, double 
     __syncthreads();
     if (act) {
       double vr = A.V0[2 * e], vi = A.V0[2 * e + 1];
-      for (int n = 0; n < A.nnbr; ++n)
-        for (int r = A.eptr[n]; r < A.eptr[n + 1]; ++r)
-          if ((A.epos[r] >> 16) == e) {
-            double tr, ti;
-            cmul(A.val[2 * r], A.val[2 * r + 1], sph[2 * n], sph[2 * n + 1], tr, ti);
-            vr += tr;
-            vi += ti;
-          }
+      for (int r = A.eptr[e]; r < A.eptr[e + 1]; ++r) {
+        const int n = A.epos[r];
+        double tr, ti;
+        cmul(A.val[2 * r], A.val[2 * r + 1], sph[2 * n], sph[2 * n + 1], tr, ti);
+        vr += tr;
+        vi += ti;
+      }
       sV[2 * e] = vr;
       sV[2 * e + 1] = vi;
     }

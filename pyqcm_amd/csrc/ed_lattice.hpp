@@ -14,6 +14,7 @@ namespace ed {
 
 // Green-function dimensions and neighbor vectors handled by the kernels
 constexpr int kLatticeMaxDim = 8;
+constexpr int kRegDim = 6;  // largest matrix kept in one lane's registers
 constexpr int kLatticeMaxNbr = 64;
 
 // V(k) = V0 + sum_e val_e exp(2 pi i k . R[nbr_e]) at position (row_e, col_e),
@@ -36,8 +37,9 @@ struct KGrid {
 };
 
 // device copy of a Superlattice: the elements grouped by neighbor vector
-// (eptr[nnbr + 1]; epos: slot in plist | position << 16), plist the npos
-// column-major positions where V(k) can be nonzero (bits of mask)
+// (eptr[nnbr + 1]; epos: slot in plist), or for d > kRegDim by column-major
+// position (eptr[d^2 + 1]; epos: neighbor vector); plist the npos positions
+// where V(k) can be nonzero (bits of mask)
 struct SuperlatticeDev {
   int d = 0, nnbr = 0, npos = 0;
   unsigned long long mask = 0;
