@@ -364,18 +364,24 @@ std::vector<std::pair<int, int>> all_pairs(int ns) {
 // result arrays left to the caller
 void append_pairs(std::vector<BatchCFItem> &items, MapCache &maps, int L, const std::vector<std::pair<int, int>> &pairs,
                   const State &st, int spin, int pm) {
+  const uint32_t du_s = half_basis(L, st.sec.Nup())->dim;
+  std::vector<const MapCache::Set *> of(L, nullptr);  // by orbital: one lookup each, not one per pair
+  const auto get = [&](int o) -> const MapCache::Set & {
+    if (!of[o]) of[o] = &maps.get(L, st.sec, pm, o + spin * L);
+    return *of[o];
+  };
   for (const auto &p : pairs) {
-    const MapCache::Set &m0 = maps.get(L, st.sec, pm, p.first + spin * L);
+    const MapCache::Set &m0 = get(p.first);
     BatchCFItem it;
     it.gs = st.psi.p;
-    it.du_s = half_basis(L, st.sec.Nup())->dim;
+    it.du_s = du_s;
     it.spin = spin;
     it.norb = p.second == p.first ? 1 : 2;
     it.map[0] = m0.map.p;
     it.sgn[0] = m0.sgn.p;
     it.upar = m0.upar.p;
     if (p.second != p.first) {
-      const MapCache::Set &m1 = maps.get(L, st.sec, pm, p.second + spin * L);
+      const MapCache::Set &m1 = get(p.second);
       it.map[1] = m1.map.p;
       it.sgn[1] = m1.sgn.p;
     }
