@@ -338,11 +338,15 @@ __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int m
     __syncthreads();
     ++k;
     // The Ritz pair is a serial chain of one wave, longer than the step itself:
-    // found every kRitzEvery steps, and at each one where the Krylov space may
-    // be exhausted (as many steps as states, a small beta) or the run ends.
-    // 512 points of 2x3 (300 to 400 states, 256 threads): every step 13.5 ms,
-    // every 4th 5.7 ms.
-    if (k <= kRitzEvery || k % kRitzEvery == 0 || (uint32_t)k >= dim || !(beta > 1e-6 * be[0]) || k > max_iter) {
+    // with four waves (128 states or more) found every kRitzEvery steps, and at
+    // each one where the Krylov space may be exhausted (as many steps as states, a
+    // small beta) or the run ends.  512 points of 2x3 (300 to 400 states): every
+    // step 13.5 ms, every 4th 5.7 ms.  Smaller sectors converge as their Krylov
+    // space ends, and past that point a pair may look unconverged again (128
+    // points of 2x2, 24 and 36 states: at each step 26 steps at most, 0.28 ms, at
+    // every 4th 42, 0.31): there at each step.
+    if (BS == kW || k <= kRitzEvery || k % kRitzEvery == 0 || (uint32_t)k >= dim || !(beta > 1e-6 * be[0]) ||
+        k > max_iter) {
       if (threadIdx.x < kW) tri_lowest_wave(k, al, be, bb, &s_hi, z, D, l, &s_lam, &s_zl);
       __syncthreads();
       // a zero beta: the Krylov space is exhausted (one-state sectors end here)

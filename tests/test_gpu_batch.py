@@ -108,9 +108,9 @@ def test_batch_ground_states_with_band_lanczos_green_functions():
 @pytest.mark.parametrize("L,N,S,dim", [(2, 1, 1, 2), (4, 1, 1, 4), (5, 1, 1, 5), (3, 2, 0, 9), (5, 2, 2, 10),
                                        (4, 4, 0, 36), (5, 4, 0, 100), (6, 4, 0, 225)])
 def test_ground_states_whose_krylov_space_ends_between_checks(L, N, S, dim):
-    """Ritz pairs are found every fourth step and wherever the Krylov space may
-    end: as many states as one, between one and two checks, and more, in the
-    one-wave and the four-wave workgroup."""
+    """Ritz pairs are found at each step in the one-wave workgroup, in the
+    four-wave one every fourth and wherever the Krylov space may end: as many
+    states as one, between one and two checks, and more."""
     wl = dataclasses.replace(W.hubbard_chain(L, U=4.0, mu=1.3), sector="R0:N%d:S%d" % (N, S))
     assert math.comb(L, (N + S) // 2) * math.comb(L, (N - S) // 2) == dim
     _compare(wl, [{"t": 1.0, "U": 4.0, "mu": 1.3}, {"t": 1.0, "U": 7.0, "mu": 2.2}], "F", W.matsubara(16, 20.0))
