@@ -7,6 +7,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <future>
 #include <map>
 #include <tuple>
 
@@ -192,19 +194,50 @@ void launch_classes(const std::vector<Item> &items, const std::vector<Cls> &cls,
   sync();
 }
 
-// the register-tile fractions, by tile shape
-void launch_tiles(const TablePack &tabs, const std::vector<BatchCFItem> &items, const std::vector<Cls> &cls,
-                  const std::vector<int> &tab, int max_cf, double acc) {
-  std::vector<BatchCFItem> part[2][2];
+// The register-tile fractions, by tile shape.  As many as the SIMDs hold two of (a
+// wave each) or fewer go as one launch of the shape that holds them all: what a
+// larger tile adds is zero, term by term, and the launches' dependent steps would
+// add up (2x1 with 5 bath orbitals, halves of 1 to 21 states, whole solve of 2
+// points: 2.14 ms shape by shape, 1.83 so; 12 points of 2x3 5.9 and 4.7).
+constexpr size_t kTilesAtOnce = 2048;
+using TileParts = std::vector<BatchCFItem>[2][2];
+void sort_tiles(const TablePack &tabs, const std::vector<BatchCFItem> &items, const std::vector<Cls> &cls,
+                const std::vector<int> &tab, TileParts &part) {
+  size_t ntile = 0;
+  int rmax = 0, cmax = 0;
   for (size_t k = 0; k < items.size(); ++k)
-    if (cls[k] == kTile) part[tabs.offs[tab[k]].dd > 16][tabs.offs[tab[k]].du > 16].push_back(items[k]);
-  DevBuf<BatchCFItem> d[2][2];
-  for (int r = 0; r < 2; ++r)
-    for (int c = 0; c < 2; ++c) {
-      if (part[r][c].empty()) continue;
-      d[r][c].upload(part[r][c]);
-      tile_cf(d[r][c].p, (int)part[r][c].size(), r + 1, c + 1, max_cf, acc, stream());
+    if (cls[k] == kTile) {
+      ++ntile;
+      rmax |= tabs.offs[tab[k]].dd > 16;
+      cmax |= tabs.offs[tab[k]].du > 16;
     }
+  const bool one = ntile <= kTilesAtOnce;
+  for (size_t k = 0; k < items.size(); ++k)
+    if (cls[k] == kTile)
+      part[one ? rmax : tabs.offs[tab[k]].dd > 16][one ? cmax : tabs.offs[tab[k]].du > 16].push_back(items[k]);
+}
+
+// Launch groups that do not depend on each other, with few enough items in all to
+// leave part of the chip idle: side by side, each but the first on a host thread
+// and stream of its own, since one after the other their dependent steps add up
+// (2x2 with 3 bath orbitals, 35 x 21 states from LDS and 21 x 7 in tiles, whole
+// solve of 2 points: 4.45 ms one after the other, 3.59 so).  The inputs are complete
+// before the threads start and a thread's work before it ends.
+constexpr size_t kBesideItems = 8192;
+void run_beside(const std::vector<std::function<void()>> &groups, size_t items) {
+  if (groups.size() < 2 || items > kBesideItems) {
+    for (const auto &g : groups) g();
+    return;
+  }
+  sync();
+  std::vector<std::future<void>> rest;  // (a future of async waits for its thread where it is dropped)
+  for (size_t k = 1; k < groups.size(); ++k)
+    rest.push_back(std::async(std::launch::async, [&groups, k] {
+      groups[k]();
+      sync();
+    }));
+  groups[0]();
+  for (auto &f : rest) f.get();
 }
 
 // The wide items (tab[k]: item k's sector), by shape and then in groups whose
@@ -418,10 +451,28 @@ void run_fractions(TablePack &tabs, std::vector<BatchCFItem> &items, const std::
     it.b = bv.p + (size_t)(max_cf + 1) * k;
     it.out = out.p + 2 * k;
   }
-  launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds, bool) {
-    batch_cf(d, n, block, lds, max_cf, acc, stream());
-  });
-  launch_tiles(tabs, items, cls, tab, max_cf, acc);
+  TileParts tiles;
+  sort_tiles(tabs, items, cls, tab, tiles);
+  std::vector<std::function<void()>> groups;
+  size_t nlds = 0, ntile = 0;
+  for (Cls c : cls) nlds += c < kLdsClasses;
+  if (nlds)
+    groups.push_back([&] {
+      launch_classes(items, cls, lds_max, [&](const BatchCFItem *d, int n, int block, size_t lds, bool) {
+        batch_cf(d, n, block, lds, max_cf, acc, stream());
+      });
+    });
+  for (int r = 0; r < 2; ++r)
+    for (int c = 0; c < 2; ++c) {
+      if (tiles[r][c].empty()) continue;
+      ntile += tiles[r][c].size();
+      groups.push_back([&, r, c] {
+        DevBuf<BatchCFItem> d;
+        d.upload(tiles[r][c]);
+        tile_cf(d.p, (int)tiles[r][c].size(), r + 1, c + 1, max_cf, acc, stream());
+      });
+    }
+  run_beside(groups, nlds + ntile);
   launch_wide(tabs, items, cls, tab, 2, 0, [&](const WideShape &W, const WideItem *w, const BatchCFItem *q, int n) {
     wide_cf(W, w, q, n, max_cf, acc, stream());
   });

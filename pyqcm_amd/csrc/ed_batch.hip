@@ -296,6 +296,7 @@ __device__ __forceinline__ void tri_lowest_wave(int n, const double *a, const do
 }
 
 constexpr int kRitzEvery = 4;
+constexpr uint32_t kRitzEach = 48;
 // TRI: the tridiagonal arrays in LDS too; else (more steps allowed than fit
 // beside the sector) the item's own in memory
 template <int BS, bool TRI>
@@ -338,14 +339,14 @@ __global__ __launch_bounds__(BS) void k_batch_gs(const BatchGSItem *items, int m
     __syncthreads();
     ++k;
     // The Ritz pair is a serial chain of one wave, longer than the step itself:
-    // with four waves (128 states or more) found every kRitzEvery steps, and at
-    // each one where the Krylov space may be exhausted (as many steps as states, a
-    // small beta) or the run ends.  512 points of 2x3 (300 to 400 states): every
-    // step 13.5 ms, every 4th 5.7 ms.  Smaller sectors converge as their Krylov
-    // space ends, and past that point a pair may look unconverged again (128
-    // points of 2x2, 24 and 36 states: at each step 26 steps at most, 0.28 ms, at
-    // every 4th 42, 0.31): there at each step.
-    if (BS == kW || k <= kRitzEvery || k % kRitzEvery == 0 || (uint32_t)k >= dim || !(beta > 1e-6 * be[0]) ||
+    // found every kRitzEvery steps, and at each one where the Krylov space may be
+    // exhausted (as many steps as states, a small beta) or the run ends.  512 points
+    // of 2x3 (300 to 400 states): every step 13.5 ms, every 4th 5.7; 12 of 2x2 with a
+    // bath orbital (50 and 100 states), whole solve: 2.24 and 1.54 ms.  The smallest
+    // sectors converge as their Krylov space ends, and past that point a pair may
+    // look unconverged again (128 points of 2x2, 24 and 36 states: at each step 26
+    // steps at most, 0.28 ms, at every 4th 42, 0.31): there at each step.
+    if (dim < kRitzEach || k <= kRitzEvery || k % kRitzEvery == 0 || (uint32_t)k >= dim || !(beta > 1e-6 * be[0]) ||
         k > max_iter) {
       if (threadIdx.x < kW) tri_lowest_wave(k, al, be, bb, &s_hi, z, D, l, &s_lam, &s_zl);
       __syncthreads();

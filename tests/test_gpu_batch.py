@@ -312,3 +312,28 @@ def test_register_tiles_at_their_edges(nb):
         qcm.set_global_parameterC("hv_variant", 0)
         for lab in (30900, 30901):
             qcm.erase_model_instance(lab)
+
+
+def test_tiles_at_once_and_shape_by_shape():
+    """2x1 with 5 bath orbitals, halves of 1 to 21 states: a few points' register
+    tiles go as one launch of the largest shape, many points' shape by shape and
+    side by side.  A point's energy and Green function are the same to the last
+    bit either way."""
+    wl = W.vca_cluster_bath(2, 1, 5)
+    name = _model(wl)
+    pts = [{**wl.values, **v} for v in W.vca_points(400, seed=12)]
+    z = W.real_axis(24)
+    qcm.set_global_parameterC("GF_method", "F")
+    out = []
+    for which in (range(400), (0, 399)):
+        labels = {k: _new_label() for k in which}
+        for k, lab in labels.items():
+            qcm.new_model_instanceC(name, pts[k], wl.sector, lab)
+        qcm.solve_batch(list(labels.values()))
+        out.append([(qcm.ground_state_solve(labels[k])[0],
+                     *(qcm.Green_function_grid(z, spin_down=s, label=labels[k]) for s in (0, 1))) for k in (0, 399)])
+        for lab in labels.values():
+            qcm.erase_model_instance(lab)
+    for a, b in zip(*out):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
